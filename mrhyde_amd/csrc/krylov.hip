@@ -655,8 +655,10 @@ __global__ __launch_bounds__(256) void k_mupdate_dot(long n, int K, const T* __r
       p = fma(-hk[j], v[j], p);
     }
     s_p[buf][wv][l] = p;
-    __syncthreads();  // (two buffers: the next sweep step writes the other one)
+    // w_i before the barrier: wavefront 0 overwrites it after the barrier,
+    // and every wavefront needs the value from before the update
     const double wi = in ? (double)w[i] : 0.0;
+    __syncthreads();  // (two buffers: the next sweep step writes the other one)
     const T ws = (T)((wi + (s_p[buf][0][l] + s_p[buf][1][l])) + (s_p[buf][2][l] + s_p[buf][3][l]));
     if (in && wv == 0) {
       w[i] = ws;

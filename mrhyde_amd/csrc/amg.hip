@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "lattice.hpp"
+#include "lattice_product.hpp"
 #include "mhx_internal.hpp"
 
 namespace mhx {
@@ -652,8 +653,6 @@ __device__ __forceinline__ double row_dot(const int32_t* __restrict__ rp, CI ci,
   return acc;
 }
 
-// one Chebyshev step: r = b - A xin (A xin skipped when zero_x),
-// d = alpha d + beta D^-1 r, xout = xin + d (xin = 0 when zero_x)
 // LAT: the level-0 operator in the context's lattice pattern, columns from its
 // closed form instead of ci (same entries, same order, same sums)
 template <bool LAT>
@@ -663,18 +662,64 @@ __device__ __forceinline__ auto level_cols(const BoxMesh& m, const int32_t* __re
   else return CsrCols{ci};
 }
 
+// The row ends of the level kernels: what happens with (A x)_row.
+// w = s * D^-1 A v, s = *sp
+struct DinvRow {
+  const double* __restrict__ dinv;
+  const double* __restrict__ sp;
+  double* __restrict__ w;
+  struct Pre {
+    double s;
+  };
+  __device__ __forceinline__ Pre load(long row) const { return {*sp * dinv[row]}; }
+  __device__ __forceinline__ void operator()(long row, double ax, Pre p) const { w[row] = p.s * ax; }
+};
+// d = alpha d + beta D^-1 (b - A xin), xout = xin + d (xin = 0 when zero_x)
+template <class T>
+struct ChebRow {
+  const T* __restrict__ b;
+  const T* __restrict__ xin;
+  T* __restrict__ xout;
+  T* __restrict__ d;
+  const T* __restrict__ dinv;
+  double alpha, beta;
+  int zero_x;
+  struct Pre {
+    T b, x, d, dinv;
+  };
+  __device__ __forceinline__ Pre load(long row) const {
+    return {b[row], zero_x ? (T)0 : xin[row], alpha != 0.0 ? d[row] : (T)0, dinv[row]};
+  }
+  __device__ __forceinline__ void operator()(long row, double ax, const Pre& p) const {
+    const double r = (double)p.b - ax;
+    const double dn = (alpha != 0.0 ? alpha * (double)p.d : 0.0) + beta * (double)p.dinv * r;
+    d[row] = (T)dn;
+    xout[row] = (T)((double)p.x + dn);
+  }
+};
+// r = b - A x
+template <class T>
+struct ResidRow {
+  const T* __restrict__ b;
+  T* __restrict__ r;
+  struct Pre {
+    T b;
+  };
+  __device__ __forceinline__ Pre load(long row) const { return {b[row]}; }
+  __device__ __forceinline__ void operator()(long row, double ax, Pre p) const { r[row] = (T)((double)p.b - ax); }
+};
+
 // w = s * D^-1 A v  (s = *sp, on the device: the scale applied to v, so v
 // need not be normalised in place)
 template <int LANES, bool LAT>
 __global__ __launch_bounds__(256) void k_amg_dinv_spmv(BoxMesh m, long n, const int32_t* __restrict__ rp,
                                                        const int32_t* __restrict__ ci, const double* __restrict__ A,
-                                                       const double* __restrict__ dinv, const double* __restrict__ sp,
-                                                       const double* __restrict__ v, double* __restrict__ w) {
+                                                       const double* __restrict__ v, DinvRow end) {
   const long row = ((long)blockIdx.x * blockDim.x + threadIdx.x) / LANES;
   const int l = threadIdx.x % LANES;
   if (row >= n) return;
   const double acc = row_dot<LANES, double>(rp, level_cols<LAT>(m, rp, ci, row), A, v, row, l);
-  if (l == 0) w[row] = *sp * dinv[row] * acc;
+  if (l == 0) end(row, acc, end.load(row));
 }
 
 // scalar steps of the power iteration, one thread; st = (s, lambda, stopped).
@@ -699,35 +744,28 @@ __global__ void k_amg_power(int phase, const double* __restrict__ d0, const doub
   }
 }
 
+// one Chebyshev step (A xin skipped when zero_x)
 template <int LANES, bool LAT, class T>
 __global__ __launch_bounds__(256) void k_amg_cheb(BoxMesh m, long n, const int32_t* __restrict__ rp,
                                                   const int32_t* __restrict__ ci, const T* __restrict__ A,
-                                                  const T* __restrict__ b, const T* __restrict__ xin,
-                                                  T* __restrict__ xout, T* __restrict__ d,
-                                                  const T* __restrict__ dinv, double alpha, double beta, int zero_x) {
+                                                  ChebRow<T> end) {
   const long row = ((long)blockIdx.x * blockDim.x + threadIdx.x) / LANES;
   const int l = threadIdx.x % LANES;
   if (row >= n) return;
-  const double ax = zero_x ? 0.0 : row_dot<LANES, T>(rp, level_cols<LAT>(m, rp, ci, row), A, xin, row, l);
-  if (l == 0) {
-    const double r = (double)b[row] - ax;
-    const double dn = (alpha != 0.0 ? alpha * (double)d[row] : 0.0) + beta * (double)dinv[row] * r;
-    d[row] = (T)dn;
-    xout[row] = (T)((zero_x ? 0.0 : (double)xin[row]) + dn);
-  }
+  const double ax =
+      end.zero_x ? 0.0 : row_dot<LANES, T>(rp, level_cols<LAT>(m, rp, ci, row), A, end.xin, row, l);
+  if (l == 0) end(row, ax, end.load(row));
 }
 
-// r = b - A x
 template <int LANES, bool LAT, class T>
 __global__ __launch_bounds__(256) void k_amg_resid(BoxMesh m, long n, const int32_t* __restrict__ rp,
                                                    const int32_t* __restrict__ ci, const T* __restrict__ A,
-                                                   const T* __restrict__ b, const T* __restrict__ x,
-                                                   T* __restrict__ r) {
+                                                   const T* __restrict__ x, ResidRow<T> end) {
   const long row = ((long)blockIdx.x * blockDim.x + threadIdx.x) / LANES;
   const int l = threadIdx.x % LANES;
   if (row >= n) return;
   const double ax = row_dot<LANES, T>(rp, level_cols<LAT>(m, rp, ci, row), A, x, row, l);
-  if (l == 0) r[row] = (T)((double)b[row] - ax);
+  if (l == 0) end(row, ax, end.load(row));
 }
 
 // One colour of a multicolour nodal block Gauss-Seidel sweep: for every node
@@ -825,6 +863,7 @@ struct AmgLevel {
   DevBuf<double> P, R;
   DevBuf<double> binv;  // nodal nf x nf diagonal-block inverses (block-Jacobi smoother)
   bool lat = false;     // level 0 in the context's lattice pattern: closed-form columns
+  bool q2 = false;      // level 0 by the order-2 lattice product (lattice_product.hpp)
   double lambda = 1.0;
   AmgVals<float> f32;
   AmgVals<double> f64;  // FP64 work vectors (values live in A/P/R above)
@@ -924,12 +963,17 @@ static void power_estimate(Ctx& c, AmgLevel& L, const double* A, double* v, doub
   dot_dev(c, v, v, n, slots);
   hipLaunchKernelGGL(k_amg_power, dim3(1), dim3(1), 0, c.stream, 0, slots, slots, st);
   for (int it = 0; it < kAmgPowerIters; ++it) {
-    by_lanes(L.lanes, [&](auto LN) {
-      by_lat(L.lat, [&](auto LT) {
-        hipLaunchKernelGGL((k_amg_dinv_spmv<decltype(LN)::value, decltype(LT)::value>), g1(n * LN), dim3(256), 0,
-                           c.stream, c.mesh, n, L.rp, L.ci, A, L.dinv.p, st, v, w);
+    const DinvRow end{L.dinv.p, st, w};
+    if (L.q2) {
+      q2_product<double>(c, A, v, end);
+    } else {
+      by_lanes(L.lanes, [&](auto LN) {
+        by_lat(L.lat, [&](auto LT) {
+          hipLaunchKernelGGL((k_amg_dinv_spmv<decltype(LN)::value, decltype(LT)::value>), g1(n * LN), dim3(256), 0,
+                             c.stream, c.mesh, n, L.rp, L.ci, A, v, end);
+        });
       });
-    });
+    }
     MHX_HIP(hipGetLastError());
     dot_dev(c, v, w, n, slots);
     dot_dev(c, w, w, n, slots + 1);
@@ -1006,6 +1050,7 @@ void amg_setup(Ctx& c, const double* A, bool fp32) {
   L->ci = c.colidx.p;
   L->lanes = c.spmv_lanes;
   L->lat = c.lattice_cols != 0;
+  L->q2 = q2_product_applies(c);
   L->dinv.alloc(L->n);
   L->ns.alloc(L->n);
   hipLaunchKernelGGL(k_amg_diag, g1(L->n), dim3(256), 0, c.stream, L->n, L->rp, L->ci, A, L->dinv.p);
@@ -1169,12 +1214,17 @@ LvView<float> view<float>(Amg& H, int l, const float* A0) {
 template <class T>
 static void cheb_step(Ctx& c, AmgLevel& V, const LvView<T>& W, const T* b, const T* xin, T* xout, double alpha,
                       double beta, int zero_x) {
+  const ChebRow<T> end{b, xin, xout, W.d, W.dinv, alpha, beta, zero_x};
+  if (V.q2 && !zero_x) {
+    q2_product<double>(c, W.A, xin, end);
+    return;
+  }
   by_lanes(zero_x ? 4 : V.lanes, [&](auto LN) {
     by_lat(V.lat, [&](auto LT) {
       constexpr int K = decltype(LN)::value;
       constexpr bool LAT = decltype(LT)::value;
       hipLaunchKernelGGL((k_amg_cheb<K, LAT, T>), g1(V.n * K), dim3(256), 0, c.stream, c.mesh, V.n, V.rp, V.ci, W.A,
-                         b, xin, xout, W.d, W.dinv, alpha, beta, zero_x);
+                         end);
     });
   });
 }
@@ -1182,12 +1232,17 @@ static void cheb_step(Ctx& c, AmgLevel& V, const LvView<T>& W, const T* b, const
 // r = b - A x on one level
 template <class T>
 static void level_resid(Ctx& c, AmgLevel& V, const LvView<T>& W, const T* b, const T* x, T* r) {
+  const ResidRow<T> end{b, r};
+  if (V.q2) {
+    q2_product<double>(c, W.A, x, end);
+    return;
+  }
   by_lanes(V.lanes, [&](auto LN) {
     by_lat(V.lat, [&](auto LT) {
       constexpr int K = decltype(LN)::value;
       constexpr bool LAT = decltype(LT)::value;
       hipLaunchKernelGGL((k_amg_resid<K, LAT, T>), g1(V.n * K), dim3(256), 0, c.stream, c.mesh, V.n, V.rp, V.ci,
-                         W.A, b, x, r);
+                         W.A, x, end);
     });
   });
 }

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "lattice.hpp"
+#include "lattice_product.hpp"
 #include "mhx_internal.hpp"
 
 namespace mhx {
@@ -72,8 +73,20 @@ __global__ __launch_bounds__(256) void k_spmv(BoxMesh m, long n, const int32_t* 
   if (l == 0) y[row] = acc;
 }
 
+template <class T>
+struct StoreRow {
+  T* __restrict__ y;
+  struct Pre {};
+  __device__ __forceinline__ Pre load(long) const { return {}; }
+  __device__ __forceinline__ void operator()(long row, T v, Pre) const { y[row] = v; }
+};
+
 template <class TA, class TX>
 static void spmv_t(Ctx& c, const TA* A, const TX* s, const TX* x, TX* y) {
+  if (!s && q2_product_applies(c)) {
+    q2_product<TX>(c, A, x, StoreRow<TX>{y});
+    return;
+  }
   long n = c.mesh.ndof;
   int L = c.spmv_lanes;
   long threads = n * L;

@@ -267,7 +267,7 @@ void build_box(Ctx& c) {
   double avg = (double)c.nnz / (double)m.ndof;
   int lanes = 4;
   while (lanes < 64 && lanes * 14 < avg) lanes *= 2;
-  c.spmv_lanes = lanes;
+  c.spmv_lanes = c.spmv_lanes_default = lanes;
 }
 
 }  // namespace mhx

@@ -226,6 +226,7 @@ struct Ctx {
   bool own_stream = false;
   Profiler prof;
   int spmv_lanes = 16;
+  int spmv_lanes_default = 16;  // the context's own choice (set at build)
   int lattice_cols = 1;  // sparse products take columns from the lattice closed form (0: from colidx)
   int amg_smoother = -1;  // -1 automatic, 0 Chebyshev(2) on the point diagonal, 1 nodal block Jacobi, 2 block Gauss-Seidel
   int amg_reuse = 0;       // 1: later AMG set-ups keep the coarse levels and refresh the fine level

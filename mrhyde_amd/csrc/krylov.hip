@@ -611,7 +611,11 @@ static int cg_core(Ctx& c, const T* A, const Prec<T>& P, const T* b, T* x, doubl
 // of w, which HBM then delivers once per sweep.
 constexpr int kGsChunk = 17;  // 4 x 17 >= 65 basis vectors
 
-// h[k] = V_k . w for k < K  (V row-major: vector k at V + k*ld), FP64 sums
+// h[k] = V_k . w for k < K  (V row-major: vector k at V + k*ld), FP64 sums.
+// Two rows a lane and up to four vectors a group: the group's eight loads have
+// no branch between them (past the chunk's end they repeat its last vector),
+// so they are in flight together; with one load per branch the sweep ran at
+// 3.4 TB/s at 64^3 Q2 (2.1 M rows).
 template <class T>
 __global__ __launch_bounds__(256) void k_mdot(long n, int K, const T* __restrict__ V, long ld,
                                               const T* __restrict__ w, double* __restrict__ part,
@@ -622,11 +626,27 @@ __global__ __launch_bounds__(256) void k_mdot(long n, int K, const T* __restrict
   double acc[kGsChunk];
 #pragma unroll
   for (int j = 0; j < kGsChunk; ++j) acc[j] = 0.0;
-  for (long i = (long)blockIdx.x * 64 + l; i < n; i += (long)gridDim.x * 64) {
-    const double wi = (double)w[i];
+  if (kc > 0) {
+    const T* Vw = V + (long)k0 * ld;
+    for (long b = (long)blockIdx.x * 128; b < n; b += (long)gridDim.x * 128) {
+      const long i0 = min(b + l, n - 1), i1 = min(b + 64 + l, n - 1);
+      const double w0 = b + l < n ? (double)w[i0] : 0.0, w1 = b + 64 + l < n ? (double)w[i1] : 0.0;
 #pragma unroll
-    for (int j = 0; j < kGsChunk; ++j)
-      if (j < kc) acc[j] = fma((double)V[(long)(k0 + j) * ld + i], wi, acc[j]);
+      for (int g = 0; g < kGsChunk; g += 4) {
+        if (g < kc) {
+          T a0[4], a1[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const T* Vj = Vw + (long)min(g + u, kc - 1) * ld;
+            a0[u] = Vj[i0];
+            a1[u] = Vj[i1];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (g + u < kGsChunk) acc[g + u] = fma((double)a0[u], w0, fma((double)a1[u], w1, acc[g + u]));
+        }
+      }
+    }
   }
 #pragma unroll
   for (int j = 0; j < kGsChunk; ++j) {
@@ -660,25 +680,35 @@ __global__ __launch_bounds__(256) void k_mupdate_dot(long n, int K, const T* __r
   for (long base = (long)blockIdx.x * 64; base < n; base += (long)gridDim.x * 64, buf ^= 1) {
     const long i = base + l;
     const bool in = i < n;
-    double v[kGsChunk];
+    const long ic = in ? i : n - 1;
+    // the chunk's loads in groups of four without a branch between them, all
+    // groups ahead of the first use (past the chunk's end: its last vector)
+    T v[kGsChunk + 3];
+#pragma unroll
+    for (int g = 0; g < kGsChunk; g += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[g + u] = (T)0;
+      if (g < kc) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[g + u] = V[(long)(k0 + min(g + u, kc - 1)) * ld + ic];
+      }
+    }
     double p = 0.0;
 #pragma unroll
-    for (int j = 0; j < kGsChunk; ++j) {
-      v[j] = (j < kc && in) ? (double)V[(long)(k0 + j) * ld + i] : 0.0;
-      p = fma(-hk[j], v[j], p);
-    }
+    for (int j = 0; j < kGsChunk; ++j) p = fma(-hk[j], (double)v[j], p);
     s_p[buf][wv][l] = p;
     // w_i before the barrier: wavefront 0 overwrites it after the barrier,
     // and every wavefront needs the value from before the update
     const double wi = in ? (double)w[i] : 0.0;
     __syncthreads();  // (two buffers: the next sweep step writes the other one)
-    const T ws = (T)((wi + (s_p[buf][0][l] + s_p[buf][1][l])) + (s_p[buf][2][l] + s_p[buf][3][l]));
+    const T ws =
+        in ? (T)((wi + (s_p[buf][0][l] + s_p[buf][1][l])) + (s_p[buf][2][l] + s_p[buf][3][l])) : (T)0;
     if (in && wv == 0) {
       w[i] = ws;
       nrm = fma((double)ws, (double)ws, nrm);
     }
 #pragma unroll
-    for (int j = 0; j < kGsChunk; ++j) acc[j] = fma(v[j], (double)ws, acc[j]);
+    for (int j = 0; j < kGsChunk; ++j) acc[j] = fma((double)v[j], (double)ws, acc[j]);
   }
 #pragma unroll
   for (int j = 0; j < kGsChunk; ++j) {

@@ -9,58 +9,57 @@
 //   thermal<EvalT>::volumeResidual          thermal.cpp:71-165
 //   AssemblyManager::scatter                assemblyManager_scatter.hpp:164-278
 //
-// Work unit.  One 64-lane wavefront (one workgroup) owns an x-segment of one
-// element pencil (fixed ey, ez) and walks it two elements per step: lanes
-// 32h .. 32h+31 take element ex = xa + h of the step starting at xa.
+// Rows, not elements, are owned: the row lines (Y, Z) = (2 ey + jy, 2 ez + jz)
+// of block (ey, ez) need the elements (ey - 1, ey) x (ez - 1, ez), and every
+// CRS entry is summed on chip and written once, in one launch: no colours, no
+// read-back, no first-touch rule.  (Scattering element matrices from eight
+// colour launches wrote 0.74 and re-read 0.44 GB per launch, one 8-byte store
+// per lane and line, at two wavefronts per SIMD: 4.10 ms at 96^3.)
 //
-// Element matrix by pair sum factorisation.  On a box element J = diag(J_c)
-// and the thermal flux is isotropic (dflux_c / d(grad u)_c' = 0 for c != c'),
+// Work unit.  A workgroup of four wavefronts owns 2 x 2 such blocks (one per
+// wavefront in the last stage) and walks an x-segment one element layer per
+// step: 3 x 3 elements, the low ones in y and z shared with the neighbouring
+// workgroup and evaluated by both.  Only the point stage is repeated (2.25
+// times); the contractions are indexed by owned rows.
+//
+// Element matrices by pair sum factorisation.  On a box element J = diag(J_c)
+// and the thermal flux is isotropic with dflux_c / d(grad u)_c = k for every c,
 // so with reference derivatives
-//   A_ij = sum_q sum_c [ alpha_c(q) dphi_i/dxi_c dphi_j/dxi_c
-//                      + beta_c(q)  dphi_i/dxi_c phi_j ]
-//   alpha_c = w|J| dflux_c/d(grad u)_c / J_c^2,   beta_c = w|J| dflux_c/du / J_c
-// (the point physics in forward-mode dual arithmetic gives both slots).  Each
-// term is a product over the axes of 1-D pair tables
-//   M_t[(i_d, j_d)][q_d] = l_a(i_d, q_d) l_b(j_d, q_d),  l_0 = value, l_1 = slope
-// with types t = (a, b): 0 = (0,0), 1 = (1,0), 3 = (1,1), so
-//   A[(i1,j1),(i2,j2),(i3,j3)] = sum_q1 M_t1 sum_q2 M_t2 sum_q3 M_t3 field(q)
-// follows from three contractions (q3, then q2, then q1) of the six point
-// fields; terms are merged as soon as their remaining types agree:
-//   after q3: groups (t1,t2) = (3,0) {alpha_x}, (1,0) {beta_x}, (0,3) {alpha_y},
-//             (0,1) {beta_y}, (0,0) {alpha_z (t3 = 3), beta_z (t3 = 1)}
-//   after q2: groups t1 = 3, 1, 0
-// 11.7k FMA per element (27 sum-factorised columns: ~33k).  The products
-// after q2 (3 q1 slices x 3 groups x 81) overwrite the point fields in LDS,
-// and the q1 contraction runs per row task into register accumulators.
-//
-// Scatter.  Each lane's task in the last stage is one row (i1, i2, i3) and the
-// x-run of three columns (j1 = 0..2) at (j2, j3).  Half 0 takes the rows in
-// the mirrored x order of half 1 (i1 = 2 - m against m), so the lane holding
-// element A's rows on the x-plane it shares with element B holds B's rows on
-// that plane in the other half; the shared column is summed across the
-// halves (shuffle) and the lane pair writes the row's x-run of five once.  The
-// plane shared with the next step is carried in half 1's registers.  Entries
-// shared with a neighbouring pencil (row and column on the same y or z vertex
-// plane) or segment (the segment's end planes) are written by the first
-// scheduled unit and added by later ones: 8 launches, one per colour of
-// (segment parity, ey parity, ez parity), as in element colouring.  Strong
-// Dirichlet rows are written as e_d by their first toucher
-// (assemblyManager_scatter.hpp:208,253; constraints.hpp:125-141).
+//   A_ij = sum_q [ kappa sum_c dphi_i/dxi_c dphi_j/dxi_c / J_c^2
+//                + sum_c beta_c dphi_i/dxi_c phi_j ]
+//   kappa = w|J| k,   beta_c = w|J| k' (du/dx_c) / J_c.
+// With 1-D values B and slopes D the sum is three contractions:
+//   z: t0 = BB kappa, t1 = BB beta_x, t2 = BB beta_y,
+//      t3 = DD kappa / J_z^2 + DB beta_z        per (q1, q2) and z pair (Z, Z')
+//   y: S3 = BB t0, S1 = BB t1, S0 = DD t0 / J_y^2 + DB t2 + BB t3
+//                                               per q1 and pair (Y, Y', Z, Z')
+//   x: DD S3 / J_x^2 + DB S1 + BB S0            per (X, X')
+// A pair on a shared vertex plane sums both elements in the contraction itself
+// (eight assembled pairs per element and axis instead of nine), so block
+// (ey, ez) has 64 (Y, Y', Z, Z') pairs: one per lane of its wavefront.  The
+// lane walks x with the pair, keeps the row 2e + 2's share of element e in
+// three registers, and forms the runs of rows 2e (five columns) and 2e + 1
+// (three) of its (Y', Z') column line.  The wavefront's 512 entries of a step
+// are four contiguous pieces of the CRS values (one per row line); they pass
+// through LDS once to be stored as contiguous 512-byte runs.
+// The residual takes the same contractions with one index (the dual's value).
+// Row starts follow from the lattice pattern in closed form.  Strong
+// Dirichlet rows are written as e_d (assemblyManager_scatter.hpp:208,253;
+// constraints.hpp:125-141).
 // Global residual = -F (scatter.hpp:227); Jacobian = +dF/du (:261).
 //
-// Memory order.  A later touch loads, adds and stores.  Vector-memory
-// counters retire in issue order, so a load issued after a store waits for
-// that store: the scatter issues all nine rounds' loads of a step before its
-// first store, and the wavefront waits for memory about once per step.  The
-// runs of one step are disjoint entries, and no entry is written in one step
-// and read in the next (the carry), so the early loads see final values.
-// The next step's gather is prefetched before the scatter.  Per-workgroup
-// LDS (19 KB) and registers (<= 256) give 2 wavefronts per SIMD.
+// Stages of a step, a barrier after each: point fields (lane = point of the
+// 3 x 3 x 1 elements), z contraction and, on the fourth wavefront, the nodal
+// planes of the next step contracted to (value, d/dy, d/dz) at the nine
+// (q2, q3) of every pencil (two new planes per step: an element shares one
+// with the step before), y contraction, x contraction and store.
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
 #include "lattice.hpp"
+#include "lattice_product.hpp"
 #include "mhx_internal.hpp"
 #include "thermal.hpp"
 
@@ -74,581 +73,582 @@ __device__ __forceinline__ double sel3(int i, double a0, double a1, double a2) {
   return i == 0 ? a0 : (i == 1 ? a1 : a2);
 }
 
-// LDS copy of the 1-D tables for reads at lane-dependent indices: value and
-// slope of basis i at point q at [i * 3 + q] and [9 + i * 3 + q], points at
-// [18 + q], weights at [21 + q].  (Selecting from the constants per lane
-// would be hoisted out of the step loop and hold ~70 registers for the whole
-// kernel; LDS reads behind the loop's barriers are re-issued instead.)
-constexpr int kTabN = 24;
-
-// Ordering of LDS traffic between the lanes of the kernel's single-wavefront
-// workgroups: a workgroup-scope release / acquire pair restricted to LDS
-// around the barrier.  Fences at wavefront scope did not keep one lane's LDS
-// store ahead of another lane's load in every build; __syncthreads() orders
-// global memory too, i.e. waits for every outstanding store of the scatter at
-// each of the step's stages.
-__device__ __forceinline__ void wave_sync() {
+// LDS-only workgroup barrier: __syncthreads() would also wait for the stores
+// of the step before
+__device__ __forceinline__ void lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
+// LDS traffic between the lanes of one wavefront (LDS operations of a
+// wavefront complete in order; the fences keep the compiler from reordering
+// and wait for outstanding ones)
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
-// The first-touch rule of every entry: the first scheduled unit among those
-// sharing the entry stores it (0/1 on a strong-Dirichlet row), later ones
-// load, add and store; accumulate mode adds everywhere except on Dirichlet
-// rows.  The first scheduled unit runs in an earlier launch than every other,
-// and within one launch an entry has one writer, so the order of additions is
-// the launch order and the sums are reproducible.
+// LDS strides, chosen so that 16 lanes of a read or write meet 16 banks: a pair
+// (Y, Y', Z, Z') sits at z pair * 9 + y pair, a (q1, group) row of pairs has 72
+// slots, a (z block, pencil) of T 73; F is [q3][pencil][q1 + 3 q2]
+constexpr int kSRow = 72;
+constexpr int kSCol = 9 * kSRow;   // a wavefront's pairs
+constexpr int kTPen = 73, kTArr = 6 * kTPen;
 
-// column range of Q2 row coordinate r along an axis of n nodes: first column
-// lo and count len of the row's lattice box
-struct Range {
-  int lo, len;
-};
-__device__ __forceinline__ Range q2_axis(int r, int n) {
-  if (r & 1) return {r - 1, 3};
-  const int lo = r - 2 < 0 ? 0 : r - 2;
-  const int hi = r + 2 > n - 1 ? n - 1 : r + 2;
-  return {lo, hi - lo + 1};
+// three columns j of row i against a field in one z or y direction: BB
+__device__ __forceinline__ void bb3(int i, const double (&f)[3], double (&o)[3]) {
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const double v = kT.B[i][q] * f[q];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) o[j] = q == 0 ? kT.B[j][q] * v : fma(kT.B[j][q], v, o[j]);
+  }
+}
+// o[j] += c D_i D_j f + D_i B_j g
+__device__ __forceinline__ void dd_db3(int i, double c, const double (&f)[3], const double (&g)[3], double (&o)[3]) {
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const double v = kT.D[i][q] * (c * f[q]), w = kT.D[i][q] * g[q];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) o[j] = fma(kT.D[j][q], v, fma(kT.B[j][q], w, o[j]));
+  }
 }
 
 }  // namespace
 
-// MODES: the source has sine modes (their double-precision sin sizes the
-// register file of the whole kernel, so the modeless source has its own build)
+// MODES: the source has sine modes
 template <bool JAC, bool MODES>
-__global__ __launch_bounds__(64) void k_q2box(AsmArgs args) {
-  // the arguments the kernel reads, as scalars: member accesses of the
-  // by-value argument inside the lambdas below made the compiler copy the
-  // whole structure to per-lane scratch memory and read it back from there
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_q2box(AsmArgs args) {
+  // the arguments the kernel reads, as scalars (a lambda naming the by-value
+  // argument would copy the structure to per-lane scratch)
   const double* __restrict__ ga_u = args.u;
   const double* __restrict__ ga_vx = args.vx;
-  const int32_t* __restrict__ ga_rowptr = args.rowptr;
   const uint8_t* __restrict__ ga_fixed = args.fixed;
   const double* __restrict__ ga_k0 = args.coef.k0;
   const double* __restrict__ ga_src = args.coef.src;
   double* const ga_res = args.res;
   double* const ga_jac = args.jac;
-  const double ga_diff_u2 = args.coef.diff_u2;
-  const int ga_n_modes = args.coef.n_modes;
-  const int ga_first_touch = args.first_touch;
-  const int nel0 = args.m.nel[0], nel1 = args.m.nel[1], nel2 = args.m.nel[2];
+  const double diff_u2 = args.coef.diff_u2;
+  const int n_modes = MODES ? args.coef.n_modes : 0;
+  const bool add = args.first_touch == 0;
+  const int n0 = args.m.nel[0], n1 = args.m.nel[1], n2 = args.m.nel[2];
+  const int N0 = 2 * n0 + 1, N1 = 2 * n1 + 1, N2 = 2 * n2 + 1;
   const int nvx0 = args.m.nvx[0], nvx1 = args.m.nvx[1];
-  const int ga_color = args.color, ga_cn0 = args.cn[0], ga_cn1 = args.cn[1], ga_seg = args.gpb, ga_nseg = args.nseg;
-  __shared__ double s_u[45];         // nodal values: x 0..4, y 0..2, z 0..2 of the step
-  __shared__ double s_v[4][3];       // corners: A low, A high, B low, B high
-  // per half: the point fields (alpha_x, alpha_y, alpha_z, beta_x, beta_y,
-  // beta_z at [0, 162); residual fields w|J| flux_c / J_c, w|J| src at
-  // [162, 270)), later overwritten by the products after q2:
-  // [q1][group][i2 * 3 + j2][i3 * 3 + j3]
-  __shared__ double s_a[2][729];
-  __shared__ double s_s1[2][5][81];  // after q3: [group][q1 + 3 q2][i3 * 3 + j3]
-  __shared__ double s_t[kTabN];      // 1-D tables (see kTabN)
-  __shared__ int s_rp[45];           // CRS offsets of the step's rows (-1 - offset: strong Dirichlet row)
-  __shared__ double s_ek[4];         // k0 of A, B; element source of A, B
-  // sine-mode sources: factor sin(w_md x_d(q_d)) (1 where w_md = 0) per
-  // element, mode, axis and 1-D point
-  __shared__ double s_sin[MODES ? 2 : 1][MODES ? MHX_MAX_MODES : 1][3][3];
-  // the sine modes (amplitude, frequencies), copied from the kernel argument
-  // with compile-time indices: indexing the by-value argument with a run-time
-  // mode number changed the code generated for the rest of the kernel (wrong
-  // Jacobians from the second step of a segment on, even with no modes)
-  __shared__ double s_mode[MODES ? MHX_MAX_MODES : 1][4];
 
-  const int lane = threadIdx.x, h = lane >> 5, l = lane & 31;
-  if (lane < 9) {
-    s_t[lane] = sel3(lane / 3, kT.B[0][lane % 3], kT.B[1][lane % 3], kT.B[2][lane % 3]);
-    s_t[9 + lane] = sel3(lane / 3, kT.D[0][lane % 3], kT.D[1][lane % 3], kT.D[2][lane % 3]);
-  } else if (lane < 12) {
-    s_t[18 + lane - 9] = sel3(lane - 9, kT.X[0], kT.X[1], kT.X[2]);
-    s_t[21 + lane - 9] = sel3(lane - 9, kT.W[0], kT.W[1], kT.W[2]);
+  // F: point fields [8][9 pencils][27]; S: [4 wavefronts][q1][group][pair],
+  // then the wavefront's entries on their way out
+  constexpr int kF = JAC ? 8 : 4;
+  __shared__ double s_fs[JAC ? 4 * kSCol : kF * 243];
+  __shared__ double s_t[JAC ? 4 * kTArr : 1];      // [4][zc 2][py 3][z pair 8][q1 + 3 q2]
+  __shared__ double s_tr[3 * 2 * 54];              // residual: [3][z row 2][zc 2][py 3][q1 + 3 q2]
+  __shared__ double s_sr[2][4 * 4 * 3 * 2];        // residual: [step parity][block][line][q1][2]
+  __shared__ double s_pl[3][3][81];                // nodal planes: [X mod 3][value, d/dy, d/dz][pencil][q2 + 3 q3]
+  __shared__ double s_u[2][49];                    // nodes of the next two planes
+  __shared__ double s_mx[MODES ? MHX_MAX_MODES : 1][3];      // sin(w_x x(q1)) of the step
+  __shared__ double s_myz[MODES ? MHX_MAX_MODES : 1][81];    // amplitude and the y, z factors
+
+  __shared__ double s_tab[2][3][3];                // B[q][j], D[q][j]
+  __shared__ double s_mode[MODES ? MHX_MAX_MODES : 1][4];    // amplitude and frequencies
+
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
+  const int nseg = args.nseg, L = args.gpb;
+  int bq = blockIdx.x / nseg;
+  const int x0 = (blockIdx.x - bq * nseg) * L, x1 = min(x0 + L, n0);
+  const int nby = args.cn[1];
+  const int ey0 = 2 * (bq % nby), ez0 = 2 * (bq / nby);
+  const int eb = x0 > 0 ? x0 - 1 : 0;  // first layer: the one before the segment fills the carry
+
+  if (tid < 9) {
+    s_tab[0][tid % 3][tid / 3] = sel3(tid / 3, sel3(tid % 3, kT.B[0][0], kT.B[0][1], kT.B[0][2]),
+                                      sel3(tid % 3, kT.B[1][0], kT.B[1][1], kT.B[1][2]),
+                                      sel3(tid % 3, kT.B[2][0], kT.B[2][1], kT.B[2][2]));
+    s_tab[1][tid % 3][tid / 3] = sel3(tid / 3, sel3(tid % 3, kT.D[0][0], kT.D[0][1], kT.D[0][2]),
+                                      sel3(tid % 3, kT.D[1][0], kT.D[1][1], kT.D[1][2]),
+                                      sel3(tid % 3, kT.D[2][0], kT.D[2][1], kT.D[2][2]));
   }
   if constexpr (MODES) {
+    // (compile-time indices into the by-value argument)
 #pragma unroll
     for (int m = 0; m < MHX_MAX_MODES; ++m)
-      if (lane == m) {
+      if (tid == m) {
         s_mode[m][0] = args.coef.amp[m];
 #pragma unroll
         for (int d = 0; d < 3; ++d) s_mode[m][1 + d] = args.coef.freq[m][d];
       }
   }
-  auto Bq = [&](int i, int q) __attribute__((always_inline)) { return s_t[i * 3 + q]; };
-  auto Dq = [&](int i, int q) __attribute__((always_inline)) { return s_t[9 + i * 3 + q]; };
-  auto Xq = [&](int q) __attribute__((always_inline)) { return s_t[18 + q]; };
-  auto Wq = [&](int q) __attribute__((always_inline)) { return s_t[21 + q]; };
-  int t = blockIdx.x;
-  const int sx = 2 * (t % ga_cn0) + (ga_color & 1);
-  t /= ga_cn0;
-  const int ey = 2 * (t % ga_cn1) + ((ga_color >> 1) & 1);
-  t /= ga_cn1;
-  const int ez = 2 * t + ((ga_color >> 2) & 1);
-  const int L = ga_seg;
-  const int x0 = sx * L;
-  const int x1 = min(x0 + L, nel0);
-  const int nnx = (2 * nel0 + 1), nny = (2 * nel1 + 1), nnzn = (2 * nel2 + 1);
-  // first scheduled unit along each axis among the (at most two) sharing a
-  // vertex plane: even units run first (colour bit 0)
-  const bool flx = sx == 0 || (sx & 1) == 0, fhx = sx == ga_nseg - 1 || (sx & 1) == 0;
-  const bool fly = ey == 0 || (ey & 1) == 0, fhy = ey == nel1 - 1 || (ey & 1) == 0;
-  const bool flz = ez == 0 || (ez & 1) == 0, fhz = ez == nel2 - 1 || (ez & 1) == 0;
-  const int Y0 = 2 * ey, Z0 = 2 * ez;
-
-  // (y, z) column ranges of the pencil's rows (i2, i3 = 0, 1, 2) and the
-  // first-writer flags of their shared (y, z) entries
-  const Range ry0 = q2_axis(Y0, nny), ry1 = q2_axis(Y0 + 1, nny), ry2 = q2_axis(Y0 + 2, nny);
-  const Range rz0 = q2_axis(Z0, nnzn), rz1 = q2_axis(Z0 + 1, nnzn), rz2 = q2_axis(Z0 + 2, nnzn);
-
-  // gather of the step starting at xs into registers: lane < 45 the value
-  // and the CRS offset of node (2 xs + lane % 5, Y0 + lane / 5 % 3, Z0 + lane
-  // / 15), lanes 48..59 the corner coordinates.  The next step's loads are
-  // issued before this step's scatter stores, so their latency overlaps.
-  // Every lane issues its loads on every step, from an address that is
-  // always valid (roles without data of their own read a neighbour's), so
-  // the prefetched registers are defined on all lanes: no value lives across
-  // the step under a lane-divergent definition.
-  double g_val = 0.0;
-  int g_rp = 0;
-  auto fetch = [&](int xs) __attribute__((always_inline)) {
-    const bool hb = xs + 1 < x1;
-    // nodal value and CRS offset (lanes < 45; others repeat node 0)
-    const int li = lane < 45 ? lane : 0;
-    int X = li % 5;
-    if (!hb && X > 2) X = 2;
-    const long node = (2 * xs + X) + (long)nnx * ((Y0 + (li / 5) % 3) + (long)nny * (Z0 + li / 15));
-    const int rp = ga_rowptr[node];
-    const bool fx = ga_fixed[node] != 0;
-    // corner coordinate (lanes 48..59), element coefficient (lanes 60..63)
-    const int lv = lane >= 48 && lane < 60 ? lane - 48 : 0;
-    int v = lv / 3;
-    if (!hb && v >= 2) v -= 2;
-    const int hi = v & 1;
-    const long vid = (long)(xs + (v >> 1) + hi) +
-                     (long)nvx0 * ((long)(ey + hi) + (long)nvx1 * (long)(ez + hi));
-    const long ee = (xs + (hb ? (lane & 1) : 0)) + (long)nel0 * (ey + (long)nel1 * ez);
-    const double* cf = lane < 62 ? ga_k0 : ga_src;
-    const double dflt = lane < 62 ? 1.0 : 0.0;
-    const double* ptr = lane < 48 ? ga_u + node : (lane < 60 ? ga_vx + (vid * 3 + lv % 3) : (cf ? cf + ee : ga_u));
-    const double val = *ptr;
-    g_val = (lane >= 60 && !cf) ? dflt : val;
-    g_rp = fx ? -1 - rp : rp;
+  lds_sync();
+  // ---- roles that hold for the whole walk -------------------------------------
+  // point of the point stage: tid < 243 = q1 + 3 q2 + 9 pencil + 81 q3
+  const int pq = tid < 243 ? tid : 242;
+  const int q1 = pq % 3, q2 = (pq / 3) % 3, q3 = pq / 81, ppen = (pq / 9) % 9;
+  const int pey = ey0 - 1 + ppen % 3, pez = ez0 - 1 + ppen / 3;
+  const bool pact = tid < 243 && pey >= 0 && pey < n1 && pez >= 0 && pez < n2;
+  const int cey = pact ? pey : 0, cez = pact ? pez : 0;
+  auto vert = [&](int x, int y, int z, int d) { return ga_vx[((long)x + (long)nvx0 * (y + (long)nvx1 * z)) * 3 + d]; };
+  const double Jy = 0.5 * (vert(0, cey + 1, 0, 1) - vert(0, cey, 0, 1));
+  const double Jz = 0.5 * (vert(0, 0, cez + 1, 2) - vert(0, 0, cez, 2));
+  const double iJy2 = 1.0 / (Jy * Jy), iJz2 = 1.0 / (Jz * Jz);
+  const double wyz = fabs(Jy * Jz) * sel3(q1, kT.W[0], kT.W[1], kT.W[2]) * sel3(q2, kT.W[0], kT.W[1], kT.W[2]) *
+                     sel3(q3, kT.W[0], kT.W[1], kT.W[2]);
+  double b1[3], d1[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    b1[j] = sel3(q1, kT.B[j][0], kT.B[j][1], kT.B[j][2]);
+    d1[j] = sel3(q1, kT.D[j][0], kT.D[j][1], kT.D[j][2]);
+  }
+  // plane stage: the last wavefront, lane < 54 = q3 + 3 pencil + 27 plane
+  const int ll = lane < 54 ? lane : 53;
+  const int lq3 = ll % 3, lpen = (ll / 3) % 9, lpl = ll / 27;
+  const int lnode = 2 * (lpen % 3) + 7 * 2 * (lpen / 3);
+  // node of the gather: tid < 98 = plane * 49 + y + 7 z (nodes off the mesh: 0)
+  const int gpl = tid / 49, gn = tid % 49;
+  const int gY = 2 * ey0 - 2 + gn % 7, gZ = 2 * ez0 - 2 + gn / 7;
+  const bool gin = tid < 98 && gY >= 0 && gY < N1 && gZ >= 0 && gZ < N2;
+  const long gbase = gin ? (long)N0 * (gY + (long)N1 * gZ) : 0;
+  // z and y contractions: 1 / J^2 of the low and high element
+  auto inv_j2 = [&](int e, int n, int axis) {
+    const int c = e < 0 ? 0 : (e >= n ? n - 1 : e);
+    const double j = axis == 1 ? 0.5 * (vert(0, c + 1, 0, 1) - vert(0, c, 0, 1))
+                               : 0.5 * (vert(0, 0, c + 1, 2) - vert(0, 0, c, 2));
+    return 1.0 / (j * j);
   };
-  fetch(x0);
+  const int zt = lane < 54 ? lane : 53;  // (zc, py, q12)
+  const int zq = zt % 9, zpy = (zt / 9) % 3, zzc = zt / 27;
+  const double cz_lo = inv_j2(ez0 - 1 + zzc, n2, 2), cz_hi = inv_j2(ez0 + zzc, n2, 2);
+  const int yt = lane < 48 ? lane : 47;  // q1, z pair, block: wavefronts 0, 2: zc = 0, 1, 3: zc = 1
+  const int yq1 = yt % 3, yzp = (yt / 3) % 8, yyc = yt / 24, yzc = wv & 1;
+  const double cy_lo = inv_j2(ey0 - 1 + yyc, n1, 1), cy_hi = inv_j2(ey0 + yyc, n1, 1);
 
-  // the step-to-step carry of B's last-plane rows (their Jacobian runs of the
-  // three last rounds, their residuals), held by the half-1 lanes in
-  // registers and read by the half-0 lanes of the next step through
-  // cross-half lane exchanges
-  double carry_j[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
-  double carry_r = 0.0;
-  for (int xa = x0; xa < x1; xa += 2) {
-    const bool hasB = xa + 1 < x1;
-    const bool act = h == 0 || hasB;
-    const int ex = xa + h;
-    const long e = ex + (long)nel0 * (ey + (long)nel1 * ez);
-    const bool first_step = xa == x0, last_step = xa + 2 >= x1;
-
-    // 1. gather ---------------------------------------------------------------
-    wave_sync();  // the previous step's LDS reads are done
-    if (lane < 45) {
-      s_u[lane] = g_val;
-      s_rp[lane] = g_rp;
-    } else if (lane >= 48 && lane < 60) {
-      s_v[(lane - 48) / 3][(lane - 48) % 3] = g_val;
-    } else if (lane >= 60) {
-      s_ek[lane - 60] = g_val;
+  // last stage: block (ey, ez) of the wavefront (yc = wv & 1, zc = wv >> 1),
+  // its row lines j = jy + 2 jz with nr column lines each, one pair per lane
+  const int ey = ey0 + (wv & 1), ez = ez0 + (wv >> 1);
+  const bool own = ey <= n1 && ez <= n2;
+  const unsigned T0 = 8u * n0 + 1, T1 = 8u * n1 + 1;
+  const int EYv = !own ? 0 : (ey > 0 && ey < n1 ? 5 : 3), EYm = own && ey < n1 ? 3 : 0;
+  const int EZv = !own ? 0 : (ez > 0 && ez < n2 ? 5 : 3), EZm = own && ez < n2 ? 3 : 0;
+  const int nr0 = EYv * EZv, nr1 = EYm * EZv, nr2 = EYv * EZm, nr3 = EYm * EZm;
+  const int lb_1 = nr0, lb_2 = lb_1 + nr1, lb_3 = lb_2 + nr2, lb_4 = lb_3 + nr3;  // first lanes, total
+  const unsigned zv = (unsigned)q2_prefix(2 * ez) * T1 * T0, zm = (unsigned)q2_prefix(2 * ez + 1) * T1 * T0;
+  const unsigned yv = (unsigned)q2_prefix(2 * ey) * T0, ym = (unsigned)q2_prefix(2 * ey + 1) * T0;
+  const unsigned line0 = zv + EZv * yv, line1 = zv + EZv * ym, line2 = zm + EZm * yv, line3 = zm + EZm * ym;
+  const int pj = (lane >= lb_1) + (lane >= lb_2) + (lane >= lb_3);
+  const int pt = lane - (pj == 0 ? 0 : pj == 1 ? lb_1 : pj == 2 ? lb_2 : lb_3);
+  const int pEY = (pj & 1) ? 3 : (EYv ? EYv : 3);
+  const int piy = pt % pEY, piz = pt / pEY;
+  const int pyp = (pj & 1) ? 5 + piy : (ey == 0 ? 2 + piy : piy);  // assembled pair 0..7 of the axis
+  const int pzp = (pj >> 1) ? 5 + piz : (ez == 0 ? 2 + piz : piz);
+  const bool pair = lane < lb_4;
+  const int canon = pair ? pzp * 9 + pyp : 0;
+  const bool dnode = pyp == ((pj & 1) ? 6 : 2) && pzp == ((pj >> 1) ? 6 : 2);
+  const int pnr = pj == 0 ? nr0 : pj == 1 ? nr1 : pj == 2 ? nr2 : nr3;
+  const int plb = lane - pt;
+  const long prow = (long)N0 * ((2 * ey + (pj & 1)) + (long)N1 * (2 * ez + (pj >> 1)));
+  // this lane's entries of a full step on their way out (index lane + 64 s of
+  // the 8 lb_4 staged ones): CRS position at layer e = goff + e * ginc
+  unsigned goff[8], ginc[8];
+  if constexpr (JAC) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int idx = lane + 64 * s;
+      const int j = (idx >= 8 * lb_1) + (idx >= 8 * lb_2) + (idx >= 8 * lb_3);
+      const int nr = j == 0 ? nr0 : j == 1 ? nr1 : j == 2 ? nr2 : nr3;
+      const int lb = j == 0 ? 0 : j == 1 ? lb_1 : j == 2 ? lb_2 : lb_3;
+      goff[s] = (j == 0 ? line0 : j == 1 ? line1 : j == 2 ? line2 : line3) + (unsigned)(idx - 8 * lb - 2 * nr);
+      ginc[s] = 8u * nr;
     }
-    wave_sync();
-    // the LDS stores above read the registers the next gather loads into:
-    // they complete before those loads are issued
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    if (xa + 2 < x1) fetch(xa + 2);
+  }
 
-    // read-backs.  The scatters add to what is stored (later touches of rows
-    // that are not strong Dirichlet rows).  The runs of one step are entries
-    // no other run of the wavefront touches (shared-plane sums go through
-    // lane exchanges and the step-to-step carry), so a batch of loads can go
-    // before the stores; a load issued after a store waits for that store,
-    // so each batch is issued as early as its compute allows.
-    //
-    // residual: lane (l < 27) = row (i1, i2, i3) of its half's element
-    const int il[3] = {l % 3, (l / 3) % 3, l / 9};
-    bool r_write = false, r_first = true, r_fixed = false;
-    long r_row = 0;
-    double r_old = 0.0;
-    if (ga_res && act && l < 27) {
-      const int i1 = il[0];
-      const int X = 2 * ex + i1, Y = Y0 + il[1], Z = Z0 + il[2];
-      bool xsh = false, xfirst = true;
-      r_write = true;
-      if (h == 0 && i1 == 2) {
-        if (!hasB && x1 < nel0) xsh = true, xfirst = fhx;
-      } else if (h == 0 && i1 == 0) {
-        if (first_step && x0 > 0) xsh = true, xfirst = flx;
-      } else if (h == 1 && i1 == 0) {
-        r_write = false;  // summed into A's row
-      } else if (h == 1 && i1 == 2) {
-        r_write = last_step;  // otherwise carried to the next step
-        if (last_step && x1 < nel0) xsh = true, xfirst = fhx;
+  if constexpr (MODES) {
+    for (int k = tid; k < n_modes * 81; k += 256) {
+      const int m = k / 81, p = k % 81, pen = p / 9, a2 = p % 3, a3 = (p / 3) % 3;
+      const int my = ey0 - 1 + pen % 3, mz = ez0 - 1 + pen / 3;
+      double f = s_mode[m][0];
+      const double wy = s_mode[m][2], wz = s_mode[m][3];
+      if (my >= 0 && my < n1 && mz >= 0 && mz < n2) {
+        const double v0 = vert(0, my, 0, 1), j = 0.5 * (vert(0, my + 1, 0, 1) - v0);
+        const double v1 = vert(0, 0, mz, 2), jz = 0.5 * (vert(0, 0, mz + 1, 2) - v1);
+        if (wy != 0.0) f *= sin(wy * fma(sel3(a2, kT.X[0], kT.X[1], kT.X[2]) + 1.0, j, v0));
+        if (wz != 0.0) f *= sin(wz * fma(sel3(a3, kT.X[0], kT.X[1], kT.X[2]) + 1.0, jz, v1));
       }
-      r_row = X + (long)nnx * (Y + (long)nny * Z);
-      const bool ysh = il[1] != 1, zsh = il[2] != 1;
-      r_first = ga_first_touch && (!xsh || xfirst) && (!ysh || (il[1] == 0 ? fly : fhy)) &&
-                (!zsh || (il[2] == 0 ? flz : fhz));
-      r_fixed = s_rp[(X - 2 * xa) + 5 * il[1] + 15 * il[2]] < 0;
-      if (r_write && !r_fixed && !r_first) r_old = ga_res[r_row];
+      s_myz[m][p] = f;
     }
-    // 2. point stage (lane = cubature point) ------------------------------------
-    double Jc[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) Jc[d] = 0.5 * (s_v[2 * h + 1][d] - s_v[2 * h][d]);
-    const double detJ = fabs(Jc[0] * Jc[1] * Jc[2]);
-    // 1 / J_c once per element: the point stage multiplies (one division
-    // per axis instead of four per axis and point)
-    double iJ[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) iJ[d] = 1.0 / Jc[d];
+  }
+  // x factors of the sine modes at layer e
+  auto mode_x = [&](int e) __attribute__((always_inline)) {
     if constexpr (MODES) {
-      // the sine factors of the source, in a stage of their own: the
-      // double-precision sin needs many registers, and here few others are live
-      const int nf = ga_n_modes * 9;
-      for (int t = l; t < nf; t += 32) {
-        const int m = t / 9, d = (t / 3) % 3, q = t % 3;
-        const double w = s_mode[m][1 + d];
-        const double xd = fma(Xq(q) + 1.0, Jc[d], s_v[2 * h][d]);
-        s_sin[h][m][d][q] = w != 0.0 ? sin(w * xd) : 1.0;
+      const int k = tid - 192;
+      if (k >= 0 && k < 3 * n_modes) {
+        const int m = k / 3, a = k % 3;
+        const double wx = s_mode[m][1];
+        const double v0 = vert(e, 0, 0, 0), j = 0.5 * (vert(e + 1, 0, 0, 0) - v0);
+        s_mx[m][a] = wx != 0.0 ? sin(wx * fma(sel3(a, kT.X[0], kT.X[1], kT.X[2]) + 1.0, j, v0)) : 1.0;
       }
-      wave_sync();
     }
-    if (act && l < 27) {
-      const int qv[3] = {l % 3, (l / 3) % 3, l / 9};
-      double b[3][3], dd[3][3];  // [axis][j] = l_0(j, q_axis), l_1(j, q_axis)
+  };
+  // contraction of a nodal plane (X mod 3 = slot) from s_u[pl]: one (pencil,
+  // q3) a lane, all three q2 (their tables at compile time)
+  auto plane = [&](int pl, int slot) __attribute__((always_inline)) {
+    double v[3] = {0.0, 0.0, 0.0}, vy[3] = {0.0, 0.0, 0.0}, vz[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-      for (int ax = 0; ax < 3; ++ax)
+    for (int j3 = 0; j3 < 3; ++j3) {
+      double un[3];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          b[ax][j] = Bq(j, qv[ax]);
-          dd[ax][j] = Dq(j, qv[ax]);
-        }
-      // u and its reference gradient by sum factorisation over the nodes
-      double U = 0.0, G[3] = {0.0, 0.0, 0.0};
+      for (int j2 = 0; j2 < 3; ++j2) un[j2] = s_u[pl][lnode + j2 + 7 * j3];
+      const double b3 = s_tab[0][lq3][j3], d3 = s_tab[1][lq3][j3];
 #pragma unroll
-      for (int j3 = 0; j3 < 3; ++j3) {
-        double cu = 0.0, cx = 0.0, cy = 0.0;
+      for (int q = 0; q < 3; ++q) {
+        double a = 0.0, ay = 0.0;
 #pragma unroll
         for (int j2 = 0; j2 < 3; ++j2) {
-          double au = 0.0, axx = 0.0;
-#pragma unroll
-          for (int j1 = 0; j1 < 3; ++j1) {
-            const double uj = s_u[2 * h + j1 + 5 * j2 + 15 * j3];
-            au = fma(b[0][j1], uj, au);
-            axx = fma(dd[0][j1], uj, axx);
-          }
-          cu = fma(b[1][j2], au, cu);
-          cx = fma(b[1][j2], axx, cx);
-          cy = fma(dd[1][j2], au, cy);
+          a = fma(kT.B[j2][q], un[j2], a);
+          ay = fma(kT.D[j2][q], un[j2], ay);
         }
-        U = fma(b[2][j3], cu, U);
-        G[0] = fma(b[2][j3], cx, G[0]);
-        G[1] = fma(b[2][j3], cy, G[1]);
-        G[2] = fma(dd[2][j3], cu, G[2]);
+        v[q] = fma(b3, a, v[q]);
+        vy[q] = fma(b3, ay, vy[q]);
+        vz[q] = fma(d3, a, vz[q]);
       }
-      const double w = detJ * Wq(qv[0]) * Wq(qv[1]) * Wq(qv[2]);
-      const double k0 = s_ek[h];
-      // thermal source: element value plus the sine modes (thermal_source in
-      // thermal.hpp, the same products in the same order)
-      double f = s_ek[2 + h];
-      if constexpr (MODES) {
-        for (int m = 0; m < ga_n_modes; ++m) {
-          double tm = s_mode[m][0];
-#pragma unroll
-          for (int d = 0; d < 3; ++d)
-            if (s_mode[m][1 + d] != 0.0) tm = tm * s_sin[h][m][d][qv[d]];
-          f += tm;
-        }
-      }
-      // physics in dual arithmetic, slots 0..2 = d/d(grad u)_c, 3 = d/du
-      QDual<4> Ud = qd_seed<4>(U, 3);
-      QDual<4> Gd[3];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) Gd[c] = qd_seed<4>(G[c] * iJ[c], c);
-      QDual<4> flux[3], src;
-      ThermalPhysics::volume<3>(k0, ga_diff_u2, f, Ud, Gd, flux, src);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        s_a[h][162 + 27 * c + l] = w * flux[c].v * iJ[c];
-        if constexpr (JAC) {
-          s_a[h][27 * c + l] = w * flux[c].d[c] * (iJ[c] * iJ[c]);
-          s_a[h][27 * (3 + c) + l] = w * flux[c].d[3] * iJ[c];
-        }
-      }
-      s_a[h][162 + 81 + l] = w * src.v;
     }
-    wave_sync();
-
-    // 3. residual (lane = test function i) and the first contraction ------------
-    double R = 0.0;
-    if (act && l < 27 && ga_res) {
-      double bi[3][3], di[3][3];  // [axis][q]
 #pragma unroll
-      for (int ax = 0; ax < 3; ++ax)
+    for (int q = 0; q < 3; ++q) {
+      const int o = lpen * 9 + 3 * lq3 + q;
+      s_pl[slot][0][o] = v[q];
+      s_pl[slot][1][o] = vy[q];
+      s_pl[slot][2][o] = vz[q];
+    }
+  };
+
+  // ---- planes 2 eb, 2 eb + 1, 2 eb + 2 -----------------------------------------
+  if (tid < 49) s_u[0][gn] = gin ? ga_u[gbase + 2 * eb] : 0.0;
+  lds_sync();
+  if (wv == 3 && lane < 27) plane(0, (2 * eb) % 3);
+  lds_sync();
+  if (tid < 98) s_u[gpl][gn] = gin ? ga_u[gbase + 2 * eb + 1 + gpl] : 0.0;
+  mode_x(eb);
+  lds_sync();
+  if (wv == 3 && lane < 54) plane(lpl, (2 * eb + 1 + lpl) % 3);
+  // values of the next layer, one step ahead
+  const long ce0 = (long)n0 * (cey + (long)n1 * cez);
+  double k0n = ga_k0 ? ga_k0[ce0 + eb] : 1.0, srn = ga_src ? ga_src[ce0 + eb] : 0.0;
+  double un = 0.0;
+  if (eb + 1 < x1 && gin) un = ga_u[gbase + 2 * eb + 3 + gpl];
+  lds_sync();
+
+  double carry[3] = {0.0, 0.0, 0.0};
+  for (int e = eb; e < x1; ++e) {
+    const bool emit = e >= x0;
+    // 1. point fields ---------------------------------------------------------------
+    const double vxl = ga_vx[3 * (long)e], vxh = ga_vx[3 * (long)(e + 1)];
+    const double Jx = 0.5 * (vxh - vxl), iJx2 = 1.0 / (Jx * Jx);
+    if (tid < 243) {
+      const double k0 = k0n;
+      double f = srn;
+      const int pp = ppen * 9 + q2 + 3 * q3;
+      double U = 0.0, Gx = 0.0, Gy = 0.0, Gz = 0.0;
+      int slot = (2 * e) % 3;
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const double v = s_pl[slot][0][pp], vy = s_pl[slot][1][pp], vz = s_pl[slot][2][pp];
+        U = fma(b1[j], v, U);
+        Gx = fma(d1[j], v, Gx);
+        Gy = fma(b1[j], vy, Gy);
+        Gz = fma(b1[j], vz, Gz);
+        slot = slot == 2 ? 0 : slot + 1;
+      }
+      // (pencils outside the mesh share nodes with it)
+      if (!pact) U = Gx = Gy = Gz = 0.0;
+      if constexpr (MODES) {
+        for (int m = 0; m < n_modes; ++m) f = fma(s_myz[m][pp], s_mx[m][q1], f);
+      }
+      // k = k0 (1 + a u^2) and k' (ThermalPhysics in thermal.hpp)
+      const double w = pact ? wyz * fabs(Jx) : 0.0;
+      const double wk0 = w * k0;
+      const double kap = wk0 * fma(diff_u2 * U, U, 1.0);
+      const double gx = Gx * iJx2, gy = Gy * iJy2, gz = Gz * iJz2;
+      double* F = s_fs + tid;
+      F[0] = kap * gx;
+      F[243] = kap * gy;
+      F[2 * 243] = kap * gz;
+      F[3 * 243] = -w * f;
+      if constexpr (JAC) {
+        const double wkp = wk0 * (2.0 * diff_u2 * U);
+        F[4 * 243] = kap;
+        F[5 * 243] = wkp * gx;
+        F[6 * 243] = wkp * gy;
+        F[7 * 243] = wkp * gz;
+      }
+    }
+    // the gathered nodes of the next planes; coefficients of the next layer
+    if (tid < 98) s_u[gpl][gn] = un;
+    if (e + 1 < x1) {
+      if (ga_k0) k0n = ga_k0[ce0 + e + 1];
+      if (ga_src) srn = ga_src[ce0 + e + 1];
+    }
+    lds_sync();
+
+    // 2. z contraction: wavefront 0 vertex rows (low and high element), 1
+    // interior rows, 2 the residual, 3 the planes of the next step ------------------------
+    if (e + 1 < x1) {
+      if (wv == 3 && lane < 54) plane(lpl, (2 * e + 3 + lpl) % 3);
+      if (e + 2 < x1 && gin) un = ga_u[gbase + 2 * e + 5 + gpl];
+    }
+    if (JAC && wv < 2 && lane < 54) {
+      const double* Flo = s_fs + 4 * 243 + (zpy + 3 * zzc) * 9 + zq;  // low element; the high one 27 on
+      auto contract = [&](int i, const double* Fe, double cz, double (&o)[4][3]) __attribute__((always_inline)) {
+        double f[4][3];
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int q = 0; q < 3; ++q) f[a][q] = Fe[a * 243 + 81 * q];
+        bb3(i, f[0], o[0]);
+        bb3(i, f[1], o[1]);
+        bb3(i, f[2], o[2]);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) o[3][j] = 0.0;
+        dd_db3(i, cz, f[0], f[3], o[3]);
+      };
+      double* Td = s_t + (zzc * 3 + zpy) * kTPen + zq;
+      double hi[4][3];
+      if (wv == 0) {
+        double lo[4][3];
+        contract(2, Flo, cz_lo, lo);
+        contract(0, Flo + 27, cz_hi, hi);
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          Td[a * kTArr] = lo[a][0];
+          Td[a * kTArr + 9] = lo[a][1];
+          Td[a * kTArr + 18] = lo[a][2] + hi[a][0];
+          Td[a * kTArr + 27] = hi[a][1];
+          Td[a * kTArr + 36] = hi[a][2];
+        }
+      } else {
+        contract(1, Flo + 27, cz_hi, hi);
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) Td[a * kTArr + 9 * (5 + j)] = hi[a][j];
+      }
+    }
+    if (wv == 2 && lane < 54 && ga_res) {
+      const double* Flo = s_fs + (zpy + 3 * zzc) * 9 + zq;
+      double v[3] = {0.0, 0.0, 0.0}, m[3] = {0.0, 0.0, 0.0};  // x, y, value rows
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const double* lo = Flo + 81 * q;
+        const double* hi = lo + 27;
+        const double hx = hi[0], hy = hi[243], hz = hi[2 * 243], hs = hi[3 * 243];
+        v[0] = fma(kT.B[2][q], lo[0], fma(kT.B[0][q], hx, v[0]));
+        v[1] = fma(kT.B[2][q], lo[243], fma(kT.B[0][q], hy, v[1]));
+        v[2] = fma(kT.D[2][q], lo[2 * 243], fma(kT.D[0][q], hz, v[2]));
+        v[2] = fma(kT.B[2][q], lo[3 * 243], fma(kT.B[0][q], hs, v[2]));
+        m[0] = fma(kT.B[1][q], hx, m[0]);
+        m[1] = fma(kT.B[1][q], hy, m[1]);
+        m[2] = fma(kT.D[1][q], hz, fma(kT.B[1][q], hs, m[2]));
+      }
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        s_tr[a * 108 + lane] = v[a];
+        s_tr[a * 108 + 54 + lane] = m[a];
+      }
+    }
+    lds_sync();
+
+    // 3. y contraction: wavefronts 0, 1 vertex rows, 2, 3 interior rows (lanes 48..
+    // of 2 and 3: the residual) ----------------------------------------------------
+    if (JAC && lane < 48) {
+      const double* Tlo = s_t + (yzc * 3 + yyc) * kTPen + yzp * 9 + yq1;  // low element; the high one kTPen on
+      auto contract = [&](int i, const double* Te, double cy, double (&o)[3][3]) __attribute__((always_inline)) {
+        double f[4][3];
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int q = 0; q < 3; ++q) f[a][q] = Te[a * kTArr + 3 * q];
+        bb3(i, f[0], o[0]);
+        bb3(i, f[1], o[1]);
+        bb3(i, f[3], o[2]);
+        dd_db3(i, cy, f[0], f[2], o[2]);
+      };
+      double* Sd = s_fs + (yyc + 2 * yzc) * kSCol + yq1 * 3 * kSRow + yzp * 9;
+      double hi[3][3];
+      if (wv < 2) {
+        double lo[3][3];
+        contract(2, Tlo, cy_lo, lo);
+        contract(0, Tlo + kTPen, cy_hi, hi);
+#pragma unroll
+        for (int g = 0; g < 3; ++g) {
+          Sd[g * kSRow] = lo[g][0];
+          Sd[g * kSRow + 1] = lo[g][1];
+          Sd[g * kSRow + 2] = lo[g][2] + hi[g][0];
+          Sd[g * kSRow + 3] = hi[g][1];
+          Sd[g * kSRow + 4] = hi[g][2];
+        }
+      } else {
+        contract(1, Tlo + kTPen, cy_hi, hi);
+#pragma unroll
+        for (int g = 0; g < 3; ++g)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) Sd[g * kSRow + 5 + j] = hi[g][j];
+      }
+    }
+    if (wv >= 2 && lane >= 48 && lane < 60 && ga_res) {
+      const int r = lane - 48;  // q1, z row, yc; zc = wv & 1
+      const int a1 = r % 3, zr = (r / 3) % 2, yc = r / 6;
+      const double* Tl = s_tr + zr * 54 + ((wv & 1) * 3 + yc) * 9 + a1;  // low element; the high one 9 on
+      double vx = 0.0, v0 = 0.0, mx = 0.0, m0 = 0.0;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const double* lo = Tl + 3 * q;
+        const double* hi = lo + 9;
+        vx = fma(kT.B[2][q], lo[0], fma(kT.B[0][q], hi[0], vx));
+        v0 = fma(kT.D[2][q], lo[108], fma(kT.D[0][q], hi[108], v0));
+        v0 = fma(kT.B[2][q], lo[216], fma(kT.B[0][q], hi[216], v0));
+        mx = fma(kT.B[1][q], hi[0], mx);
+        m0 = fma(kT.D[1][q], hi[108], fma(kT.B[1][q], hi[216], m0));
+      }
+      double* o = s_sr[e & 1] + ((yc + 2 * (wv & 1)) * 4 + 2 * zr) * 6 + a1 * 2;
+      o[0] = vx;
+      o[1] = v0;
+      o[6] = mx;
+      o[7] = m0;
+    }
+    lds_sync();
+
+    // 4. x contraction and store ------------------------------------------------------------
+    if (e + 1 < x1) mode_x(e + 1);
+    // residual rows 2e and 2e + 1 of the 16 row lines: one wavefront per step in turn
+    const bool last = e + 1 == n0;
+    if (ga_res && emit && wv == (e & 3) && lane < 16) {
+      const int b = lane >> 2, j = lane & 3;
+      const int ry = ey0 + (b & 1), rz = ez0 + (b >> 1);
+      const int Y = 2 * ry + (j & 1), Z = 2 * rz + (j >> 1);
+      if (Y < N1 && Z < N2) {
+        const double* cur = s_sr[e & 1] + lane * 6;
+        const double* old = s_sr[(e & 1) ^ 1] + lane * 6;
+        double r0 = 0.0, r1 = 0.0, r2 = 0.0;
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-          bi[ax][q] = Bq(il[ax], q);
-          di[ax][q] = Dq(il[ax], q);
+          const double cx = cur[2 * q], c0 = cur[2 * q + 1];
+          r0 = fma(kT.D[0][q], cx, fma(kT.B[0][q], c0, r0));
+          r1 = fma(kT.D[1][q], cx, fma(kT.B[1][q], c0, r1));
+          r2 = fma(kT.D[2][q], cx, fma(kT.B[2][q], c0, r2));
+          if (e > 0) r0 = fma(kT.D[2][q], old[2 * q], fma(kT.B[2][q], old[2 * q + 1], r0));
         }
+        const long row = 2 * (long)e + (long)N0 * (Y + (long)N1 * Z);
+        const double rr[3] = {r0, r1, r2};
 #pragma unroll
-      for (int q3 = 0; q3 < 3; ++q3) {
-        double tv = 0.0, tz = 0.0;
-#pragma unroll
-        for (int q2 = 0; q2 < 3; ++q2) {
-          double svx = 0.0, sy = 0.0, sz = 0.0;
-#pragma unroll
-          for (int q1 = 0; q1 < 3; ++q1) {
-            const int q = q1 + 3 * q2 + 9 * q3;
-            const double* fr = &s_a[h][162];
-            svx = fma(bi[0][q1], fr[81 + q], fma(di[0][q1], fr[q], svx));
-            sy = fma(bi[0][q1], fr[27 + q], sy);
-            sz = fma(bi[0][q1], fr[54 + q], sz);
-          }
-          tv = fma(bi[1][q2], svx, fma(di[1][q2], sy, tv));
-          tz = fma(bi[1][q2], sz, tz);
-        }
-        R = fma(bi[2][q3], tv, fma(di[2][q3], tz, R));
-      }
-    }
-    if constexpr (JAC) {
-      // q3 contraction: task (q1 + 3 q2, i3), outputs j3 = 0..2 of the five groups
-      if (act && l < 27) {
-        const int qq = l % 9, i3 = l / 9;
-        double vax[3], vbx[3], vay[3], vby[3], vaz[3], vbz[3];
-#pragma unroll
-        for (int q3 = 0; q3 < 3; ++q3) {
-          const double bb = Bq(i3, q3), db = Dq(i3, q3);
-          const int q = qq + 9 * q3;
-          vax[q3] = bb * s_a[h][q];
-          vay[q3] = bb * s_a[h][27 + q];
-          vaz[q3] = db * s_a[h][54 + q];
-          vbx[q3] = bb * s_a[h][81 + q];
-          vby[q3] = bb * s_a[h][108 + q];
-          vbz[q3] = db * s_a[h][135 + q];
-        }
-#pragma unroll
-        for (int j3 = 0; j3 < 3; ++j3) {
-          double g30 = 0.0, g10 = 0.0, g03 = 0.0, g01 = 0.0, g00 = 0.0;
-#pragma unroll
-          for (int q3 = 0; q3 < 3; ++q3) {
-            const double bj = kT.B[j3][q3], dj = kT.D[j3][q3];
-            g30 = fma(bj, vax[q3], g30);
-            g10 = fma(bj, vbx[q3], g10);
-            g03 = fma(bj, vay[q3], g03);
-            g01 = fma(bj, vby[q3], g01);
-            g00 = fma(dj, vaz[q3], fma(bj, vbz[q3], g00));
-          }
-          const int p3 = 3 * i3 + j3;
-          s_s1[h][0][qq * 9 + p3] = g30;
-          s_s1[h][1][qq * 9 + p3] = g10;
-          s_s1[h][2][qq * 9 + p3] = g03;
-          s_s1[h][3][qq * 9 + p3] = g01;
-          s_s1[h][4][qq * 9 + p3] = g00;
-        }
-      }
-    }
-
-    // residual scatter: A's x-plane 2 + B's x-plane 0 summed; A's x-plane 0
-    // takes the carry of the previous step's B; B's x-plane 2 is carried
-    if (ga_res) {
-      const int i1 = il[0];
-      // lanes of the partner rows in the other half (same i2, i3)
-      const int srcA2 = 32 + l - 2;  // half 0, i1 == 2: B's row with i1 == 0
-      const int srcA0 = 32 + l + 2;  // half 0, i1 == 0: the carried row of B with i1 == 2
-      const double fromB = __shfl(R, (h == 0 && l < 27 && i1 == 2) ? srcA2 : lane, 64);
-      const double cprev = __shfl(carry_r, (h == 0 && l < 27 && i1 == 0) ? srcA0 : lane, 64);
-      carry_r = (h == 1 && l < 27 && i1 == 2 && act) ? R : carry_r;
-      if (act && l < 27) {
-        double v = R;
-        if (h == 0 && i1 == 2 && hasB) v = R + fromB;
-        else if (h == 0 && i1 == 0 && !first_step) v = cprev + R;
-        // strong Dirichlet row: 0, written by its first toucher
-        if (r_write && (!r_fixed || r_first)) ga_res[r_row] = r_fixed ? 0.0 : (r_first ? -v : r_old - v);
-      }
-    }
-    if constexpr (!JAC) continue;
-
-    // 4. q2 contraction for the three q1 slices ---------------------------------
-    wave_sync();  // s_s1 complete; the point and residual fields are read
-    if (act && l < 27) {
-      // task (p3, i2), outputs j2 = 0..2 of the three groups
-      const int p3 = l % 9, i2 = l / 9;
-      const double bb[3] = {Bq(i2, 0), Bq(i2, 1), Bq(i2, 2)}, db[3] = {Dq(i2, 0), Dq(i2, 1), Dq(i2, 2)};
-#pragma unroll 1
-      for (int q1 = 0; q1 < 3; ++q1) {
-        double v30[3], v10[3], v03[3], v01[3];
-#pragma unroll
-        for (int q2 = 0; q2 < 3; ++q2) {
-          const int o = (q1 + 3 * q2) * 9 + p3;
-          v30[q2] = bb[q2] * s_s1[h][0][o];
-          v10[q2] = bb[q2] * s_s1[h][1][o];
-          v03[q2] = db[q2] * s_s1[h][2][o];
-          v01[q2] = fma(db[q2], s_s1[h][3][o], bb[q2] * s_s1[h][4][o]);
-        }
-        double* s2 = &s_a[h][q1 * 243];
-#pragma unroll
-        for (int j2 = 0; j2 < 3; ++j2) {
-          double c3 = 0.0, c1 = 0.0, c0 = 0.0;
-#pragma unroll
-          for (int q2 = 0; q2 < 3; ++q2) {
-            const double bj = kT.B[j2][q2], dj = kT.D[j2][q2];
-            c3 = fma(bj, v30[q2], c3);
-            c1 = fma(bj, v10[q2], c1);
-            c0 = fma(dj, v03[q2], fma(bj, v01[q2], c0));
-          }
-          const int o = (3 * i2 + j2) * 9 + p3;
-          s2[o] = c3;
-          s2[81 + o] = c1;
-          s2[162 + o] = c0;
-        }
-      }
-    }
-    wave_sync();
-
-    // 5. q1 contraction and Jacobian scatter ---------------------------------
-    // Jacobian read-backs, all issued before the first store.  Round r: tasks pp = l + 32 (r % 3) = j2 + 3
-    // j3 + 9 i2 + 27 i3 < 81, rows i1 = (h ? m : 2 - m), m = r / 3; each lane
-    // writes n consecutive columns of its row from column ox, at g_off[r];
-    // g_meta[r] = n | ox << 3 | fixed << 6 | go << 7 | firstm << 8 (fixed:
-    // strong Dirichlet row; go: the lane writes in this round; firstm bit k:
-    // the lane writes column k first)
-    double old[9][5];
-    unsigned g_off[9], g_meta[9];
-    if constexpr (JAC) {
-#pragma unroll
-    for (int r = 0; r < 9; ++r) {
-      const int m = r / 3, pp = l + 32 * (r % 3);
-      const bool task = act && pp < 81;
-      const int i1 = h ? m : 2 - m;
-      const int j2 = pp % 3, j3 = (pp / 3) % 3, i2 = (pp / 9) % 3, i3 = pp / 27;
-      int n = 3, ox = 0;
-      bool xs_lo = false, xs_hi = false;  // first / last column shared with another segment
-      bool go = task && ga_jac != nullptr;
-      const int X = 2 * ex + i1;
-      if (m == 0) {
-        if (h == 0) {
-          if (!hasB) xs_hi = x1 < nel0;
-        } else {
-          n = 2, ox = 3;
-        }
-      } else if (m == 2) {
-        if (h == 0) {
-          if (!first_step) {
-            n = 5;
+        for (int k = 0; k < 3; ++k) {
+          if (k == 2 && !last) continue;
+          const bool fx = ga_fixed[row + k] != 0;
+          if (add) {
+            if (!fx) ga_res[row + k] -= rr[k];
           } else {
-            ox = X >= 2 ? 2 : 0;
-            xs_lo = x0 > 0;
+            ga_res[row + k] = fx ? 0.0 : -rr[k];
           }
-        } else {
-          go = go && last_step;  // otherwise carried to the next step
-          xs_hi = x1 < nel0;
         }
       }
-      const int rpl = s_rp[(X - 2 * xa) + 5 * i2 + 15 * i3];
-      const bool fixed = rpl < 0;
-      const int rp = fixed ? -1 - rpl : rpl;
-      const int lx = (X & 1) ? 3 : ((X == 0 || X == 2 * nel0) ? 3 : 5);
-      // (scalar selects: selecting a Range structure by a lane value would
-      // place the structures in scratch memory)
-      const int ylo = i2 == 0 ? ry0.lo : (i2 == 1 ? ry1.lo : ry2.lo);
-      const int ylen = i2 == 0 ? ry0.len : (i2 == 1 ? ry1.len : ry2.len);
-      const int zlo = i3 == 0 ? rz0.lo : (i3 == 1 ? rz1.lo : rz2.lo);
-      const unsigned off = (unsigned)(rp + ((Z0 + j3 - zlo) * ylen + (Y0 + j2 - ylo)) * lx + ox);
-      const bool ysh = i2 == j2 && i2 != 1, zsh = i3 == j3 && i3 != 1;
-      const bool yzf = (!ysh || (i2 == 0 ? fly : fhy)) && (!zsh || (i3 == 0 ? flz : fhz));
-      unsigned firstm = 0;
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        bool f = yzf;
-        if (k == 0 && xs_lo) f = f && flx;
-        if (k == n - 1 && xs_hi) f = f && fhx;
-        if (ga_first_touch && f) firstm |= 1u << k;
-      }
-      g_off[r] = off;
-      g_meta[r] = (unsigned)n | (unsigned)ox << 3 | (unsigned)fixed << 6 | (unsigned)go << 7 | firstm << 8;
-      // read-backs: later touches of entries of non-Dirichlet rows (a run
-      // has at most 3 columns in rounds r < 6, 5 after)
-#pragma unroll
-      for (int k = 0; k < 5; ++k)
-        old[r][k] = (k < (r < 6 ? 3 : 5) && go && k < n && !fixed && !((firstm >> k) & 1)) ? ga_jac[off + k] : 0.0;
     }
-    }
-
-
+    if (JAC && own && ga_jac) {
+      double* S = s_fs + wv * kSCol;
+      double a[3][3];  // a[i][j]
 #pragma unroll
-      for (int r = 0; r < 9; ++r) {
-        const int m = r / 3, pp = l + 32 * (r % 3);
-        const bool task = act && pp < 81;
-        const int i1 = h ? m : 2 - m;
-        const int j2 = pp % 3, j3 = (pp / 3) % 3, i2 = (pp / 9) % 3, i3 = pp / 27;
-        double acc[3] = {0.0, 0.0, 0.0};
-        if (task) {
-          const int o = (3 * i2 + j2) * 9 + 3 * i3 + j3;
+      for (int i = 0; i < 3; ++i)
 #pragma unroll
-          for (int q1 = 0; q1 < 3; ++q1) {
-            const double* s2 = &s_a[h][q1 * 243];
-            const double di = Dq(i1, q1), bi = Bq(i1, q1);
-            const double v = di * s2[o];
-            const double wv = fma(bi, s2[162 + o], di * s2[81 + o]);
+        for (int j = 0; j < 3; ++j) a[i][j] = 0.0;
 #pragma unroll
-            for (int j1 = 0; j1 < 3; ++j1) acc[j1] = fma(kT.D[j1][q1], v, fma(kT.B[j1][q1], wv, acc[j1]));
-          }
-        }
-        // the column A shares with B on their common plane (m == 0) comes
-        // from the other half; so does the previous step's carry (m == 2),
-        // which half 1 then replaces with its own rows
-        double fromB0 = 0.0, cin[3] = {0.0, 0.0, 0.0};
-        if (m == 0) fromB0 = __shfl_xor(acc[0], 32, 64);
-        if (m == 2) {
+      for (int q = 0; q < 3; ++q) {
+        const double s3 = iJx2 * S[(3 * q) * kSRow + canon], s1 = S[(3 * q + 1) * kSRow + canon],
+                     s0 = S[(3 * q + 2) * kSRow + canon];
 #pragma unroll
-          for (int k = 0; k < 3; ++k) {
-            cin[k] = __shfl_xor(carry_j[r - 6][k], 32, 64);
-            carry_j[r - 6][k] = (h == 1 && task) ? acc[k] : carry_j[r - 6][k];
-          }
-        }
-        const unsigned off = g_off[r], meta = g_meta[r];
-        if (!((meta >> 7) & 1)) continue;
-        const int n = meta & 7, ox = (meta >> 3) & 7;
-        const bool fixed = (meta >> 6) & 1;
-        const unsigned firstm = meta >> 8;
-        // the run's values
-        double val[5] = {acc[0], acc[1], acc[2], 0.0, 0.0};
-        if (m == 0) {
-          if (h == 0) {
-            if (hasB) val[2] = acc[2] + fromB0;
-          } else {
-            val[0] = acc[1], val[1] = acc[2];
-          }
-        } else if (m == 2 && h == 0 && !first_step) {
-          val[0] = cin[0], val[1] = cin[1], val[2] = cin[2] + acc[0], val[3] = acc[1], val[4] = acc[2];
-        }
-        const int X = 2 * ex + i1;
-        const int lox = (X & 1) ? X - 1 : (X - 2 < 0 ? 0 : X - 2);
-        if (__any(fixed)) {
+        for (int i = 0; i < 3; ++i) {
+          const double v = kT.D[i][q] * s3, w = fma(kT.B[i][q], s0, kT.D[i][q] * s1);
 #pragma unroll
-          for (int k = 0; k < (r < 6 ? 3 : 5); ++k) {
-            const bool first = (firstm >> k) & 1;
-            if (k >= n || (fixed && !first)) continue;
-            // strong Dirichlet row: e_d, written by its first toucher
-            const double v = fixed ? ((i2 == j2 && i3 == j3 && lox + ox + k == X) ? 1.0 : 0.0)
-                                   : (first ? val[k] : old[r][k] + val[k]);
-            ga_jac[off + k] = v;
-          }
-        } else {
-          // no strong-Dirichlet row in the round (the common case): a first
-          // touch read nothing (old = +0) and val is never -0 (sums started
-          // from +0), so old + val is val exactly
-#pragma unroll
-          for (int k = 0; k < (r < 6 ? 3 : 5); ++k)
-            if (k < n) ga_jac[off + k] = old[r][k] + val[k];
+          for (int j = 0; j < 3; ++j) a[i][j] = fma(kT.D[j][q], v, fma(kT.B[j][q], w, a[i][j]));
         }
       }
+      if (emit) {
+        // rows on the box's x planes have three columns per run
+        const bool full = e > 0;
+        bool fx0 = false, fx1 = false, fx2 = false;
+        if (pair) {
+          fx0 = ga_fixed[prow + 2 * e] != 0;
+          fx1 = ga_fixed[prow + 2 * e + 1] != 0;
+          if (last) fx2 = ga_fixed[prow + 2 * e + 2] != 0;
+        }
+        const double one = dnode && !add ? 1.0 : 0.0;
+        wave_lds_sync();  // S is read by every lane: the entries take its place
+        if (full) {
+          if (pair) {
+            double r0[5] = {carry[0], carry[1], carry[2] + a[0][0], a[0][1], a[0][2]};
+            double r1[3] = {a[1][0], a[1][1], a[1][2]};
+            if (__any(fx0 || fx1)) {
+#pragma unroll
+              for (int k = 0; k < 5; ++k) r0[k] = fx0 ? (k == 2 ? one : 0.0) : r0[k];
+#pragma unroll
+              for (int k = 0; k < 3; ++k) r1[k] = fx1 ? (k == 1 ? one : 0.0) : r1[k];
+            }
+            double* o = S + 8 * plb + 5 * pt;
+#pragma unroll
+            for (int k = 0; k < 5; ++k) o[k] = r0[k];
+            double* p = S + 8 * plb + 5 * pnr + 3 * pt;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) p[k] = r1[k];
+          }
+          wave_lds_sync();
+          const int total = 8 * lb_4;
+          double v[8];
+#pragma unroll
+          for (int s = 0; s < 8; ++s) v[s] = S[lane + 64 * s];
+          if (add) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+              if (lane + 64 * s < total) v[s] += ga_jac[goff[s] + (unsigned)e * ginc[s]];
+          }
+#pragma unroll
+          for (int s = 0; s < 8; ++s)
+            if (lane + 64 * s < total) ga_jac[goff[s] + (unsigned)e * ginc[s]] = v[s];
+        } else {
+          if (pair) {
+            double* o = S + 6 * plb + 3 * pt;
+            o[0] = fx0 ? one : a[0][0];
+            o[1] = fx0 ? 0.0 : a[0][1];
+            o[2] = fx0 ? 0.0 : a[0][2];
+            double* p = S + 6 * plb + 3 * pnr + 3 * pt;
+            p[0] = fx1 ? 0.0 : a[1][0];
+            p[1] = fx1 ? one : a[1][1];
+            p[2] = fx1 ? 0.0 : a[1][2];
+          }
+          wave_lds_sync();
+          for (int idx = lane; idx < 6 * lb_4; idx += 64) {
+            const int j = (idx >= 6 * lb_1) + (idx >= 6 * lb_2) + (idx >= 6 * lb_3);
+            const int lb = j == 0 ? 0 : j == 1 ? lb_1 : j == 2 ? lb_2 : lb_3;
+            double* g = ga_jac + ((j == 0 ? line0 : j == 1 ? line1 : j == 2 ? line2 : line3) + (unsigned)(idx - 6 * lb));
+            *g = add ? *g + S[idx] : S[idx];
+          }
+        }
+        if (last) {
+          // the row plane 2 n0
+          wave_lds_sync();
+          if (pair) {
+            double* o = S + 3 * lane;
+            o[0] = fx2 ? 0.0 : a[2][0];
+            o[1] = fx2 ? 0.0 : a[2][1];
+            o[2] = fx2 ? one : a[2][2];
+          }
+          wave_lds_sync();
+          for (int idx = lane; idx < 3 * lb_4; idx += 64) {
+            const int j = (idx >= 3 * lb_1) + (idx >= 3 * lb_2) + (idx >= 3 * lb_3);
+            const int lb = j == 0 ? 0 : j == 1 ? lb_1 : j == 2 ? lb_2 : lb_3;
+            const int nr = j == 0 ? nr0 : j == 1 ? nr1 : j == 2 ? nr2 : nr3;
+            double* g = ga_jac + ((j == 0 ? line0 : j == 1 ? line1 : j == 2 ? line2 : line3) +
+                                  (unsigned)nr * (unsigned)(8 * n0 - 2) + (unsigned)(idx - 3 * lb));
+            *g = add ? *g + S[idx] : S[idx];
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 3; ++k) carry[k] = a[2][k];
+    }
+    lds_sync();  // F, S and the planes change hands
   }
 }
 
@@ -660,29 +660,47 @@ bool q2box_applicable(const Ctx& c) {
          c.desc.physics == MHX_PHYS_THERMAL && !c.xh.active;
 }
 
+// Elements per x-segment.  A workgroup repeats the layer before its segment
+// and fills its pipeline (about two layers), and the device runs `slots`
+// workgroups at a time: the fewest layers in sequence win.  96^3, us by
+// segment: 8 1,953, 12 1,924, 16 1,865, 24 1,877, 48 1,896, 96 2,014; 16^3: 2
+// 26.4, 4 31.2, 8 38.9, 16 64.4.
+static int q2_auto_segment(const Ctx& c, int slots) {
+  const int n0 = c.mesh.nel[0];
+  const long nyz = (long)((c.mesh.nel[1] + 2) / 2) * ((c.mesh.nel[2] + 2) / 2);
+  int best = 2;
+  double best_cost = 1e300;
+  for (int L : {2, 4, 6, 8, 12, 16, 24, 32, 48}) {
+    const long wgs = ((n0 + L - 1) / L) * nyz;
+    const double cost = (double)((wgs + slots - 1) / slots) * (std::min(L, n0) + 2);
+    if (cost < best_cost) best = L, best_cost = cost;
+    if (L >= n0) break;
+  }
+  return best;
+}
+
+int q2box_segment(const Ctx& c, bool jac) {
+  // workgroups resident per CU: three (LDS) for the Jacobian, two with sine
+  // modes (registers), four for the residual
+  return c.q2_segment ? c.q2_segment : q2_auto_segment(c, 256 * (jac ? (c.desc.n_modes > 0 ? 2 : 3) : 4));
+}
+
 void launch_q2box(Ctx& c, AsmArgs& a, bool jac) {
-  const int L = c.q2_segment;
+  const int L = q2box_segment(c, jac);
   a.gpb = L;
   a.nseg = (c.mesh.nel[0] + L - 1) / L;
-  for (int col = 0; col < 8; ++col) {
-    a.color = col;
-    const int cxb = col & 1, cyb = (col >> 1) & 1, czb = (col >> 2) & 1;
-    a.cn[0] = (a.nseg - cxb + 1) / 2;
-    a.cn[1] = (c.mesh.nel[1] - cyb + 1) / 2;
-    a.cn[2] = (c.mesh.nel[2] - czb + 1) / 2;
-    const long blocks = (long)a.cn[0] * a.cn[1] * a.cn[2];
-    if (blocks == 0) continue;
-    ScopedPhase ph(c.prof, jac ? "k_q2box<jacres>" : "k_q2box<res>", c.stream);
-    const dim3 grid((unsigned)blocks), block(64);
-    if (a.coef.n_modes > 0) {
-      if (jac) hipLaunchKernelGGL((k_q2box<true, true>), grid, block, 0, c.stream, a);
-      else hipLaunchKernelGGL((k_q2box<false, true>), grid, block, 0, c.stream, a);
-    } else {
-      if (jac) hipLaunchKernelGGL((k_q2box<true, false>), grid, block, 0, c.stream, a);
-      else hipLaunchKernelGGL((k_q2box<false, false>), grid, block, 0, c.stream, a);
-    }
-    MHX_HIP(hipGetLastError());
+  a.cn[1] = (c.mesh.nel[1] + 2) / 2;
+  a.cn[2] = (c.mesh.nel[2] + 2) / 2;
+  ScopedPhase ph(c.prof, jac ? "k_q2box<jacres>" : "k_q2box<res>", c.stream);
+  const dim3 grid((unsigned)(a.nseg * a.cn[1] * a.cn[2])), block(256);
+  if (a.coef.n_modes > 0) {
+    if (jac) hipLaunchKernelGGL((k_q2box<true, true>), grid, block, 0, c.stream, a);
+    else hipLaunchKernelGGL((k_q2box<false, true>), grid, block, 0, c.stream, a);
+  } else {
+    if (jac) hipLaunchKernelGGL((k_q2box<true, false>), grid, block, 0, c.stream, a);
+    else hipLaunchKernelGGL((k_q2box<false, false>), grid, block, 0, c.stream, a);
   }
+  MHX_HIP(hipGetLastError());
 }
 
 }  // namespace mhx

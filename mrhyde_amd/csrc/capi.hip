@@ -1044,7 +1044,7 @@ int mhx_get_option(const mhx_ctx* ctx, const char* name, int64_t* value) {
   if (!ctx || !name || !value) return MHX_ERR_ARG;
   const std::string k(name);
   if (k == "assembly.segment") {
-    *value = ctx->q2_segment;
+    *value = q2box_segment(*ctx, true);
     return MHX_OK;
   }
   if (k == "assembly.colouring") {

@@ -235,7 +235,7 @@ struct Ctx {
   int nfield = 1;  // unknowns per node (consecutive DOFs): block size of block Jacobi
   int scatter_mode = kElementColouring;
   bool box_mesh = false;  // every element an axis-aligned box (structured box, no node perturbation)
-  int q2_segment = 12;    // pencil streaming: elements per x-segment (even)
+  int q2_segment = 0;     // pencil streaming: elements per x-segment (even; 0: chosen per launch)
   std::shared_ptr<Amg> amg;  // built by a solve with the AMG preconditioner, kept for reuse of its buffers
   // time-integration state (mhx_set_time_state); bdf_order 0 = steady
   int bdf_order = 0;
@@ -257,9 +257,10 @@ void lagrange_equispaced(int p, double xi, double* L, double* dL);
 
 // assembly (assemble.hip)
 bool thermal_supported(int dim, int p, int nq1);
-// Q2 hexahedra on box meshes: pencil-streamed pair-factorised assembly (assemble_q2box.hip)
+// Q2 hexahedra on box meshes: row-owned pair-factorised assembly (assemble_q2box.hip)
 bool q2box_applicable(const Ctx& c);
 void launch_q2box(Ctx& c, AsmArgs& a, bool jac);
+int q2box_segment(const Ctx& c, bool jac);  // elements per x-segment of a launch
 // thermal assembly with compiled coefficient functions, element colouring
 // (assemble_expr.hip)
 void launch_thermal_expr(Ctx& c, AsmArgs& a, bool jac);

@@ -274,7 +274,7 @@ int  mhx_linear_solve(mhx_ctx* ctx, const double* jac_vals, const double* r, dou
  * MHX_PREC_JACOBI (FP64), so x, the iteration count and rel_res are the
  * same bits; the Krylov vectors, the Jacobi scaling and the reduction
  * partials live in one file-scope device array per GPU of
- * 5 * MHX_NOALLOC_MAX_DOF + 1280 doubles (40 MiB, held by every GPU the
+ * 5 * MHX_NOALLOC_MAX_DOF + 3328 doubles (40 MiB, held by every GPU the
  * library runs on until the process ends) instead of context buffers.
  * It calls no hipMalloc/hipFree and records no phase timers.
  *   - n_dof <= MHX_NOALLOC_MAX_DOF, else MHX_ERR_ARG;

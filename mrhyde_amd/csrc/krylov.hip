@@ -475,62 +475,204 @@ static void op_apply(Ctx& c, const T* A, const Prec<T>& P, const T* v, T* w, T* 
 }
 
 // ---- CG (Jacobi PCG as SolverManager::PCG) -----------------------------------
-// z = minv .* r (minv == nullptr: z = r) fused with rho = r.z
+// An iteration is two steps that depend on each other: p, q = A p and p.q, then
+// x, r, z = D^-1 r, ||r||^2 and r.z.  Small systems run it in two launches
+// (k_cg_dir, k_cg_update): each block adds up the partial sums of the launch
+// before by itself, so no launch is spent on a final reduction, and k_cg_dir
+// forms p at the gathered columns (z + beta p_old, both in cache) into the other
+// of two p vectors.  With a launch per step of the recurrence and per reduction
+// (nine) an iteration of the 64^2 Q1 problem took 25-29 us, nearly all latency;
+// now 13 us (a whole Newton solve of it 11.2 -> 5.3 ms).
+// Larger systems keep the product apart, with the final reductions still folded
+// into their readers (four launches).
+// The CG scalars stay on the device: rho (two slots, alternating by
+// iteration) and ||r||^2 per iteration in a window that the host reads once per
+// window (one synchronisation every W iterations).  An exhausted direction (p.q
+// == 0 or rho_old == 0) turns the update into a no-op, so iterations run past
+// convergence inside a window leave x and r unchanged.
+constexpr int kCgRho = 0, kCgHist = 4;
+constexpr int kCgParts = 3;  // partial sums: r.z, ||r||^2, p.q
+
+// sum of nb partials in every thread of the block, in a fixed order
+__device__ __forceinline__ double block_total(const double* __restrict__ part, int nb) {
+  __shared__ double sh[4];
+  double v = 0.0;
+  for (int i = threadIdx.x; i < nb; i += 256) v += part[i];
+  v = wave_sum(v);
+  __syncthreads();  // sh may be read from an earlier call
+  if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = v;
+  __syncthreads();
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+// block sum of v, valid in thread 0
+__device__ __forceinline__ double block_sum0(double v) {
+  __shared__ double sh[4];
+  const double s = wave_sum(v);
+  __syncthreads();
+  if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = s;
+  __syncthreads();
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+// rho of the iteration from the partials of r.z and beta = rho / rho_old; block
+// 0 stores rho
+__device__ __forceinline__ double cg_beta(double* __restrict__ cgs, int cur, const double* __restrict__ rz, int nb) {
+  const double ro = cgs[kCgRho + (cur ^ 1)];
+  const double rn = block_total(rz, nb);
+  if (blockIdx.x == 0 && threadIdx.x == 0) cgs[kCgRho + cur] = rn;
+  return ro != 0.0 ? rn / ro : 0.0;
+}
+// the launch's last block, in both forms of the direction step: ||r||^2 of the
+// iteration before into the window (beside the other blocks' work)
+__device__ __forceinline__ bool cg_hist_block(const double* __restrict__ rr, int nb, double* __restrict__ hist) {
+  if (blockIdx.x != gridDim.x - 1) return false;
+  if (hist) {
+    const double h = block_total(rr, nb);
+    if (threadIdx.x == 0) *hist = h;
+  }
+  return true;
+}
+
+// z = minv .* r (minv == nullptr: z = r, not stored) and partial r.z
 template <class T>
 __global__ __launch_bounds__(256) void k_prec_dot(long n, const T* __restrict__ minv, const T* __restrict__ r,
                                                   T* __restrict__ z, double* __restrict__ part) {
   double v = 0.0;
   for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    const T zi = minv ? minv[i] * r[i] : r[i];
-    z[i] = zi;
-    v = fma((double)r[i], (double)zi, v);
+    const T ri = r[i], zi = minv ? minv[i] * ri : ri;
+    if (minv) z[i] = zi;
+    v = fma((double)ri, (double)zi, v);
   }
   block_store1(v, part);
 }
-// The CG scalars stay on the device: rho (two slots, alternating by
-// iteration), p.q, and ||r||^2 per iteration in a window that the host reads
-// once per window (one synchronisation every W iterations instead of three
-// per iteration).  An exhausted direction (p.q == 0 or rho_old == 0) turns
-// the update into a no-op, so iterations run past convergence inside a
-// window leave x and r unchanged.
-constexpr int kCgRho = 0, kCgPq = 2, kCgHist = 4;
-
-// p = z + beta p, beta = rho_new / rho_old ; first iteration p = z (p may
-// hold uninitialised bits, and 0 * NaN would not clear them)
-template <class T>
-__global__ void k_xpby(long n, const T* __restrict__ z, const double* __restrict__ cgs, int cur, int first,
-                       T* __restrict__ p) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double rn = cgs[kCgRho + cur], ro = cgs[kCgRho + (cur ^ 1)];
-  const double beta = ro != 0.0 ? rn / ro : 0.0;
-  p[i] = first ? z[i] : (T)fma(beta, (double)p[i], (double)z[i]);
+// p = z + beta p_old, q = A p, partial p.q.  First iteration: p = z (p_old may
+// hold uninitialised bits, and 0 * NaN would not clear them).
+template <int LANES, bool LAT, class T>
+__global__ __launch_bounds__(256) void k_cg_dir(BoxMesh m, long n, const int32_t* __restrict__ rp,
+                                                const int32_t* __restrict__ colidx, const T* __restrict__ A,
+                                                const T* __restrict__ z, const T* __restrict__ po,
+                                                T* __restrict__ p, T* __restrict__ q, double* __restrict__ cgs,
+                                                int cur, int first, const double* __restrict__ rz,
+                                                const double* __restrict__ rr, int nb, double* __restrict__ hist,
+                                                double* __restrict__ pq) {
+  if (cg_hist_block(rr, nb, hist)) return;
+  const long row = ((long)blockIdx.x * blockDim.x + threadIdx.x) / LANES;
+  const int l = threadIdx.x % LANES;
+  const bool act = row < n;
+  // the row's first entries and what they gather go out ahead of the
+  // reduction that beta waits for
+  constexpr int U = 4;
+  int b = 0, e = 0;
+  std::conditional_t<LAT, LatCols, CsrCols> ci;
+  T av[U], zv[U], pv[U], z0 = 0, p0 = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) av[u] = zv[u] = pv[u] = 0;
+  if (act) {
+    b = rp[row], e = rp[row + 1];
+    if constexpr (LAT) ci = LatCols{lat_row(m, row), b};
+    else ci = CsrCols{colidx};
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = b + l + u * LANES;
+      if (k < e) {
+        const int j = ci(k);
+        av[u] = A[k];
+        zv[u] = z[j];
+        if (!first) pv[u] = po[j];
+      }
+    }
+    if (l == 0) {
+      z0 = z[row];
+      if (!first) p0 = po[row];
+    }
+  }
+  const double beta = cg_beta(cgs, cur, rz, nb);
+  auto dir = [&](T zi, T pi) { return first ? zi : (T)fma(beta, (double)pi, (double)zi); };
+  T acc = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) acc += av[u] * dir(zv[u], pv[u]);
+  for (int k = b + l + U * LANES; k < e; k += LANES) {
+    const int j = ci(k);
+    acc += A[k] * dir(z[j], first ? (T)0 : po[j]);
+  }
+#pragma unroll
+  for (int off = LANES / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, LANES);
+  double v = 0.0;
+  if (act && l == 0) {
+    const T pi = dir(z0, p0);
+    p[row] = pi;
+    q[row] = acc;
+    v = (double)pi * (double)acc;
+  }
+  block_store1(v, pq);
 }
-// x += alpha p ; r -= alpha q ; partial ||r||^2 ; alpha = rho / p.q
+// p = z + beta p in place (the product follows in a launch of its own)
+template <class T>
+__global__ __launch_bounds__(256) void k_xpby(long n, const T* __restrict__ z, double* __restrict__ cgs, int cur,
+                                              int first, const double* __restrict__ rz,
+                                              const double* __restrict__ rr, int nb, double* __restrict__ hist,
+                                              T* __restrict__ p) {
+  if (cg_hist_block(rr, nb, hist)) return;
+  const double beta = cg_beta(cgs, cur, rz, nb);
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)(gridDim.x - 1) * 256)
+    p[i] = first ? z[i] : (T)fma(beta, (double)p[i], (double)z[i]);
+}
+// alpha = rho / p.q; x += alpha p; r -= alpha q; partial ||r||^2 and, where z
+// is the diagonal scaling (minv) or r itself, z and partial r.z (rz)
 template <class T>
 __global__ __launch_bounds__(256) void k_cg_update(long n, const double* __restrict__ cgs, int cur,
-                                                   const T* __restrict__ p, const T* __restrict__ q,
-                                                   T* __restrict__ x, T* __restrict__ r, double* __restrict__ part) {
-  const double pq = cgs[kCgPq];
-  const double al = pq != 0.0 ? cgs[kCgRho + cur] / pq : 0.0;
+                                                   const double* __restrict__ pq, int nbq, const T* __restrict__ p,
+                                                   const T* __restrict__ q, T* __restrict__ x, T* __restrict__ r,
+                                                   const T* __restrict__ minv, T* __restrict__ z,
+                                                   double* __restrict__ rr, double* __restrict__ rz) {
+  // the thread's first row is loaded ahead of the reduction that alpha waits for
+  const long step = (long)gridDim.x * 256;
+  long i = (long)blockIdx.x * 256 + threadIdx.x;
+  T xi = 0, pi = 0, qi = 0, ri = 0, mi = 0;
+  auto fetch = [&]() {
+    if (i < n) {
+      xi = x[i], pi = p[i], qi = q[i], ri = r[i];
+      if (rz && minv) mi = minv[i];
+    }
+  };
+  fetch();
+  const double t = block_total(pq, nbq);
+  const double al = t != 0.0 ? cgs[kCgRho + cur] / t : 0.0;
   const T a = (T)al;
-  double v = 0.0;
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    x[i] = fma(a, p[i], x[i]);
-    const T ri = fma(-a, q[i], r[i]);
-    r[i] = ri;
-    v = fma((double)ri, (double)ri, v);
+  double v = 0.0, w = 0.0;
+  while (i < n) {
+    x[i] = fma(a, pi, xi);
+    const T rn = fma(-a, qi, ri);
+    r[i] = rn;
+    v = fma((double)rn, (double)rn, v);
+    if (rz) {
+      const T zi = minv ? mi * rn : rn;
+      if (minv) z[i] = zi;
+      w = fma((double)rn, (double)zi, w);
+    }
+    i += step;
+    fetch();
   }
-  block_store1(v, part);
+  const double sv = block_sum0(v);
+  if (threadIdx.x == 0) rr[blockIdx.x] = sv;
+  if (rz) {
+    const double sw = block_sum0(w);
+    if (threadIdx.x == 0) rz[blockIdx.x] = sw;
+  }
 }
 
-// Device storage of one CG solve: the four Krylov vectors, the reduction
+// Device storage of one CG solve: the Krylov vectors (two directions for the
+// small systems' two-launch iteration), kCgParts x kRedBlocks reduction
 // partials, the CG scalars and one reduction slot.
 template <class T>
 struct CgBufs {
-  T *r, *z, *p, *q;
+  T *r, *z, *p, *p2, *q;
   double *part, *cgs, *slot;
 };
+
+// The two-launch iteration gathers two vectors per entry instead of one and
+// needs a partial sum per block of rows: it is taken while the product's blocks
+// fit the partials (n up to 65,536 at four lanes a row).
+static bool cg_two_launch(const Ctx& c, long n) { return n * c.spmv_lanes <= 256L * kRedBlocks; }
 
 template <class T>
 static int cg_run(Ctx& c, const T* A, const Prec<T>& P, const T* b, T* x, double tol, int maxit, double* relres,
@@ -539,6 +681,7 @@ static int cg_run(Ctx& c, const T* A, const Prec<T>& P, const T* b, T* x, double
   constexpr int kMaxW = 16;
   const int W = n < 2000000 ? kMaxW : 4;  // iterations per host check
   double* cgs = v.cgs;
+  double *rz = v.part, *rr = v.part + kRedBlocks, *pq = v.part + 2 * kRedBlocks;
   const int nb = red_blocks(n);
   auto nrm = [&](const T* a) { return std::sqrt(reduce_to<T>(c, n, a, a, 0, v.part, v.slot)); };
   const double bn = nrm(b);
@@ -551,30 +694,62 @@ static int cg_run(Ctx& c, const T* A, const Prec<T>& P, const T* b, T* x, double
   hipLaunchKernelGGL(k_resid<T>, grid1(n), dim3(256), 0, c.stream, n, b, v.q, v.r);
   double rn = nrm(v.r);
   if (!std::isfinite(rn)) throw Error{MHX_ERR_NONFINITE, "CG: non-finite residual"};
+  // z is stored by a preconditioner; without one it is r
+  const bool cycle = P.kind == MHX_PREC_BLOCK_JACOBI || P.kind == MHX_PREC_AMG;
+  const T* minv = P.kind == MHX_PREC_JACOBI ? P.d : nullptr;
+  const T* z = cycle || minv ? v.z : v.r;
+  const bool two = cg_two_launch(c, n);
+  const int nbq = two ? (int)((n * c.spmv_lanes + 255) / 256) : nb;
+  T *pc = v.p, *po = two ? v.p2 : v.p;
+  auto direction = [&](int cur, int first, double* hist) {
+    if (!two) {
+      hipLaunchKernelGGL(k_xpby<T>, dim3(nb + 1), dim3(256), 0, c.stream, n, z, cgs, cur, first, rz, rr, nb, hist, pc);
+      spmv_t<T, T>(c, A, nullptr, pc, v.q);
+      hipLaunchKernelGGL(k_dot<T>, dim3(nb), dim3(256), 0, c.stream, n, pc, v.q, pq, 0);
+      return;
+    }
+    auto go = [&](auto LN, auto LT) {
+      hipLaunchKernelGGL((k_cg_dir<decltype(LN)::value, decltype(LT)::value, T>), dim3(nbq + 1), dim3(256), 0, c.stream,
+                         c.mesh, n, c.rowptr.p, c.colidx.p, A, z, po, pc, v.q, cgs, cur, first, rz, rr, nb, hist, pq);
+    };
+    auto lanes = [&](auto LT) {
+      switch (c.spmv_lanes) {
+        case 4: go(std::integral_constant<int, 4>{}, LT); break;
+        case 8: go(std::integral_constant<int, 8>{}, LT); break;
+        case 16: go(std::integral_constant<int, 16>{}, LT); break;
+        case 32: go(std::integral_constant<int, 32>{}, LT); break;
+        default: go(std::integral_constant<int, 64>{}, LT); break;
+      }
+    };
+    if (c.lattice_cols) lanes(std::true_type{});
+    else lanes(std::false_type{});
+  };
+  // z and r.z of the first direction (later ones come with the update)
+  auto precondition = [&]() {
+    if (cycle) {
+      prec_apply<T>(c, P, v.r, v.z);
+      hipLaunchKernelGGL(k_dot<T>, dim3(nb), dim3(256), 0, c.stream, n, v.r, v.z, rz, 0);
+    } else {
+      hipLaunchKernelGGL(k_prec_dot<T>, dim3(nb), dim3(256), 0, c.stream, n, minv, v.r, v.z, rz);
+    }
+  };
   int it = 0;
   double hist[kMaxW];
   Profiler off;
+  if (!cycle) precondition();
   while (it < maxit && rn / bn > tol) {
     const int w = std::min(W, maxit - it);
     {
       ScopedPhase ph(timers ? c.prof : off, "Krylov::cg_window", c.stream);
       for (int k = 0; k < w; ++k) {
         const int cur = (it + k) & 1;
-        if (P.kind == MHX_PREC_BLOCK_JACOBI || P.kind == MHX_PREC_AMG) {
-          prec_apply<T>(c, P, v.r, v.z);
-          hipLaunchKernelGGL(k_dot<T>, dim3(nb), dim3(256), 0, c.stream, n, v.r, v.z, v.part, 0);
-        } else {
-          hipLaunchKernelGGL(k_prec_dot<T>, dim3(nb), dim3(256), 0, c.stream, n,
-                             P.kind == MHX_PREC_JACOBI ? P.d : (const T*)nullptr, v.r, v.z, v.part);
-        }
-        hipLaunchKernelGGL(k_final, dim3(1), dim3(256), 0, c.stream, v.part, nb, 0, cgs + kCgRho + cur, nullptr);
-        hipLaunchKernelGGL(k_xpby<T>, grid1(n), dim3(256), 0, c.stream, n, v.z, cgs, cur, it + k == 0 ? 1 : 0, v.p);
-        spmv_t<T, T>(c, A, nullptr, v.p, v.q);
-        hipLaunchKernelGGL(k_dot<T>, dim3(nb), dim3(256), 0, c.stream, n, v.p, v.q, v.part, 0);
-        hipLaunchKernelGGL(k_final, dim3(1), dim3(256), 0, c.stream, v.part, nb, 0, cgs + kCgPq, nullptr);
-        hipLaunchKernelGGL(k_cg_update<T>, dim3(nb), dim3(256), 0, c.stream, n, cgs, cur, v.p, v.q, x, v.r, v.part);
-        hipLaunchKernelGGL(k_final, dim3(1), dim3(256), 0, c.stream, v.part, nb, 0, cgs + kCgHist + k, nullptr);
+        if (cycle) precondition();
+        direction(cur, it + k == 0 ? 1 : 0, k > 0 ? cgs + kCgHist + k - 1 : nullptr);
+        hipLaunchKernelGGL(k_cg_update<T>, dim3(nb), dim3(256), 0, c.stream, n, cgs, cur, pq, nbq, pc, v.q, x, v.r,
+                           minv, v.z, rr, cycle ? (double*)nullptr : rz);
+        std::swap(pc, po);
       }
+      hipLaunchKernelGGL(k_final, dim3(1), dim3(256), 0, c.stream, rr, nb, 0, cgs + kCgHist + w - 1, nullptr);
       MHX_HIP(hipGetLastError());
       MHX_HIP(hipMemcpyAsync(hist, cgs + kCgHist, w * sizeof(double), hipMemcpyDeviceToHost, c.stream));
       MHX_HIP(hipStreamSynchronize(c.stream));
@@ -598,9 +773,10 @@ static int cg_core(Ctx& c, const T* A, const Prec<T>& P, const T* b, T* x, doubl
   const long n = c.mesh.ndof;
   KrylovVecs<T>& v = vecs<T>(c);
   v.r.alloc(n); v.z.alloc(n); v.p.alloc(n); v.q.alloc(n);
-  ensure_red(c, 1);
+  if (cg_two_launch(c, n)) v.tmp.alloc(n);
+  ensure_red(c, kCgParts);
   if (c.kw.cgs.n < (size_t)(kCgHist + 16)) c.kw.cgs.alloc(kCgHist + 16);
-  const CgBufs<T> bufs{v.r.p, v.z.p, v.p.p, v.q.p, c.kw.part.p, c.kw.cgs.p, c.kw.scal.p + kScalN};
+  const CgBufs<T> bufs{v.r.p, v.z.p, v.p.p, v.tmp.p, v.q.p, c.kw.part.p, c.kw.cgs.p, c.kw.scal.p + kScalN};
   return cg_run<T>(c, A, P, b, x, tol, maxit, relres, bufs, true);
 }
 
@@ -962,7 +1138,7 @@ static int mixed_solve(Ctx& c, const double* A, const double* b, double* x, cons
 // krylov_solve_noalloc.  Its host-side name is only a symbol: the device
 // address is taken once per device with hipGetSymbolAddress and used
 // everywhere the host hands the memory to a kernel.
-constexpr long kNoAllocTail = kRedBlocks + 256;  // partials, CG scalars, one slot
+constexpr long kNoAllocTail = kCgParts * kRedBlocks + 256;  // partials, CG scalars, one slot
 constexpr long kNoAllocDoubles = 5L * MHX_NOALLOC_MAX_DOF + kNoAllocTail;
 static __device__ __align__(256) double scratch[kNoAllocDoubles];
 
@@ -999,8 +1175,10 @@ int krylov_solve_noalloc(Ctx& c, const double* A, const double* b, double* x, co
               "allocation-free solve: no preconditioner or point Jacobi in FP64 only");
   double* s = scratch_ptr();
   const long N = MHX_NOALLOC_MAX_DOF;
-  CgBufs<double> v{s, s + N, s + 2 * N, s + 3 * N, s + 5 * N, s + 5 * N + kRedBlocks,
-                   s + 5 * N + kRedBlocks + 128};
+  // (the second direction vector of small systems: the free half of p's array)
+  double* tail = s + 5 * N + kCgParts * kRedBlocks;
+  CgBufs<double> v{s, s + N, s + 2 * N, s + 2 * N + N / 2, s + 3 * N, s + 5 * N, tail, tail + 128};
+  MHX_REQUIRE(!cg_two_launch(c, n) || n <= N / 2, MHX_ERR_STATE, "allocation-free solve: no room for the second direction");
   double* minv = s + 4 * N;
   // the array keeps the last call's contents: the CG scalars start cleared
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, c.stream, 256L, 0.0, v.cgs);

@@ -291,7 +291,8 @@ constexpr int kApLanes = 8;
 // P = (I - omega D^-1 A) T.  The row's box of at most 2x2x2 aggregates x nf
 // fields collects sum_j A_ij ns_j; T's normalisation (1 / nrm per aggregate
 // and field) is applied to the sums.  (One thread per row walked its CRS row
-// alone, every lane in lines of its own: 655 us at 48^3 Q2, now 150.)
+// alone, every lane in lines of its own: mean over the levels of 48^3 Q2 655
+// us, now 271.)
 __global__ __launch_bounds__(kAmgBlk) void k_amg_P(Geo G, LevelBox B, long n, const int32_t* __restrict__ rp,
                                                    const double* __restrict__ A, const double* __restrict__ dinv,
                                                    const double* __restrict__ ns, const double* __restrict__ nrm,
@@ -381,7 +382,8 @@ __global__ __launch_bounds__(kAmgBlk) void k_amg_R(Geo G, const int32_t* __restr
 // AP(i, (J, g)) in a dense 3x3x3 aggregate box per (fine row i, coarse field
 // g), a group of kApLanes lanes each (see k_amg_P).  A column's first aggregate
 // is the row's first or the next one per axis.  (With two index divisions and
-// seven table loads per entry: 1,010 us at 48^3 Q2, now 420.)
+// seven table loads per entry: mean over the levels of 48^3 Q2 1,010 us, now
+// 455.)
 __global__ __launch_bounds__(kAmgBlk) void k_amg_AP(Geo G, LevelBox B, long n, const int32_t* __restrict__ rp,
                                                     const double* __restrict__ A, const int32_t* __restrict__ prp,
                                                     const double* __restrict__ P, double* __restrict__ AP) {
@@ -449,8 +451,8 @@ __global__ __launch_bounds__(kAmgBlk) void k_amg_AP(Geo G, LevelBox B, long n, c
 // boxes (one contiguous read per box, four R entries in flight), and add into
 // the group's own copy of the coarse row in LDS; the copies are summed in
 // group order.  (One thread per coarse entry walking every R entry left 27 of
-// 125 threads active and one dependent load in flight: 1,185 us at 48^3 Q2,
-// now 190.)
+// 125 threads active and one dependent load in flight: mean over the levels of
+// 48^3 Q2 1,185 us, now 724.)
 constexpr int kAcGroups = 8;    // groups of 32 lanes
 constexpr int kAcMaxCols = 500;  // 5^3 coarse nodes x 4 fields
 __global__ __launch_bounds__(32 * kAcGroups) void k_amg_Ac(Geo G, const int32_t* __restrict__ rrp,
@@ -603,7 +605,7 @@ __global__ __launch_bounds__(1024) void k_amg_gauss_jordan(int n, double* __rest
 // (rows are marked as used) and the permutation is applied on the way out:
 // with p_k the pivot row of column k, (A^-1)(k, p_j) = M(p_k, j).  Per column
 // one wavefront finds the pivot and two 128-value vectors cross LDS.  (On an
-// n x 2n matrix in global memory: 2,017 us for 108 rows, now 170.)
+// n x 2n matrix in global memory: 2,017 us for the 32^3 cavity's, now 271.)
 constexpr int kAmgRegInv = 128;
 __global__ __launch_bounds__(1024) void k_amg_inverse(int n, const double* __restrict__ M, double* __restrict__ out,
                                                       int* __restrict__ err) {

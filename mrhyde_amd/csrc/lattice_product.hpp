@@ -6,9 +6,9 @@
 // is small, so the floor is the HBM read rate (6.1 TB/s for a plain read).
 // The general product (a lane group per row that finds each entry's column
 // and gathers x through the vector cache) spends its time on column arithmetic
-// and on the gathers.  Q2 FP64, general -> here: 64^3 343 -> 232 us (3.1 ->
-// 4.7 TB/s), 48^3 131 -> 101 us; the Chebyshev step at 48^3 146 -> 106 us, the
-// residual 134 -> 106 us.
+// and on the gathers.  Q2 FP64, general -> here: 64^3 343 -> 229 us (3.1 ->
+// 4.7 TB/s), 48^3 131 -> 98 us; the Chebyshev step at 48^3 146 -> 100 us, the
+// residual 134 -> 99 us.
 //
 // Layout.  The rows of one lattice line (Y, Z) are contiguous, and the line's
 // rows 2e (vertex, 5 columns a run) and 2e + 1 (interior, 3 columns a run)
@@ -62,58 +62,57 @@ struct Q2Tile {
   static constexpr int W = 2 * EX + 4;                          // columns of a line
 };
 
-// runs of the rows of one line: EY x EZ column lines, vo the lane's first
-// entry relative to the line, len its row's columns per run
-template <int EY, int EZ, int LY, int W, bool COLIDX, class TA, class TX, class ACC>
-__device__ __forceinline__ ACC q2_line_sum(const TA* __restrict__ A, const int32_t* __restrict__ ci,
-                                           const TX* __restrict__ x, const ACC* s_x, unsigned vo, unsigned len) {
-  constexpr int NR = EY * EZ;
-  ACC acc = 0;
-  TA a[NR];
-  // (a line's entries are within 4 GB: one uniform base, 32-bit lane offsets)
-  const unsigned b0 = vo * (unsigned)sizeof(TA), bl = len * (unsigned)sizeof(TA);
-#pragma unroll
-  for (int t = 0; t < NR; ++t) a[t] = *(const TA*)((const char*)A + (size_t)(b0 + t * bl));
-#pragma unroll
-  for (int t = 0; t < NR; ++t) {
-    ACC xv;
-    if constexpr (COLIDX) xv = (ACC)x[ci[vo + t * len]];
-    else xv = s_x[((t / EY) * LY + t % EY) * W];
-    acc = fma((ACC)a[t], xv, acc);
-  }
-  return acc;
-}
-
-// epi(row, (A x)_row, epi.load(row)) for every row; the row's operands are
-// loaded ahead of its sums.  COLIDX: columns from the index stream instead of
-// the tile (the same sums in the same order).
+// epi(row, (A x)_row, epi.load(row)) for every row.  Order of the loads: the x
+// tile, the row ends' operands, then the wavefront's matrix values, all in
+// flight together; the tile goes to LDS when it arrives (the values behind it
+// still under way), so a workgroup waits for memory once.  COLIDX: columns from
+// the index stream instead of the tile (the same sums in the same order).
 template <int DIM, bool COLIDX, class TA, class TX, class ACC, class Epi>
 __global__ __launch_bounds__(256) void k_q2_product(BoxMesh m, unsigned nbx, unsigned nby,
                                                     const int32_t* __restrict__ colidx, const TA* __restrict__ A,
                                                     const TX* __restrict__ x, Epi epi) {
   using T = Q2Tile<DIM>;
-  constexpr int LY = T::LY, LZ = T::LZ, W = T::W;
-  __shared__ ACC s_x[COLIDX ? 1 : LZ * LY * W];
+  constexpr int LY = T::LY, LZ = T::LZ, W = T::W, NT = LZ * LY * W, NTL = (NT + 255) / 256;
+  __shared__ ACC s_x[COLIDX ? 1 : NT];
   const unsigned bq = blockIdx.x / nbx;
   const int e0 = (int)(blockIdx.x - bq * nbx) * T::EX;
   const int ey0 = (int)(bq % nby) * T::TY, ez = DIM == 3 ? (int)(bq / nby) : 0;
   const int n0 = m.nel[0], n1 = m.nel[1], n2 = m.nel[2];
   const int N0 = m.nn[0], N1 = m.nn[1], N2 = m.nn[2];
+  // (straight-line code from here to the sums: loads with clamped addresses and
+  // selects in place of branches, so each wait counts the loads behind it)
+  TX xt[NTL];
+  bool xin[NTL];
   if constexpr (!COLIDX) {
     const int X0 = 2 * e0 - 2, Y0 = 2 * ey0 - 2, Z0 = DIM == 3 ? 2 * ez - 2 : 0;
-    for (int k = threadIdx.x; k < LZ * LY * W; k += 256) {
+#pragma unroll
+    for (int i = 0; i < NTL; ++i) {
+      const int k = threadIdx.x + 256 * i;
       const int X = X0 + k % W, Y = Y0 + (k / W) % LY, Z = Z0 + k / (W * LY);
-      const bool in = X >= 0 && X < N0 && Y >= 0 && Y < N1 && Z >= 0 && Z < N2;
-      s_x[k] = in ? (ACC)x[((long)Z * N1 + Y) * N0 + X] : (ACC)0;
+      const bool in = k < NT && X >= 0 && X < N0 && Y >= 0 && Y < N1 && Z >= 0 && Z < N2;
+      unsigned at = in ? (unsigned)(((long)Z * N1 + Y) * N0 + X) : 0u;
+      // (opaque, so that load and select are not folded back into a branch)
+      __asm__ volatile("" : "+v"(at));
+      xt[i] = x[at];
+      xin[i] = in;
     }
-    __syncthreads();
   }
+  // the tile's values to LDS, and an LDS-only barrier: the matrix values loaded
+  // before it stay in flight
+  auto fill_tile = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NTL; ++i)
+      if (256 * i + 256 <= NT || threadIdx.x + 256 * i < NT) s_x[threadIdx.x + 256 * i] = xin[i] ? (ACC)xt[i] : (ACC)0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
   // the wavefront's row line (Y, Z) = (2 ey + jy, 2 ez + jz)
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int jy = wv & 1, jz = DIM == 3 ? wv >> 1 : 0, by = DIM == 3 ? 0 : wv >> 1;
   const int ey = ey0 + by;
   const int Y = 2 * ey + jy, Z = DIM == 3 ? 2 * ez + jz : 0;
-  if (Y >= N1 || Z >= N2) return;
+  const bool on = Y < N1 && Z < N2;
   const bool y5 = !jy && ey > 0 && ey < n1, z5 = DIM == 3 && !jz && ez > 0 && ez < n2;
   const int EY = y5 ? 5 : 3, EZ = DIM == 3 ? (z5 ? 5 : 3) : 1;
   // first column line relative to the tile
@@ -122,7 +121,6 @@ __global__ __launch_bounds__(256) void k_q2_product(BoxMesh m, unsigned nbx, uns
   const unsigned T0 = 8u * n0 + 1, T1 = 8u * n1 + 1;
   const unsigned line = (DIM == 3 ? (unsigned)q2_prefix(Z) * T1 * T0 : 0u) + (unsigned)EZ * (unsigned)q2_prefix(Y) * T0;
   const TA* Al = A + line;
-  const int32_t* cl = COLIDX ? colidx + line : nullptr;
   const int eg = lane >> 3, l = lane & 7;
   const int r = l >= 5;          // 0: vertex row 2e, 1: row 2e + 1
   const int dx = r ? l - 3 : l;  // column 2e - 2 + dx
@@ -130,27 +128,49 @@ __global__ __launch_bounds__(256) void k_q2_product(BoxMesh m, unsigned nbx, uns
   // lane 3 ends the vertex row, lane 4 the other
   const int Xo = 2 * e + (l == 4);
   const long row = ((long)Z * N1 + Y) * N0 + Xo;
-  const bool owner = (l == 3 || l == 4) && Xo < N0;
-  typename Epi::Pre pre{};
-  if (owner) pre = epi.load(row);
+  const bool owner = on && (l == 3 || l == 4) && Xo < N0;
+  const typename Epi::Pre pre = epi.load(owner ? row : 0);
   const int dlo = (r || e == 0) ? 2 : 0;
   const unsigned len = (r || e == 0 || e == n0) ? 3u : 5u;
-  ACC acc = 0;
-  if (X < N0 && dx >= dlo && dx < dlo + (int)len) {
-    const unsigned vo = (unsigned)(EY * EZ) * (unsigned)q2_prefix(X) + (unsigned)(dx - dlo);
-    const ACC* sx = s_x + (COLIDX ? 0 : (zo * LY + yo) * W + 2 * eg + dx);
-    if constexpr (DIM == 3) {
-      if (y5) {
-        if (z5) acc = q2_line_sum<5, 5, LY, W, COLIDX, TA, TX, ACC>(Al, cl, x, sx, vo, len);
-        else acc = q2_line_sum<5, 3, LY, W, COLIDX, TA, TX, ACC>(Al, cl, x, sx, vo, len);
-      } else {
-        if (z5) acc = q2_line_sum<3, 5, LY, W, COLIDX, TA, TX, ACC>(Al, cl, x, sx, vo, len);
-        else acc = q2_line_sum<3, 3, LY, W, COLIDX, TA, TX, ACC>(Al, cl, x, sx, vo, len);
-      }
+  const bool act = on && X < N0 && dx >= dlo && dx < dlo + (int)len;
+  // inactive lanes repeat the line's first entries
+  const unsigned vo = act ? (unsigned)(EY * EZ) * (unsigned)q2_prefix(X) + (unsigned)(dx - dlo) : 0u;
+  // (a line's entries are within 4 GB: one uniform base, 32-bit lane offsets)
+  const unsigned b0 = vo * (unsigned)sizeof(TA), bl = (act ? len : 3u) * (unsigned)sizeof(TA);
+  const ACC* sx = s_x + (COLIDX ? 0 : (zo * LY + yo) * W + 2 * eg + dx);
+  // values, tile to LDS, barrier, sums: the wavefront's 5 or 3 column lines per axis
+  auto sum = [&](auto EYc, auto EZc) __attribute__((always_inline)) {
+    constexpr int CY = decltype(EYc)::value, CZ = decltype(EZc)::value;
+    TA a[CY * CZ];
+#pragma unroll
+    for (int t = 0; t < CY * CZ; ++t) a[t] = *(const TA*)((const char*)Al + (size_t)(b0 + t * bl));
+    ACC acc = 0;
+    if constexpr (COLIDX) {
+      const int32_t* cl = colidx + line;
+#pragma unroll
+      for (int t = 0; t < CY * CZ; ++t) acc = fma((ACC)a[t], (ACC)x[cl[vo + t * (act ? len : 3u)]], acc);
     } else {
-      if (y5) acc = q2_line_sum<5, 1, LY, W, COLIDX, TA, TX, ACC>(Al, cl, x, sx, vo, len);
-      else acc = q2_line_sum<3, 1, LY, W, COLIDX, TA, TX, ACC>(Al, cl, x, sx, vo, len);
+      fill_tile();
+#pragma unroll
+      for (int t = 0; t < CY * CZ; ++t) acc = fma((ACC)a[t], sx[((t / CY) * LY + t % CY) * W], acc);
     }
+    return act ? acc : (ACC)0;
+  };
+  using C1 = std::integral_constant<int, 1>;
+  using C3 = std::integral_constant<int, 3>;
+  using C5 = std::integral_constant<int, 5>;
+  // (every branch passes the one barrier of fill_tile; the branches are uniform
+  // in the wavefront)
+  ACC acc;
+  if (!on) {
+    if constexpr (!COLIDX) fill_tile();
+    return;
+  }
+  if constexpr (DIM == 3) {
+    if (y5) acc = z5 ? sum(C5{}, C5{}) : sum(C5{}, C3{});
+    else acc = z5 ? sum(C3{}, C5{}) : sum(C3{}, C3{});
+  } else {
+    acc = y5 ? sum(C5{}, C1{}) : sum(C3{}, C1{});
   }
   // lanes 0..4 sum to row 2e (in lane 3), lanes 5..7 to row 2e + 1 (in lane 4)
   const ACC fifth = dpp_move<kDppHalfMirror>(acc);  // lane 3: lane 4's part

@@ -875,6 +875,51 @@ struct ResidRow {
   __device__ __forceinline__ void operator()(long row, double ax, Pre p) const { r[row] = (T)((double)p.b - ax); }
 };
 
+// the same ends, and the nodal block-Jacobi update, for four unknowns per node
+// (k_node4_product)
+struct DinvNode {
+  DinvRow r;
+  using Pre = DinvRow::Pre;
+  __device__ __forceinline__ Pre load(unsigned, int, int, unsigned row) const { return r.load(row); }
+  __device__ __forceinline__ void operator()(bool act, unsigned, int, int d, unsigned row, double ax, Pre p) const {
+    if (act && d == 0) r(row, ax, p);
+  }
+};
+template <class T>
+struct ResidNode {
+  ResidRow<T> r;
+  using Pre = typename ResidRow<T>::Pre;
+  __device__ __forceinline__ Pre load(unsigned, int, int, unsigned row) const { return r.load(row); }
+  __device__ __forceinline__ void operator()(bool act, unsigned, int, int d, unsigned row, double ax, Pre p) const {
+    if (act && d == 0) r(row, ax, p);
+  }
+};
+// xout = xin + omega Binv (b - A xin)
+template <class T>
+struct BjNode {
+  const T* __restrict__ binv;
+  const T* __restrict__ b;
+  const T* __restrict__ xin;
+  T* __restrict__ xout;
+  double omega;
+  struct Pre {
+    T b, x, binv;
+  };
+  __device__ __forceinline__ Pre load(unsigned node, int f, int d, unsigned row) const {
+    return {b[row], xin[row], binv[16 * node + 4 * f + d]};
+  }
+  __device__ __forceinline__ void operator()(bool act, unsigned, int, int d, unsigned row, double ax,
+                                             const Pre& p) const {
+    // lane (f, d): the residual of field d, from the first lane of its quad
+    const double r = (double)p.b - ax;
+    const int lane = threadIdx.x & 63;
+    double v = (double)p.binv * __shfl(r, (lane & ~15) + 4 * d, 64);
+    v += dpp_move<kDppXor1>(v);
+    v += dpp_move<kDppXor2>(v);
+    if (act && d == 0) xout[row] = (T)((double)p.x + omega * v);
+  }
+};
+
 // w = s * D^-1 A v  (s = *sp, on the device: the scale applied to v, so v
 // need not be normalised in place)
 template <int LANES, bool LAT>
@@ -979,16 +1024,16 @@ __global__ void k_amg_fill0(long n, T* x) {
   if (i < n) x[i] = (T)0;
 }
 
-// y = M x (add = 0) or y += M x (add = 1)
+// y = M x, or y = y0 + M x (y0 may be y)
 template <int LANES, class T>
 __global__ __launch_bounds__(256) void k_amg_spmv(long n, const int32_t* __restrict__ rp,
                                                   const int32_t* __restrict__ ci, const T* __restrict__ M,
-                                                  const T* __restrict__ x, T* __restrict__ y, int add) {
+                                                  const T* __restrict__ x, const T* y0, T* y) {
   const long row = ((long)blockIdx.x * blockDim.x + threadIdx.x) / LANES;
   const int l = threadIdx.x % LANES;
   if (row >= n) return;
   const double v = row_dot<LANES, T>(rp, CsrCols{ci}, M, x, row, l);
-  if (l == 0) y[row] = (T)(add ? (double)y[row] + v : v);
+  if (l == 0) y[row] = (T)(y0 ? (double)y0[row] + v : v);
 }
 
 // x = Cinv b, one wavefront per row of the dense coarsest inverse.  The
@@ -1029,7 +1074,9 @@ struct AmgLevel {
   DevBuf<double> P, R;
   DevBuf<double> binv;  // nodal nf x nf diagonal-block inverses (block-Jacobi smoother)
   bool lat = false;     // level 0 in the context's lattice pattern: closed-form columns
-  bool q2 = false;      // level 0 by the order-2 lattice product (lattice_product.hpp)
+  // products of lattice_product.hpp: order 2 (level 0), four unknowns per node
+  // (every level; colidx: level 0 with the index stream)
+  bool q2 = false, node4 = false, colidx = false;
   double lambda = 1.0;
   AmgVals<float> f32;
   AmgVals<double> f64;  // FP64 work vectors (values live in A/P/R above)
@@ -1130,6 +1177,8 @@ static void power_estimate(Ctx& c, AmgLevel& L, const double* A, double* v, doub
     const DinvRow end{L.dinv.p, st, w};
     if (L.q2) {
       q2_product<double>(c, A, v, end);
+    } else if (L.node4) {
+      node4_product<double>(c, L.N, L.rp, L.ci, L.colidx, A, v, DinvNode{end});
     } else {
       by_lanes(L.lanes, [&](auto LN) {
         by_lat(L.lat, [&](auto LT) {
@@ -1215,6 +1264,8 @@ void amg_setup(Ctx& c, const double* A, bool fp32) {
   L->lanes = c.spmv_lanes;
   L->lat = c.lattice_cols != 0;
   L->q2 = q2_product_applies(c);
+  L->node4 = node4_product_applies(c);
+  L->colidx = !L->lat;
   L->dinv.alloc(L->n);
   L->ns.alloc(L->n);
   hipLaunchKernelGGL(k_amg_diag, g1(L->n), dim3(256), 0, c.stream, L->n, L->rp, L->ci, A, L->dinv.p);
@@ -1243,6 +1294,8 @@ void amg_setup(Ctx& c, const double* A, bool fp32) {
     C.n = nc;
     for (int d = 0; d < 3; ++d) C.N[d] = ax[d].na;
     C.reach = rc;
+    C.node4 = L->node4 && rc == 1;
+    C.q2 = C.lat = C.colidx = false;
     C.ns.alloc(nc);
     hipLaunchKernelGGL(k_amg_nrm, g1(nc), dim3(256), 0, c.stream, G, L->ns.p, C.ns.p, nc);
     // P
@@ -1408,6 +1461,10 @@ static void level_resid(Ctx& c, AmgLevel& V, const LvView<T>& W, const T* b, con
     q2_product<double>(c, W.A, x, end);
     return;
   }
+  if (V.node4) {
+    node4_product<T>(c, V.N, V.rp, V.ci, V.colidx, W.A, x, ResidNode<T>{end});
+    return;
+  }
   by_lanes(V.lanes, [&](auto LN) {
     by_lat(V.lat, [&](auto LT) {
       constexpr int K = decltype(LN)::value;
@@ -1418,18 +1475,34 @@ static void level_resid(Ctx& c, AmgLevel& V, const LvView<T>& W, const T* b, con
   });
 }
 
-// damped nodal block-Jacobi sweeps: x <- x + omega Binv (b - A x); with
-// zero_x the first sweep starts from x = 0 and needs no residual
+// Damped nodal block-Jacobi sweeps: x <- x + omega Binv (b - A x); with zero_x
+// the first sweep starts from x = 0 and needs no residual.  With four unknowns
+// per node a sweep is one launch from one vector into the other: the starting
+// iterate is expected where bj_start says (x or W.t), and the last sweep ends
+// in x.
+template <class T>
+static T* bj_start(const Amg& H, const AmgLevel& V, const LvView<T>& W, T* x, int zero_x) {
+  const int fused = H.sweeps - (zero_x ? 1 : 0);
+  return V.node4 && (fused & 1) ? W.t : x;
+}
 template <class T>
 static void bj_smooth(Ctx& c, Amg& H, AmgLevel& V, const LvView<T>& W, const T* b, T* x, int zero_x) {
+  T* cur = bj_start<T>(H, V, W, x, zero_x);
   for (int s = 0; s < H.sweeps; ++s) {
+    const bool zero = zero_x && s == 0;
+    if (!zero && V.node4) {
+      T* nxt = cur == x ? W.t : x;
+      node4_product<T>(c, V.N, V.rp, V.ci, V.colidx, W.A, cur, BjNode<T>{W.binv, b, cur, nxt, H.omega});
+      cur = nxt;
+      continue;
+    }
     const T* r = b;
-    if (!(zero_x && s == 0)) {
-      level_resid<T>(c, V, W, b, x, W.t);
+    if (!zero) {
+      level_resid<T>(c, V, W, b, cur, W.t);
       r = W.t;
     }
-    hipLaunchKernelGGL(k_amg_bj<T>, g1(V.n), dim3(256), 0, c.stream, V.n, H.nf, W.binv, r, x, x, H.omega,
-                       (int)(zero_x && s == 0));
+    hipLaunchKernelGGL(k_amg_bj<T>, g1(V.n), dim3(256), 0, c.stream, V.n, H.nf, W.binv, r, cur, cur, H.omega,
+                       (int)zero);
   }
 }
 
@@ -1494,7 +1567,7 @@ static void vcycle(Ctx& c, Amg& H, const T* A0, const double* cinv, const T* v, 
     by_lanes(V.rlane, [&](auto LN) {
       constexpr int K = decltype(LN)::value;
       hipLaunchKernelGGL((k_amg_spmv<K, T>), g1(nc * K), dim3(256), 0, c.stream, nc, V.rrp.p, V.rci.p, W.R, W.r,
-                         Wc.b, 0);
+                         (const T*)nullptr, Wc.b);
     });
   }
   // coarsest
@@ -1515,7 +1588,7 @@ static void vcycle(Ctx& c, Amg& H, const T* A0, const double* cinv, const T* v, 
     by_lanes(V.plane, [&](auto LN) {
       constexpr int K = decltype(LN)::value;
       hipLaunchKernelGGL((k_amg_spmv<K, T>), g1(V.n * K), dim3(256), 0, c.stream, V.n, V.prp.p, V.pci.p, W.P, Wc.x,
-                         x, 1);
+                         x, H.smoother == kSmootherBlockJacobi ? bj_start<T>(H, V, W, x, 0) : x);
     });
     if (H.smoother == kSmootherBlockJacobi) {
       bj_smooth<T>(c, H, V, W, b, x, 0);

@@ -81,8 +81,24 @@ struct StoreRow {
   __device__ __forceinline__ void operator()(long row, T v, Pre) const { y[row] = v; }
 };
 
+template <class T>
+struct StoreNodeRow {
+  T* __restrict__ y;
+  struct Pre {};
+  __device__ __forceinline__ Pre load(unsigned, int, int, unsigned) const { return {}; }
+  __device__ __forceinline__ void operator()(bool act, unsigned, int, int d, unsigned row, double v, Pre) const {
+    if (act && d == 0) y[row] = (T)v;
+  }
+};
+
 template <class TA, class TX>
 static void spmv_t(Ctx& c, const TA* A, const TX* s, const TX* x, TX* y) {
+  if constexpr (std::is_same<TA, TX>::value) {
+    if (!s && node4_product_applies(c)) {
+      node4_product<TX>(c, c.mesh.nn, c.rowptr.p, c.colidx.p, !c.lattice_cols, A, x, StoreNodeRow<TX>{y});
+      return;
+    }
+  }
   if (!s && q2_product_applies(c)) {
     q2_product<TX>(c, A, x, StoreRow<TX>{y});
     return;

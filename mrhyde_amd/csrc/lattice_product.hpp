@@ -207,4 +207,107 @@ void q2_product(Ctx& c, const TA* A, const TX* x, const Epi& epi) {
   else go(std::integral_constant<int, 2>{});
 }
 
+// ---------------------------------------------------------------------------
+// Order-1 hexahedral lattices with four unknowns per node (3-D Navier-Stokes,
+// and every coarse level of its multigrid hierarchy: the same 27-node boxes).
+//
+// Sixteen lanes take a node: lane 4 f + d the row of field f and the column
+// node X - 1 + d of each of the nine (y, z) lines, i.e. four consecutive values
+// and one node's four unknowns per line, both 16- or 32-byte loads; d = 3 idles
+// through the sums.  The four lanes of a row meet by DPP, and the node's four
+// row sums sit in one group, so the nodal block-Jacobi update follows in the
+// same launch (one lane per entry of the 4 x 4 inverse).  Entry by entry with
+// the column found for each, a sweep of the 32^3 FP32 cavity took 15.0 us (the
+// residual 11.4 and a launch of 3.6 for the update, mean over the two smoothed
+// levels); now 9.1 us.
+// ---------------------------------------------------------------------------
+struct NodeLattice {
+  int N[3];
+};
+
+template <class T>
+struct alignas(sizeof(T)) Quad {
+  T v[4];
+};
+
+// end(node, f, d, row, sum): called by the sixteen lanes of every node, sum the
+// row's on all four lanes of its quad.  COLIDX: columns from the index stream
+// (the same sums in the same order).
+template <bool COLIDX, class T, class End>
+__global__ __launch_bounds__(256) void k_node4_product(NodeLattice L, long nnode, const int32_t* __restrict__ rp,
+                                                       const int32_t* __restrict__ colidx, const T* __restrict__ A,
+                                                       const T* __restrict__ x, End end) {
+  const unsigned gid = blockIdx.x * 256u + threadIdx.x;
+  const unsigned nd = gid >> 4;
+  const bool act = nd < (unsigned)nnode;
+  const unsigned node = act ? nd : 0u;
+  const int f = (threadIdx.x >> 2) & 3, d = threadIdx.x & 3;
+  const int N0 = L.N[0], N1 = L.N[1], N2 = L.N[2];
+  const unsigned yz = node / (unsigned)N0;
+  const int X = (int)(node - yz * (unsigned)N0);
+  const int Z = (int)(yz / (unsigned)N1), Y = (int)(yz - (unsigned)Z * (unsigned)N1);
+  const unsigned row = 4 * node + f;
+  const typename End::Pre pre = end.load(node, f, d, row);
+  const unsigned b = (unsigned)rp[row];
+  const int dx = d < 3 ? d : 2;
+  const bool inner = X > 0 && X < N0 - 1 && Y > 0 && Y < N1 - 1 && Z > 0 && Z < N2 - 1;
+  double acc = 0.0;
+  auto term = [&](unsigned k, unsigned col) __attribute__((always_inline)) {
+    const Quad<T> a = *(const Quad<T>*)(A + k);
+    const unsigned j = COLIDX ? (unsigned)colidx[k] : col;
+    const Quad<T> v = *(const Quad<T>*)(x + j);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc = fma((double)a.v[i], (double)v.v[i], acc);
+  };
+  if (__all(inner)) {
+    // all lines in flight ahead of the sums
+    Quad<T> a[9], v[9];
+    const unsigned k0 = b + 4 * dx, c0 = 4 * (node - (unsigned)N0 * (1 + (unsigned)N1) - 1 + dx);
+#pragma unroll
+    for (int t = 0; t < 9; ++t) {
+      const unsigned k = k0 + 12 * t;
+      a[t] = *(const Quad<T>*)(A + k);
+      unsigned col;
+      if constexpr (COLIDX) col = (unsigned)colidx[k];
+      else col = c0 + 4 * (unsigned)N0 * (t % 3 + (unsigned)N1 * (t / 3));
+      v[t] = *(const Quad<T>*)(x + col);
+    }
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc = fma((double)a[t].v[i], (double)v[t].v[i], acc);
+  } else {
+    const int x0 = X > 0 ? X - 1 : 0, x1 = X < N0 - 1 ? X + 1 : X, y0 = Y > 0 ? Y - 1 : 0, y1 = Y < N1 - 1 ? Y + 1 : Y,
+              z0 = Z > 0 ? Z - 1 : 0, z1 = Z < N2 - 1 ? Z + 1 : Z;
+    const int xc = X - 1 + dx;
+    const unsigned ex = x1 - x0 + 1;
+    if (xc >= x0 && xc <= x1) {
+      unsigned k = b + 4 * (unsigned)(xc - x0);
+      for (int z = z0; z <= z1; ++z)
+        for (int y = y0; y <= y1; ++y, k += 4 * ex) term(k, 4 * (((unsigned)z * N1 + y) * (unsigned)N0 + xc));
+    }
+  }
+  if (d == 3) acc = 0.0;
+  acc += dpp_move<kDppXor1>(acc);
+  acc += dpp_move<kDppXor2>(acc);
+  end(act, node, f, d, row, acc, pre);
+}
+
+inline bool node4_product_applies(const Ctx& c) {
+  return c.mesh.p == 1 && c.mesh.nf == 4 && c.mesh.dim == 3 && c.spmv_lanes == c.spmv_lanes_default;
+}
+
+template <class T, class End>
+void node4_product(Ctx& c, const int* N, const int32_t* rp, const int32_t* ci, bool colidx, const T* A, const T* x,
+                   const End& end) {
+  const NodeLattice L{{N[0], N[1], N[2]}};
+  const long nnode = (long)N[0] * N[1] * N[2];
+  const dim3 grid((unsigned)((nnode * 16 + 255) / 256));
+  if (colidx)
+    hipLaunchKernelGGL((k_node4_product<true, T, End>), grid, dim3(256), 0, c.stream, L, nnode, rp, ci, A, x, end);
+  else
+    hipLaunchKernelGGL((k_node4_product<false, T, End>), grid, dim3(256), 0, c.stream, L, nnode, rp, ci, A, x, end);
+  MHX_HIP(hipGetLastError());
+}
+
 }  // namespace mhx

@@ -446,72 +446,91 @@ __global__ __launch_bounds__(kAmgBlk) void k_amg_AP(Geo G, LevelBox B, long n, c
   }
 }
 
-// A_c = R (A P): one workgroup per coarse row (I, f).  Groups of 32 lanes take
-// the entries of the R row in turn, lane s the slot s of the entry's 27-slot AP
-// boxes (one contiguous read per box, four R entries in flight), and add into
-// the group's own copy of the coarse row in LDS; the copies are summed in
-// group order.  (One thread per coarse entry walking every R entry left 27 of
-// 125 threads active and one dependent load in flight: mean over the levels of
-// 48^3 Q2 1,185 us, now 724.)
-constexpr int kAcGroups = 8;    // groups of 32 lanes
+// A_c = R (A P): one workgroup per coarse row (I, f).  The R row is a box of
+// fine nodes; groups of 32 lanes take its (y, z) lines in turn, lane s the slot s
+// of the nodes' 27-slot AP boxes (a contiguous read per box, at least eight in
+// flight), and add into the group's own copy of the coarse row in LDS; the
+// copies are summed in group order.  Where a node's AP box starts relative to
+// the coarse row's comes from three small tables.  (One thread per coarse entry
+// walking every R entry left 27 of 125 threads active and one dependent load in
+// flight: mean over the levels of 48^3 Q2 1,185 us; with the tables looked up
+// per entry in global memory 724; the two levels of the 32^3 cavity 678 -> 217.)
+constexpr int kAcGroups = 8;     // groups of 32 lanes
 constexpr int kAcMaxCols = 500;  // 5^3 coarse nodes x 4 fields
+constexpr int kAcMaxExt = 64;    // nodes of an R row along an axis
+template <int NF>
 __global__ __launch_bounds__(32 * kAcGroups) void k_amg_Ac(Geo G, const int32_t* __restrict__ rrp,
-                                                           const int32_t* __restrict__ rci,
                                                            const double* __restrict__ R,
                                                            const double* __restrict__ AP,
                                                            const double* __restrict__ nrm,
                                                            const int32_t* __restrict__ arp,
                                                            int32_t* __restrict__ aci, double* __restrict__ Ac) {
   __shared__ double s_acc[kAcGroups][kAcMaxCols];
+  __shared__ int s_alo[3][kAcMaxExt], s_aex[3][kAcMaxExt];
   const long cr = blockIdx.x;
-  const int nf = G.nf;
-  const long I = cr / nf;
+  const long I = cr / NF;
   int Ic[3];
   node_xyz(I, G.ax[0].na, G.ax[1].na, Ic[0], Ic[1], Ic[2]);
-  const int clx = G.ax[0].t[kClo][Ic[0]], cly = G.ax[1].t[kClo][Ic[1]], clz = G.ax[2].t[kClo][Ic[2]];
-  const int cex = G.ax[0].t[kCext][Ic[0]], cey = G.ax[1].t[kCext][Ic[1]];
+  int cl[3], ce[3], rl[3], re[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    cl[a] = G.ax[a].t[kClo][Ic[a]];
+    ce[a] = G.ax[a].t[kCext][Ic[a]];
+    rl[a] = G.ax[a].t[kRlo][Ic[a]];
+    re[a] = G.ax[a].t[kRext][Ic[a]];
+    for (int t = threadIdx.x; t < re[a]; t += 32 * kAcGroups) {
+      s_alo[a][t] = G.ax[a].t[kAplo][rl[a] + t] - cl[a];
+      s_aex[a][t] = G.ax[a].t[kApext][rl[a] + t];
+    }
+  }
   const long base = arp[cr];
   const int cnt = arp[cr + 1] - arp[cr];
   const int grp = threadIdx.x / 32, s = threadIdx.x % 32;
   const int sx = s % 3, sy = (s / 3) % 3, sz = s / 9;  // s < 27
   double* acc = s_acc[grp];
   for (int k = s; k < cnt; k += 32) acc[k] = 0.0;
-  const int rb = rrp[cr], re = rrp[cr + 1];
-  constexpr int U = 4;
-  for (int k0 = rb + grp; k0 < re; k0 += kAcGroups * U) {
-    double rv[U];
-    long row[U];
-    int at[U];  // the lane's coarse entry (-1: none)
+  __syncthreads();
+  const double* Rr = R + rrp[cr];
+  constexpr int UX = NF == 1 ? 8 : (NF == 2 ? 2 : 1);  // nodes of a line in flight
+  for (int q = grp; q < re[1] * re[2]; q += kAcGroups) {
+    const int ly = q % re[1], lz = q / re[1];
+    const int jy = s_alo[1][ly] + sy, jz = s_alo[2][lz] + sz;
+    // (the coarse box holds every aggregate that a row of R reaches)
+    const bool line = s < 27 && sy < s_aex[1][ly] && sz < s_aex[2][lz] && jy >= 0 && jy < ce[1] && jz >= 0 &&
+                      jz < ce[2];
+    const int yz = (jz * ce[1] + jy) * ce[0];
+    const long node0 = rl[0] + (long)G.ax[0].n * ((rl[1] + ly) + (long)G.ax[1].n * (rl[2] + lz));
+    const double* Rl = Rr + (long)q * re[0] * NF;
+    for (int x0 = 0; x0 < re[0]; x0 += UX) {
+      double v[UX][NF][NF], rv[UX][NF];
+      int at[UX];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + u * kAcGroups;
-      at[u] = -1;
-      rv[u] = 0.0;
-      row[u] = 0;
-      if (k < re) {
-        const long i = rci[k];
-        rv[u] = R[k];
-        row[u] = i;
-        int px, py, pz;
-        node_xyz((long)((unsigned)i / (unsigned)nf), G.ax[0].n, G.ax[1].n, px, py, pz);
-        if (s < 27 && sx < G.ax[0].t[kApext][px] && sy < G.ax[1].t[kApext][py] && sz < G.ax[2].t[kApext][pz]) {
-          const int jx = G.ax[0].t[kAplo][px] + sx - clx, jy = G.ax[1].t[kAplo][py] + sy - cly,
-                    jz = G.ax[2].t[kAplo][pz] + sz - clz;
-          // (the coarse box holds every aggregate that a row of R reaches)
-          if (jx >= 0 && jx < cex && jy >= 0 && jy < cey && jz >= 0) {
-            const int cell = (jz * cey + jy) * cex + jx;
-            if (cell * nf < cnt) at[u] = cell * nf;
-          }
+      for (int u = 0; u < UX; ++u) {
+        const int x = x0 + u;
+        at[u] = -1;
+        if (x < re[0]) {
+          const int jx = s_alo[0][x] + sx;
+          if (line && sx < s_aex[0][x] && jx >= 0 && jx < ce[0]) at[u] = (yz + jx) * NF;
+#pragma unroll
+          for (int f = 0; f < NF; ++f) rv[u][f] = Rl[x * NF + f];
+        }
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+          for (int g = 0; g < NF; ++g)
+            v[u][f][g] = at[u] >= 0 ? AP[(((node0 + x) * NF + f) * NF + g) * 27 + s] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < UX; ++u) {
+        if (at[u] < 0) continue;
+#pragma unroll
+        for (int g = 0; g < NF; ++g) {
+          double t = acc[at[u] + g];
+#pragma unroll
+          for (int f = 0; f < NF; ++f) t = fma(rv[u][f], v[u][f][g], t);
+          acc[at[u] + g] = t;
         }
       }
-    }
-    for (int g = 0; g < nf; ++g) {
-      double v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = at[u] >= 0 ? AP[(row[u] * nf + g) * 27 + s] : 0.0;
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (at[u] >= 0) acc[at[u] + g] = fma(rv[u], v[u], acc[at[u] + g]);
     }
   }
   __syncthreads();
@@ -520,9 +539,9 @@ __global__ __launch_bounds__(32 * kAcGroups) void k_amg_Ac(Geo G, const int32_t*
     double v = 0.0;
 #pragma unroll
     for (int q = 0; q < kAcGroups; ++q) v += s_acc[q][e];
-    const int g = e % nf, cell = e / nf;
-    const int jx = clx + cell % cex, jy = cly + (cell / cex) % cey, jz = clz + cell / (cex * cey);
-    const long col = (jx + (long)nax * (jy + (long)nay * jz)) * nf + g;
+    const int g = e % NF, cell = e / NF;
+    const int jx = cl[0] + cell % ce[0], jy = cl[1] + (cell / ce[0]) % ce[1], jz = cl[2] + cell / (ce[0] * ce[1]);
+    const long col = (jx + (long)nax * (jy + (long)nay * jz)) * NF + g;
     aci[base + e] = (int32_t)col;
     // an aggregate whose near-null space vanished (all its nodes strong
     // Dirichlet) has an empty prolongator column: an identity row keeps A_c
@@ -1327,10 +1346,24 @@ void amg_setup(Ctx& c, const double* A, bool fp32) {
     C.A.alloc(a_nnz);
     hipLaunchKernelGGL(k_box_rowptr, g1(nc + 1), dim3(256), 0, c.stream, G, 1, (int)kCext, (int)kSc, nc,
                        C.rp_own.p);
-    MHX_REQUIRE((2 * rc + 1) * (2 * rc + 1) * (2 * rc + 1) * nf <= kAcMaxCols, MHX_ERR_UNSUPPORTED,
-                "AMG: coarse operator row wider than the Galerkin kernel's");
-    hipLaunchKernelGGL(k_amg_Ac, dim3((unsigned)nc), dim3(32 * kAcGroups), 0, c.stream, G, L->rrp.p, L->rci.p, L->R.p,
-                       H.scratch.p, C.ns.p, C.rp_own.p, C.ci_own.p, C.A.p);
+    for (int d = 0; d < 3; ++d) {
+      const auto& rx = ax[d].t[kRext];
+      const auto& cx = ax[d].t[kCext];
+      MHX_REQUIRE(*std::max_element(rx.begin(), rx.end()) <= kAcMaxExt, MHX_ERR_UNSUPPORTED,
+                  "AMG: restriction row longer than the Galerkin kernel's");
+      MHX_REQUIRE(*std::max_element(cx.begin(), cx.end()) <= 5, MHX_ERR_UNSUPPORTED,
+                  "AMG: coarse operator row wider than the Galerkin kernel's");
+    }
+    auto galerkin = [&](auto F) {
+      hipLaunchKernelGGL((k_amg_Ac<decltype(F)::value>), dim3((unsigned)nc), dim3(32 * kAcGroups), 0, c.stream, G,
+                         L->rrp.p, L->R.p, H.scratch.p, C.ns.p, C.rp_own.p, C.ci_own.p, C.A.p);
+    };
+    switch (nf) {
+      case 1: galerkin(std::integral_constant<int, 1>{}); break;
+      case 2: galerkin(std::integral_constant<int, 2>{}); break;
+      case 3: galerkin(std::integral_constant<int, 3>{}); break;
+      default: galerkin(std::integral_constant<int, 4>{}); break;
+    }
     MHX_HIP(hipGetLastError());
     L->plane = lanes_for((double)p_nnz / (double)n);
     L->rlane = lanes_for((double)r_nnz / (double)nc);

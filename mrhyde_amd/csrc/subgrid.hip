@@ -21,11 +21,15 @@
 // a global counter (largest instances first) until the queue is empty, so
 // every workgroup reaches the exit.  The instance lives on chip: the search
 // direction p and the element conductivities in LDS, each thread's share of
-// x, r and the Jacobi scaling in registers.  The operator is applied node by
-// node from the 27 neighbouring p values and the 8 surrounding element
-// conductivities with the closed-form Q1 stiffness of the instance's box
-// element (exact for the 2x2x2 Gauss rule the reference uses), i.e. the
-// assembled 27-point row is formed on the fly instead of being stored.
+// x, r and the Jacobi scaling in registers.  A thread owns a run of interior
+// nodes of one z column and sweeps its planes upwards: the operator is the
+// closed-form Q1 stiffness of the instance's box element (exact for the
+// 2x2x2 Gauss rule the reference uses), and a plane's values are read once
+// for the nodes below, in and above it.  Per node 9 p values and 4
+// conductivities from LDS and about 30 floating-point operations on the unit
+// cube; one node at a time from its 27 neighbours and 8 elements took 35 LDS
+// reads, 72 operations and two index divisions (1,024 unit cubes in FP64:
+// 786 us a batch).
 
 #include <algorithm>
 #include <cmath>
@@ -50,25 +54,6 @@ inline void box_stencil(double hx, double hy, double hz, double kv[8]) {
     kv[p] = cx * S[dx] * M[dy] * M[dz] + cy * M[dx] * S[dy] * M[dz] + cz * M[dx] * M[dy] * S[dz];
   }
 }
-
-// the unit-cube table (hx = hy = hz = 1): K_h = h K_unit for a cube of side h
-struct K8 {
-  double v[8][8];
-};
-constexpr K8 make_k8() {
-  K8 k{};
-  const double M[2][2] = {{1.0 / 3.0, 1.0 / 6.0}, {1.0 / 6.0, 1.0 / 3.0}};
-  const double S[2][2] = {{1.0, -1.0}, {-1.0, 1.0}};
-  for (int a = 0; a < 8; ++a)
-    for (int b = 0; b < 8; ++b) {
-      const int ax = a & 1, ay = (a >> 1) & 1, az = (a >> 2) & 1;
-      const int bx = b & 1, by = (b >> 1) & 1, bz = (b >> 2) & 1;
-      k.v[a][b] = S[ax][bx] * M[ay][by] * M[az][bz] + M[ax][bx] * S[ay][by] * M[az][bz] +
-                  M[ax][bx] * M[ay][by] * S[az][bz];
-    }
-  return k;
-}
-constexpr K8 kK8 = make_k8();
 
 constexpr int kSgMaxN = 16;                                   // elements per axis
 constexpr int kSgMaxNodes = (kSgMaxN + 1) * (kSgMaxN + 1) * (kSgMaxN + 1);
@@ -104,157 +89,187 @@ struct SgArgs {
 
 __global__ void k_sg_reset(unsigned int* q) { *q = 0u; }
 
-// q = A p at node (ix,iy,iz) (interior), p and k in LDS.  BOX (the general
-// instance: a box, possibly with sources): kv holds the box element's
-// stiffness entries by coordinate-difference pattern; else the instance is
-// the unit cube without sources and its element stiffness h K_unit (h = 1/n)
-// comes from the compile-time table.
-template <class T, bool BOX>
-__device__ __forceinline__ T sg_apply(const T* __restrict__ p, const T* __restrict__ kk, int n, const T (&kv)[8],
-                                      int ix, int iy, int iz) {
-  const int n1 = n + 1;
-  T P[3][3][3];
+// A thread's nodes: the interior column (ix, iy), z = z0 .. z0 + cnt - 1.
+struct SgCol {
+  int p, e;  // node (ix, iy, z0) in the nodal arrays; element (ix-1, iy-1, z0-1)
+  int cnt;
+};
+
+// q = A p at the thread's nodes, p and k in LDS: out(s, q_s, p_s) for s <
+// cnt.  BOX (the general instance: a box, possibly with sources): kv holds
+// the box element's stiffness entries by coordinate-difference pattern; else
+// the instance is the unit cube, whose element couples a node to itself (1/3)
+// and to its face and body diagonals (-1/12) and not along edges, scaled by
+// h = 1 / n.
+//
+// Plane j (z = z0 - 1 + j) lies below node j, holds node j - 1 and lies above
+// node j - 2; element layer j is between planes j and j + 1.  Straight-line
+// over C slots; slots from cnt on give values that the caller drops.
+template <class T, int C, bool BOX, class Out>
+__device__ __forceinline__ void sg_apply(const T* __restrict__ p, const T* __restrict__ kk, int n, const T (&kv)[8],
+                                         const SgCol& c, Out&& out) {
+  const int n1 = n + 1, pl = n1 * n1, el = n * n;
+  const T* P = p + c.p - pl;
+  const T* K = kk + c.e;
+  const T h = (T)-1 / (T)(12 * n);
+  T kl[4] = {0, 0, 0, 0}, prev = 0, cur = 0, pc_prev = 0;
 #pragma unroll
-  for (int dz = 0; dz < 3; ++dz)
-#pragma unroll
-    for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-      for (int dx = 0; dx < 3; ++dx) P[dz][dy][dx] = p[(ix - 1 + dx) + n1 * ((iy - 1 + dy) + n1 * (iz - 1 + dz))];
-  T acc = 0;
-#pragma unroll
-  for (int o = 0; o < 8; ++o) {
-    const int ox = o & 1, oy = (o >> 1) & 1, oz = (o >> 2) & 1;
-    const T ke = kk[(ix - 1 + ox) + n * ((iy - 1 + oy) + n * (iz - 1 + oz))];
-    const int a = (1 - ox) + 2 * (1 - oy) + 4 * (1 - oz);
-    T s = 0;
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const int bx = b & 1, by = (b >> 1) & 1, bz = (b >> 2) & 1;
-      const int ax = a & 1, ay = (a >> 1) & 1, az = (a >> 2) & 1;
-      const T kab = BOX ? kv[(ax ^ bx) | ((ay ^ by) << 1) | ((az ^ bz) << 2)] : (T)kK8.v[a][b];
-      s += kab * P[oz + bz][oy + by][ox + bx];
+  for (int j = 0; j < C + 2; ++j) {
+    // one plane at a time (bounds the live registers)
+    __builtin_amdgcn_sched_barrier(0);
+    // corner ab of the plane: a = 0, 1: x - 1, x + 1; b: y; edge neighbours x, y
+    const T m0 = P[-1 - n1], m1 = P[1 - n1], m2 = P[-1 + n1], m3 = P[1 + n1];
+    const T xm = P[-1], xp = P[1], ym = P[-n1], yp = P[n1], pc = P[0];
+    const T kh[4] = {K[0], K[1], K[n], K[n + 1]};
+    // what an element above or below the plane adds per unit conductivity
+    T t[4];
+    if constexpr (BOX) {
+      const T ax = kv[5] * xm, bx = kv[5] * xp, cz = kv[4] * pc;
+      const T ay = fma(kv[6], ym, cz), by = fma(kv[6], yp, cz);
+      t[0] = fma(kv[7], m0, ax + ay);
+      t[1] = fma(kv[7], m1, bx + ay);
+      t[2] = fma(kv[7], m2, ax + by);
+      t[3] = fma(kv[7], m3, bx + by);
+    } else {
+      t[0] = m0 + (xm + ym);
+      t[1] = m1 + (xp + ym);
+      t[2] = m2 + (xm + yp);
+      t[3] = m3 + (xp + yp);
     }
-    acc += ke * s;
-  }
-  if constexpr (BOX) return acc;
-  else return acc * ((T)1 / (T)n);
-}
-
-// b_i / vol8: the sum of the element sources around node (ix,iy,iz)
-__device__ __forceinline__ double sg_src(const double* __restrict__ f, int n, int ix, int iy, int iz) {
-  double s = 0.0;
+    if (j >= 2) {
+      const T q = fma(kl[0], t[0], fma(kl[1], t[1], fma(kl[2], t[2], fma(kl[3], t[3], prev))));
+      if constexpr (BOX) out(j - 2, q, pc_prev);
+      else out(j - 2, q * h, pc_prev);
+    }
+    if (j >= 1 && j <= C) {
+      const T s0 = kl[0] + kh[0], s1 = kl[1] + kh[1], s2 = kl[2] + kh[2], s3 = kl[3] + kh[3];
+      if constexpr (BOX) {
+        const T ax = kv[1] * xm, bx = kv[1] * xp, cc = kv[0] * pc;
+        const T ay = fma(kv[2], ym, cc), by = fma(kv[2], yp, cc);
+        cur = fma(s0, fma(kv[3], m0, ax + ay), cur);
+        cur = fma(s1, fma(kv[3], m1, bx + ay), cur);
+        cur = fma(s2, fma(kv[3], m2, ax + by), cur);
+        cur = fma(s3, fma(kv[3], m3, bx + by), cur);
+      } else {
+        const T d = fma(s0, m0, fma(s1, m1, fma(s2, m2, fma(s3, m3, cur))));
+        // in units of -h / 12: the diagonals, and -4 (h / 3) for the node itself
+        cur = fma((T)-4 * ((s0 + s1) + (s2 + s3)), pc, d);
+      }
+    }
+    T nxt = 0;
+    if (j < C) nxt = fma(kh[0], t[0], fma(kh[1], t[1], fma(kh[2], t[2], kh[3] * t[3])));
+    prev = cur;
+    cur = nxt;
+    pc_prev = pc;
 #pragma unroll
-  for (int o = 0; o < 8; ++o) {
-    const int ox = o & 1, oy = (o >> 1) & 1, oz = (o >> 2) & 1;
-    s += f[(ix - 1 + ox) + n * ((iy - 1 + oy) + n * (iz - 1 + oz))];
+    for (int q = 0; q < 4; ++q) kl[q] = kh[q];
+    // past the thread's last plane and layer: stay there (unused slots)
+    P += j <= c.cnt ? pl : 0;
+    K += j < c.cnt ? el : 0;
   }
-  return s;
 }
 
-template <class T, bool BOX>
-__device__ __forceinline__ T sg_diag(const T* __restrict__ kk, int n, T kv0, int ix, int iy, int iz) {
-  T d = 0;
+// sum of the eight conductivities around the thread's nodes (the operator's
+// diagonal is kv[0] times it, h / 3 on the unit cube) and, where f is given,
+// of the element sources: out(s, sum k, sum f)
+template <int C, class Out>
+__device__ __forceinline__ void sg_around(const double* __restrict__ kk, const double* __restrict__ f, int n,
+                                          const SgCol& c, Out&& out) {
+  double klo = 0.0, flo = 0.0;
 #pragma unroll
-  for (int o = 0; o < 8; ++o) {
-    const int ox = o & 1, oy = (o >> 1) & 1, oz = (o >> 2) & 1;
-    const int a = (1 - ox) + 2 * (1 - oy) + 4 * (1 - oz);
-    const T ke = kk[(ix - 1 + ox) + n * ((iy - 1 + oy) + n * (iz - 1 + oz))];
-    d += BOX ? ke : ke * (T)kK8.v[a][a];
+  for (int j = 0; j < C + 1; ++j) {
+    const int e = c.e + min(j, max(c.cnt - 1, 0) + 1) * n * n;
+    const double khi = (kk[e] + kk[e + 1]) + (kk[e + n] + kk[e + n + 1]);
+    const double fhi = f ? (f[e] + f[e + 1]) + (f[e + n] + f[e + n + 1]) : 0.0;
+    if (j >= 1) out(j - 1, klo + khi, flo + fhi);
+    klo = khi;
+    flo = fhi;
   }
-  if constexpr (BOX) return d * kv0;  // once per node at set-up
-  else return d / (T)n;
 }
 
-// Sum of two values over the workgroup, returned to every thread.
+// Sum of two values over the workgroup, returned to every thread; red holds
+// two copies used in turn (buf), so one barrier separates a copy's readers
+// from its next writers.
 template <int WG, class T>
-__device__ __forceinline__ void wg_sum2(T& a, T& b, T* red) {
+__device__ __forceinline__ void wg_sum2(T& a, T& b, T* red, int& buf) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     a += __shfl_xor(a, off, 64);
     b += __shfl_xor(b, off, 64);
   }
+  T* r = red + buf * 2 * (WG / 64);
+  buf ^= 1;
   const int w = threadIdx.x / 64, l = threadIdx.x % 64;
   if (l == 0) {
-    red[2 * w] = a;
-    red[2 * w + 1] = b;
+    r[2 * w] = a;
+    r[2 * w + 1] = b;
   }
   __syncthreads();
   a = 0;
   b = 0;
 #pragma unroll
   for (int i = 0; i < WG / 64; ++i) {
-    a += red[2 * i];
-    b += red[2 * i + 1];
+    a += r[2 * i];
+    b += r[2 * i + 1];
   }
-  __syncthreads();
 }
 
 // Jacobi-PCG on the interior nodes (SolverManager::PCG algorithm):
 //   x += CG solution of A x = r_in (r_in given in the thread's slots),
-// stopping when ||r|| / ||r_in|| <= tol.  Returns iterations; rr_out = ||r||^2.
-template <int WG, int S, class T, bool BOX>
-__device__ __forceinline__ int sg_pcg(int n, const T* kk, const T (&kv)[8], T* p_lds, T* red, T (&x)[S], T (&r)[S],
-                                      const T (&dinv)[S], bool (&in)[S], int (&node)[S], double tol, int max_iters,
-                                      T& rr_out) {
-  const int n1 = n + 1, nn = n1 * n1 * n1;
-  T pp[S];
+// stopping when ||r|| / ||r_in|| <= tol.  p_lds is 0 on the boundary nodes.
+// Returns iterations; rr_out = ||r||^2.
+template <int WG, int C, class T, bool BOX>
+__device__ __forceinline__ int sg_pcg(int n, const T* kk, const T (&kv)[8], T* p_lds, T* red, T (&x)[C], T (&r)[C],
+                                      const T (&dinv)[C], SgCol& c, double tol, int max_iters, T& rr_out) {
+  const int pl = (n + 1) * (n + 1);
+  int buf = 0;
   T rr = 0, rz = 0;
 #pragma unroll
-  for (int s = 0; s < S; ++s) {
+  for (int s = 0; s < C; ++s) {
     rr += r[s] * r[s];
-    rz += r[s] * (dinv[s] * r[s]);  // z = D^-1 r (dinv is 0 off the interior)
+    rz += r[s] * (dinv[s] * r[s]);  // z = D^-1 r (dinv is 0 in unused slots)
   }
-  wg_sum2<WG>(rr, rz, red);
+  wg_sum2<WG>(rr, rz, red, buf);
   const T rr0 = rr;
   int it = 0;
   if (rr0 > (T)0) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      pp[s] = dinv[s] * r[s];
-      if (node[s] < nn) p_lds[node[s]] = pp[s];
-    }
+    for (int s = 0; s < C; ++s)
+      if (s < c.cnt) p_lds[c.p + s * pl] = dinv[s] * r[s];
     __syncthreads();
     const T tol2 = (T)(tol * tol);
     while (it < max_iters) {
-      // The node indices are made opaque once per iteration, so the 27-point
-      // gather addresses are recomputed inside the loop instead of being
-      // hoisted for every slot and held across iterations.
+      // (opaque once per iteration: the planes' addresses are formed in the
+      // sweep instead of being hoisted and held across iterations)
+      __asm__ volatile("" : "+v"(c.p), "+v"(c.e));
+      T q[C];
 #pragma unroll
-      for (int s = 0; s < S; ++s) __asm__ volatile("" : "+v"(node[s]));
-      T q[S];
+      for (int s = 0; s < C; ++s) q[s] = 0;
       T pq = 0, dummy = 0;
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        // one slot's 27-point gather at a time (bounds the live registers)
-        __builtin_amdgcn_sched_barrier(0);
-        q[s] = 0;
-        if (in[s]) {
-          const int v = node[s];
-          q[s] = sg_apply<T, BOX>(p_lds, kk, n, kv, v % n1, (v / n1) % n1, v / (n1 * n1));
-        }
-        pq += pp[s] * q[s];
-      }
-      wg_sum2<WG>(pq, dummy, red);
+      sg_apply<T, C, BOX>(p_lds, kk, n, kv, c, [&](int s, T qs, T ps) __attribute__((always_inline)) {
+        q[s] = s < c.cnt ? qs : (T)0;
+        pq = fma(s < c.cnt ? ps : (T)0, q[s], pq);
+      });
+      wg_sum2<WG>(pq, dummy, red, buf);
       const T alpha = rz / pq;
-      T rr1 = 0, rz1 = 0;
+      T rr1 = 0, rz1 = 0, pp[C];
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
+      for (int s = 0; s < C; ++s) {
+        pp[s] = s < c.cnt ? p_lds[c.p + s * pl] : (T)0;
         x[s] += alpha * pp[s];
         r[s] -= alpha * q[s];
         rr1 += r[s] * r[s];
         rz1 += r[s] * (dinv[s] * r[s]);
       }
-      wg_sum2<WG>(rr1, rz1, red);
+      wg_sum2<WG>(rr1, rz1, red, buf);
       ++it;
       rr = rr1;
       if (!(rr > tol2 * rr0)) break;  // also leaves on NaN
       const T beta = rz1 / rz;
       rz = rz1;
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        pp[s] = dinv[s] * r[s] + beta * pp[s];
-        if (node[s] < nn) p_lds[node[s]] = pp[s];
-      }
+      for (int s = 0; s < C; ++s)
+        if (s < c.cnt) p_lds[c.p + s * pl] = dinv[s] * r[s] + beta * pp[s];
       __syncthreads();
     }
   }
@@ -262,130 +277,156 @@ __device__ __forceinline__ int sg_pcg(int n, const T* kk, const T (&kv)[8], T* p
   return it;
 }
 
-template <int WG, int S, bool MIXED, bool BOX>
+// One instance by one workgroup; C: slots of a thread, at least its run of nodes.
+template <int WG, int C, bool MIXED, bool BOX>
+__device__ __forceinline__ void sg_instance(const SgArgs& a, int id, double* p64, double* k64, double* red,
+                                            float* red32) {
+  float* p32 = reinterpret_cast<float*>(p64);  // FP32 views: p in the lower, k in the upper half of p64's storage
+  float* k32 = reinterpret_cast<float*>(p64) + kSgMaxNodes;
+  const SgInst in_ = a.inst[id];
+  const int n = in_.n, n1 = n + 1, pl = n1 * n1, nn = n1 * pl, ne = n * n * n;
+  const double* kg = a.k + in_.k_off;
+  const double* fg = a.src ? a.src + in_.k_off : nullptr;
+  const double* gg = a.g + in_.x_off;
+  double kv[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) kv[i] = in_.kv[i];
+
+  // the thread's run of nodes (idle threads: the first column, no node)
+  SgCol c{n1 + 1 + pl, 0, 0};
+  {
+    const int m = n - 1, cols = m * m, per = min(WG / cols, m), run = (m + per - 1) / per;
+    const int part = threadIdx.x / cols, col = threadIdx.x - part * cols;
+    const int cy = col / m, cx = col - cy * m, z0 = part * run;
+    if (part < per && z0 < m) {
+      c.cnt = min(run, m - z0);
+      c.p = (cx + 1) + n1 * (cy + 1) + pl * (z0 + 1);
+      c.e = cx + n * cy + n * n * z0;
+    }
+  }
+  for (int e = threadIdx.x; e < ne; e += WG) k64[e] = kg[e];
+  // u0: the Dirichlet lift (data) or 0 on the boundary nodes, 0 inside
+  auto lift = [&](bool data) {
+    for (int v = threadIdx.x; v < nn; v += WG) {
+      const int iz = v / pl, w = v - iz * pl, iy = w / n1, ix = w - iy * n1;
+      const bool bnd = ix == 0 || iy == 0 || iz == 0 || ix == n || iy == n || iz == n;
+      p64[v] = data && bnd ? gg[v] : 0.0;
+    }
+  };
+  lift(true);
+  __syncthreads();
+  // b - A u0 = -F(u0) on interior rows (assembled residual with the Dirichlet lift)
+  double r[C], x[C], dinv[C], b[BOX ? C : 1];
+#pragma unroll
+  for (int s = 0; s < C; ++s) x[s] = 0.0;
+  sg_around<C>(k64, BOX ? fg : nullptr, n, c, [&](int s, double ks, double fs) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);  // one division at a time
+    dinv[s] = s < c.cnt ? 1.0 / (kv[0] * ks) : 0.0;
+    if constexpr (BOX) b[s] = in_.vol8 * fs;
+  });
+  auto residual = [&]() __attribute__((always_inline)) {
+    sg_apply<double, C, BOX>(p64, k64, n, kv, c, [&](int s, double q, double) __attribute__((always_inline)) {
+      r[s] = s < c.cnt ? (BOX ? b[BOX ? s : 0] : 0.0) - q : 0.0;
+    });
+  };
+  residual();
+  int its = 0, refs = 0;
+  double rr = 0.0, bb = 0.0, dummy = 0.0;
+#pragma unroll
+  for (int s = 0; s < C; ++s) bb += r[s] * r[s];
+  int buf = 0;
+  wg_sum2<WG>(bb, dummy, red, buf);
+  if constexpr (!MIXED) {
+    lift(false);
+    __syncthreads();
+    its = sg_pcg<WG, C, double, BOX>(n, k64, kv, p64, red, x, r, dinv, c, a.tol, a.max_iters, rr);
+  } else {
+    // FP32 inner PCG inside FP64 iterative refinement: the residual, the
+    // accumulated correction and the convergence test stay FP64.
+    const double target2 = a.tol * a.tol * bb;
+    rr = bb;
+    while (refs < a.max_refine && rr > target2 && its < a.max_iters) {
+      const double scale = std::sqrt(rr);
+      __syncthreads();
+      for (int e = threadIdx.x; e < ne; e += WG) k32[e] = (float)k64[e];
+      for (int v = threadIdx.x; v < nn; v += WG) p32[v] = 0.f;
+      float xf[C], rf[C], df[C];
+#pragma unroll
+      for (int s = 0; s < C; ++s) {
+        xf[s] = 0.f;
+        rf[s] = (float)(r[s] / scale);
+        df[s] = (float)dinv[s];
+      }
+      __syncthreads();
+      float rrf = 0.f, kvf[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) kvf[i] = (float)kv[i];
+      its += sg_pcg<WG, C, float, BOX>(n, k32, kvf, p32, red32, xf, rf, df, c, a.inner_tol, a.max_iters - its, rrf);
+      ++refs;
+      // x += scale * xf ; r = b - A (u0 + x) in FP64
+      __syncthreads();
+      lift(true);
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < C; ++s) {
+        x[s] += scale * (double)xf[s];
+        if (s < c.cnt) p64[c.p + s * pl] = x[s];
+      }
+      __syncthreads();
+      residual();
+      double rr2 = 0.0, d2 = 0.0;
+#pragma unroll
+      for (int s = 0; s < C; ++s) rr2 += r[s] * r[s];
+      wg_sum2<WG>(rr2, d2, red, buf);
+      rr = rr2;
+    }
+  }
+  // u = u0 + du, through LDS (a thread's nodes are a plane apart)
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < C; ++s)
+    if (s < c.cnt) p64[c.p + s * pl] = x[s];
+  __syncthreads();
+  for (int v = threadIdx.x; v < nn; v += WG) {
+    const int iz = v / pl, w = v - iz * pl, iy = w / n1, ix = w - iy * n1;
+    const bool bnd = ix == 0 || iy == 0 || iz == 0 || ix == n || iy == n || iz == n;
+    a.x[in_.x_off + v] = bnd ? gg[v] : p64[v];
+  }
+  if (threadIdx.x == 0) {
+    a.iters[id] = its;
+    a.relres[id] = bb > 0.0 ? std::sqrt(rr / bb) : 0.0;
+    if (a.refinements) a.refinements[id] = refs;
+  }
+}
+
+// A thread's run of nodes: the n - 1 interior nodes of a column over as many
+// threads as the workgroup holds per column (16 elements, 225 columns: 8 at
+// 512 threads, 4 at 1024).  The sweep is built for the runs that occur, so a
+// small instance does not walk a large one's slots.
+template <int WG, bool MIXED, bool BOX>
 __global__ __launch_bounds__(WG) void k_subgrid(SgArgs a) {
   __shared__ double p64[kSgMaxNodes];
   __shared__ double k64[kSgMaxElems];
-  __shared__ double red[2 * (WG / 64)];
+  __shared__ double red[2 * 2 * (WG / 64)];
+  __shared__ float red32[MIXED ? 2 * 2 * (WG / 64) : 1];
   __shared__ int s_next;
-  float* p32 = reinterpret_cast<float*>(p64);       // FP32 views (first half of each array)
-  float* k32 = reinterpret_cast<float*>(p64) + kSgMaxNodes;  // second half of p64 storage
-  __shared__ float red32[2 * (WG / 64)];
 
   for (;;) {
     if (threadIdx.x == 0) s_next = (int)atomicAdd(a.queue, 1u);
     __syncthreads();
     // (wave-uniform: the instance's description is then read with scalar
     // loads and its stencil entries stay in scalar registers)
-    const int qpos = s_next;
+    const int qpos = __builtin_amdgcn_readfirstlane(s_next);
     __syncthreads();
     if (qpos >= a.n_inst) break;
     const int id = a.order[qpos];
-    const SgInst in_ = a.inst[id];
-    const int n = in_.n, n1 = n + 1, nn = n1 * n1 * n1, ne = n * n * n;
-    const double* kg = a.k + in_.k_off;
-    const double* fg = a.src ? a.src + in_.k_off : nullptr;
-    const double* gg = a.g + in_.x_off;
-    double kv[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) kv[i] = in_.kv[i];
-
-    for (int e = threadIdx.x; e < ne; e += WG) k64[e] = kg[e];
-    int node[S];
-    bool in[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int v = threadIdx.x + s * WG;
-      node[s] = v < nn ? v : nn;
-      const int ix = v % n1, iy = (v / n1) % n1, iz = v / (n1 * n1);
-      const bool bnd = ix == 0 || iy == 0 || iz == 0 || ix == n || iy == n || iz == n;
-      in[s] = v < nn && !bnd;
-      if (v < nn) p64[v] = bnd ? gg[v] : 0.0;  // u0: the Dirichlet lift
-    }
-    __syncthreads();
-    // b - A u0 = -F(u0) on interior rows (assembled residual with the Dirichlet lift)
-    double r[S], x[S], dinv[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      __builtin_amdgcn_sched_barrier(0);
-      x[s] = 0.0;
-      r[s] = 0.0;
-      dinv[s] = 0.0;
-      if (in[s]) {
-        const int v = node[s];
-        const int ix = v % n1, iy = (v / n1) % n1, iz = v / (n1 * n1);
-        const double b = (BOX && fg) ? in_.vol8 * sg_src(fg, n, ix, iy, iz) : 0.0;
-        r[s] = b - sg_apply<double, BOX>(p64, k64, n, kv, ix, iy, iz);
-        dinv[s] = 1.0 / sg_diag<double, BOX>(k64, n, kv[0], ix, iy, iz);
-      }
-    }
-    __syncthreads();
-    int its = 0, refs = 0;
-    double rr = 0.0, bb = 0.0, dummy = 0.0;
-#pragma unroll
-    for (int s = 0; s < S; ++s) bb += r[s] * r[s];
-    wg_sum2<WG>(bb, dummy, red);
-    if constexpr (!MIXED) {
-      its = sg_pcg<WG, S, double, BOX>(n, k64, kv, p64, red, x, r, dinv, in, node, a.tol, a.max_iters, rr);
-    } else {
-      // FP32 inner PCG inside FP64 iterative refinement: the residual, the
-      // accumulated correction and the convergence test stay FP64.
-      const double target2 = a.tol * a.tol * bb;
-      rr = bb;
-      while (refs < a.max_refine && rr > target2 && its < a.max_iters) {
-        const double scale = std::sqrt(rr);
-        // FP32 views: p32 in the lower half of p64's storage, k32 in its upper half
-        __syncthreads();
-        for (int e = threadIdx.x; e < ne; e += WG) k32[e] = (float)k64[e];
-        float xf[S], rf[S], df[S];
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          xf[s] = 0.f;
-          rf[s] = (float)(r[s] / scale);
-          df[s] = (float)dinv[s];
-        }
-        __syncthreads();
-        float rrf = 0.f, kvf[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) kvf[i] = (float)kv[i];
-        its += sg_pcg<WG, S, float, BOX>(n, k32, kvf, p32, red32, xf, rf, df, in, node, a.inner_tol, a.max_iters - its, rrf);
-        ++refs;
-        // x += scale * xf ; r = b - A (u0 + x) in FP64
-        __syncthreads();
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          x[s] += scale * (double)xf[s];
-          const int v = node[s];
-          if (v < nn) p64[v] = (in[s] ? 0.0 : gg[v]) + x[s];
-        }
-        __syncthreads();
-        double rr2 = 0.0, d2 = 0.0;
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          __builtin_amdgcn_sched_barrier(0);
-          if (in[s]) {
-            const int v = node[s];
-            const int ix = v % n1, iy = (v / n1) % n1, iz = v / (n1 * n1);
-            const double b = (BOX && fg) ? in_.vol8 * sg_src(fg, n, ix, iy, iz) : 0.0;
-            r[s] = b - sg_apply<double, BOX>(p64, k64, n, kv, ix, iy, iz);
-          }
-          rr2 += r[s] * r[s];
-        }
-        wg_sum2<WG>(rr2, d2, red);
-        rr = rr2;
-      }
-    }
-    // u = u0 + du
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const int v = node[s];
-      if (v < nn) a.x[in_.x_off + v] = (in[s] ? 0.0 : gg[v]) + x[s];
-    }
-    if (threadIdx.x == 0) {
-      a.iters[id] = its;
-      a.relres[id] = bb > 0.0 ? std::sqrt(rr / bb) : 0.0;
-      if (a.refinements) a.refinements[id] = refs;
-    }
+    const int m = a.inst[id].n - 1, per = min(WG / (m * m), m), run = (m + per - 1) / per;
+    if (run == 1) sg_instance<WG, 1, MIXED, BOX>(a, id, p64, k64, red, red32);
+    else if (run == 2) sg_instance<WG, 2, MIXED, BOX>(a, id, p64, k64, red, red32);
+    else if (run == 3) sg_instance<WG, 3, MIXED, BOX>(a, id, p64, k64, red, red32);
+    else if (WG == 1024 || run == 4) sg_instance<WG, 4, MIXED, BOX>(a, id, p64, k64, red, red32);
+    else if (run == 5) sg_instance<WG, WG == 1024 ? 4 : 5, MIXED, BOX>(a, id, p64, k64, red, red32);
+    else sg_instance<WG, WG == 1024 ? 4 : 8, MIXED, BOX>(a, id, p64, k64, red, red32);
     __syncthreads();
   }
 }
@@ -447,19 +488,14 @@ static SgArgs make_args(Batch& b) {
 static void enqueue(Batch& b, int wg) {
   SgArgs a = make_args(b);
   hipLaunchKernelGGL(k_sg_reset, dim3(1), dim3(1), 0, b.stream, b.queue.p);
-  constexpr int S1024 = (kSgMaxNodes + 1023) / 1024, S512 = (kSgMaxNodes + 511) / 512;
   auto go = [&](auto BX) {
     constexpr bool X = decltype(BX)::value;
     if (wg == 1024) {
-      if (a.fp32)
-        hipLaunchKernelGGL((k_subgrid<1024, S1024, true, X>), dim3(b.grid[1]), dim3(1024), 0, b.stream, a);
-      else
-        hipLaunchKernelGGL((k_subgrid<1024, S1024, false, X>), dim3(b.grid[1]), dim3(1024), 0, b.stream, a);
+      if (a.fp32) hipLaunchKernelGGL((k_subgrid<1024, true, X>), dim3(b.grid[1]), dim3(1024), 0, b.stream, a);
+      else hipLaunchKernelGGL((k_subgrid<1024, false, X>), dim3(b.grid[1]), dim3(1024), 0, b.stream, a);
     } else {
-      if (a.fp32)
-        hipLaunchKernelGGL((k_subgrid<512, S512, true, X>), dim3(b.grid[0]), dim3(512), 0, b.stream, a);
-      else
-        hipLaunchKernelGGL((k_subgrid<512, S512, false, X>), dim3(b.grid[0]), dim3(512), 0, b.stream, a);
+      if (a.fp32) hipLaunchKernelGGL((k_subgrid<512, true, X>), dim3(b.grid[0]), dim3(512), 0, b.stream, a);
+      else hipLaunchKernelGGL((k_subgrid<512, false, X>), dim3(b.grid[0]), dim3(512), 0, b.stream, a);
     }
   };
   if (b.box) go(std::true_type{});
@@ -506,10 +542,16 @@ static void setup_grid(Batch& b) {
   MHX_HIP(hipGetDevice(&dev));
   MHX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   int occ512 = 0, occ1024 = 0;
-  MHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &occ512, (const void*)k_subgrid<512, (kSgMaxNodes + 511) / 512, false, false>, 512, 0));
-  MHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &occ1024, (const void*)k_subgrid<1024, (kSgMaxNodes + 1023) / 1024, false, false>, 1024, 0));
+  auto occ = [&](auto MX, auto BX) {
+    constexpr bool M = decltype(MX)::value, X = decltype(BX)::value;
+    MHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ512, (const void*)k_subgrid<512, M, X>, 512, 0));
+    MHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ1024, (const void*)k_subgrid<1024, M, X>, 1024, 0));
+  };
+  const bool mixed = b.desc.precision == MHX_BATCH_FP32_REFINED;
+  if (mixed && b.box) occ(std::true_type{}, std::true_type{});
+  else if (mixed) occ(std::true_type{}, std::false_type{});
+  else if (b.box) occ(std::false_type{}, std::true_type{});
+  else occ(std::false_type{}, std::false_type{});
   MHX_REQUIRE(occ512 > 0 && occ1024 > 0, MHX_ERR_DEVICE, "subgrid kernel does not fit on a CU");
   b.grid[0] = std::max(1, std::min(b.n_inst, cus * occ512));
   b.grid[1] = std::max(1, std::min(b.n_inst, cus * occ1024));

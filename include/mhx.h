@@ -377,17 +377,24 @@ int  mhx_l2_error(mhx_ctx* ctx, const double* u, int32_t n_modes, const double* 
  *                         row's share as contiguous runs; Navier-Stokes:
  *                         segments of 8 (3-D) / 16 (2-D) elements; block
  *                         colouring runs element colouring there),
- *                         3 = pencil streaming (a wavefront walks an
- *                         x-segment of an element pencil two elements per
- *                         step and writes each row's x-run once; 3-D Q2
+ *                         3 = pencil streaming (one launch: a workgroup
+ *                         owns the rows of 2 x 2 element pencils, walks an
+ *                         x-segment and writes each row once; 3-D Q2
  *                         thermal with 3x3x3 Gauss on an unperturbed box
  *                         mesh only, MHX_ERR_ARG elsewhere).  Default: 3
- *                         where it applies, 2 for Navier-Stokes, else 0.
+ *                         where it applies, 2 for Navier-Stokes, else 0;
+ *                         while 0 is the default and not set, small
+ *                         thermal meshes (element matrices up to 24 MiB,
+ *                         3-D 80 MiB, order 1 128 MiB) are assembled in two
+ *                         launches: element matrices, then a sum per row.
  *   "assembly.segment"    pencil streaming: elements per x-segment, even,
- *                         2 .. 4096 (default 12).
+ *                         2 .. 4096 (default: from the mesh, so that the
+ *                         workgroups fill the device evenly).
  *   "krylov.spmv_lanes"   lanes that share one CRS row in the sparse
  *                         matrix-vector product: 4, 8, 16, 32 or 64 (default
- *                         chosen from the mean row length at context build).
+ *                         chosen from the mean row length at context build;
+ *                         at the default, order-2 scalar patterns run the
+ *                         product made for them).
  *   "krylov.lattice_columns"  1 (default): sparse products on the
  *                         context's lattice pattern compute each entry's
  *                         column from the pattern's closed form instead of

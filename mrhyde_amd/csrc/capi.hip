@@ -348,16 +348,7 @@ using namespace mhx;
 
 struct mhx_ctx : public Ctx {};
 
-extern "C" {
-
-const char* mhx_version(void) { return "mhx 0.1 (gfx950, fp64 assembly, sum-factorised AD columns)"; }
-
-const char* mhx_last_error(const mhx_ctx* ctx) {
-  if (ctx && !ctx->err.empty()) return ctx->err.c_str();
-  return g_last_error.c_str();
-}
-
-int mhx_ctx_create(const mhx_problem_desc* desc, mhx_ctx** out) {
+int mhx::ctx_create(const mhx_problem_desc* desc, bool element_store, mhx_ctx** out) {
   mhx_ctx* c = nullptr;
   MHX_GUARD_BEGIN
   MHX_REQUIRE(out, MHX_ERR_ARG, "null output pointer");
@@ -383,6 +374,17 @@ int mhx_ctx_create(const mhx_problem_desc* desc, mhx_ctx** out) {
   // thermal assembly then defaults to the pencil-streamed kernel
   c->box_mesh = desc->perturb == 0.0;
   if (q2box_applicable(*c)) c->scatter_mode = kPencilStream;
+  // small general meshes: element matrices to scratch (now, so that no
+  // assembly allocates), rows gathered
+  if (const int64_t ed = element_store ? element_store_doubles(*desc) : 0) {
+    try {
+      c->rscr.alloc((size_t)c->mesh.ne * c->nb);
+      c->escr.alloc((size_t)ed);
+    } catch (const Error&) {  // no room: element colouring
+      (void)hipGetLastError();
+      c->rscr.release();
+    }
+  }
   // Navier-Stokes: x-segments merged in LDS (each row's x-runs written once
   // per segment) by default
   if (desc->physics == MHX_PHYS_NAVIER_STOKES) c->scatter_mode = kSegmentMerge;
@@ -403,6 +405,17 @@ int mhx_ctx_create(const mhx_problem_desc* desc, mhx_ctx** out) {
     return e.code;
   }
 }
+
+extern "C" {
+
+const char* mhx_version(void) { return "mhx 0.1 (gfx950, fp64 assembly, sum-factorised AD columns)"; }
+
+const char* mhx_last_error(const mhx_ctx* ctx) {
+  if (ctx && !ctx->err.empty()) return ctx->err.c_str();
+  return g_last_error.c_str();
+}
+
+int mhx_ctx_create(const mhx_problem_desc* desc, mhx_ctx** out) { return ctx_create(desc, true, out); }
 
 void mhx_ctx_destroy(mhx_ctx* ctx) {
   if (!ctx) return;
@@ -896,6 +909,8 @@ int mhx_footprint(const mhx_problem_desc* d, const mhx_krylov_opts* opts, int64_
     const int64_t fine = 8 * 27 * N * nf + 2 * 12 * 8 * N * nf + 8 * 7 * N;
     bytes += fine + fine / 8;
   }
+  // element matrices and residuals of the two-launch assembly
+  bytes += element_store_bytes(*d);
   if (n_dof) *n_dof = N;
   if (nnz) *nnz = Z;
   if (device_bytes) *device_bytes = bytes;
@@ -978,6 +993,7 @@ int mhx_set_option(mhx_ctx* ctx, const char* name, int64_t value) {
       return MHX_ERR_ARG;
     }
     ctx->scatter_mode = (int)value;
+    ctx->scatter_auto = false;
     return MHX_OK;
   }
   if (k == "assembly.segment") {

@@ -64,6 +64,19 @@ __device__ __forceinline__ bool element_of(const AsmArgs& a, int g, int sub, int
   return ok && g < a.gpb;
 }
 
+// Element store: elements in lexicographic order, one per group.
+template <int DIM>
+__device__ __forceinline__ bool element_linear(const AsmArgs& a, int g, int* ec) {
+  const unsigned idx = blockIdx.x * (unsigned)a.gpb + (unsigned)g;
+  const bool in = idx < (unsigned)a.m.ne;
+  unsigned t = in ? idx : 0u;
+  ec[0] = (int)(t % (unsigned)a.m.nel[0]);
+  t /= (unsigned)a.m.nel[0];
+  ec[1] = (int)(t % (unsigned)a.m.nel[1]);
+  ec[2] = DIM == 3 ? (int)(t / (unsigned)a.m.nel[1]) : 0;
+  return in;
+}
+
 // Segment scheduling (a.blocked == 2): a workgroup owns a segment of a.gpb
 // x-consecutive elements at one (ey, ez); group g takes the segment's g-th
 // element.  One launch per colour of (segment parity, ey parity, ez parity):

@@ -97,6 +97,8 @@ struct AsmArgs {
   double alpha_u;         // A_ss / b_s
   double rho_cp;          // density * specific heat
   ExprSet xp;             // compiled coefficient functions (xp.active = 0: the closed forms)
+  double* escr;           // element store: [ne][row][column] element matrices
+  double* rscr;           // element store: [ne][row] element residuals
 };
 
 // compiled coefficient functions of a context, host side (expr.hip)
@@ -110,7 +112,8 @@ struct ExprHost {
 };
 void expr_compile(const mhx_problem_desc& d, ExprHost& out);
 
-enum ScatterMode { kElementColouring = 0, kBlockColouring = 1, kSegmentMerge = 2, kPencilStream = 3 };
+enum ScatterMode { kElementColouring = 0, kBlockColouring = 1, kSegmentMerge = 2, kPencilStream = 3,
+                   kElementStore = 4 /* element matrices to scratch, rows gathered (not an option value) */ };
 
 // ---------------------------------------------------------------------------
 // device buffers
@@ -234,6 +237,8 @@ struct Ctx {
   int amg_omega_pct = 40;  // block-Jacobi smoother: damping in percent
   int nfield = 1;  // unknowns per node (consecutive DOFs): block size of block Jacobi
   int scatter_mode = kElementColouring;
+  bool scatter_auto = true;   // assembly.colouring not set by the caller
+  DevBuf<double> escr, rscr;  // element matrices and residuals (allocated where the element store applies)
   bool box_mesh = false;  // every element an axis-aligned box (structured box, no node perturbation)
   int q2_segment = 0;     // pencil streaming: elements per x-segment (even; 0: chosen per launch)
   std::shared_ptr<Amg> amg;  // built by a solve with the AMG preconditioner, kept for reuse of its buffers
@@ -261,6 +266,14 @@ bool thermal_supported(int dim, int p, int nq1);
 bool q2box_applicable(const Ctx& c);
 void launch_q2box(Ctx& c, AsmArgs& a, bool jac);
 int q2box_segment(const Ctx& c, bool jac);  // elements per x-segment of a launch
+// element store (assemble_elem.hip): doubles of element matrices where the
+// two-launch assembly applies to the description, else 0; the bytes with the
+// residuals; and its launches
+int64_t element_store_doubles(const mhx_problem_desc& d);
+int64_t element_store_bytes(const mhx_problem_desc& d);
+// mhx_ctx_create; element_store = false leaves its scratch memory out
+int ctx_create(const mhx_problem_desc* desc, bool element_store, mhx_ctx** out);
+void launch_element_store(Ctx& c, AsmArgs& a, bool jac);
 // thermal assembly with compiled coefficient functions, element colouring
 // (assemble_expr.hip)
 void launch_thermal_expr(Ctx& c, AsmArgs& a, bool jac);

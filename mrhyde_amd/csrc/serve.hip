@@ -64,6 +64,7 @@ struct Request {
   std::vector<const char*> fn_name_p, fn_expr_p;
   Key key;
   int64_t n_dof = 0, bytes = 0;
+  bool element_store = true;  // the context gets the scratch memory of the two-launch assembly
   clk::time_point t_submit, t_start, t_end;
   bool done = false;
   int status = MHX_OK;
@@ -128,7 +129,7 @@ struct mhx_server {
   void run(Request* r, Slot& slot) {
     int rc = MHX_OK;
     if (!slot.ctx) {
-      rc = mhx_ctx_create(&r->desc, &slot.ctx);
+      rc = ctx_create(&r->desc, r->element_store, &slot.ctx);
       if (rc == MHX_OK) {
         std::lock_guard<std::mutex> lk(mu);
         ++n_created;
@@ -230,6 +231,10 @@ int mhx_server_submit(mhx_server* s, const mhx_problem_desc* desc, int64_t* tick
   int64_t nnz = 0;
   int rc = mhx_footprint(desc, &s->d.newton.linear, &r->n_dof, &nnz, &r->bytes);
   if (rc != MHX_OK) return rc;
+  if (r->bytes > s->d.hbm_budget) {  // do without the optional scratch memory (same results)
+    r->element_store = false;
+    r->bytes -= element_store_bytes(*desc);
+  }
   if (r->bytes > s->d.hbm_budget) return MHX_ERR_NOMEM;  // could never be admitted
   r->desc = *desc;
   long ne = (long)desc->nx * desc->ny * (desc->dim == 3 ? desc->nz : 1);

@@ -143,6 +143,7 @@ __global__ __launch_bounds__(256) void k_thermal(AsmArgs a) {
   constexpr int NB = C::NB, NQ = C::NQ, NV = C::NV, NC = C::NC, G = C::G, GPB = C::GPB, P1 = C::P1;
   constexpr bool BLOCKED = MODE == kBlockColouring;
   constexpr bool SEG = MODE == kSegmentMerge;
+  constexpr bool STORE = MODE == kElementStore;
   using SG = SegCfg<DIM, P, GPB>;
   __shared__ double s_seg[SEG && JAC ? SG::kSize : 1];
   __shared__ double s_sres[SEG ? SG::kRows : 1];
@@ -167,7 +168,9 @@ __global__ __launch_bounds__(256) void k_thermal(AsmArgs a) {
   if (sub) __syncthreads();  // previous sub-phase's LDS reads and global stores are complete
   int ec[3];
   int sx = 0, s_act = 0;
-  const bool active = SEG ? element_of_seg<DIM>(a, g, ec, sx, s_act) : element_of<DIM>(a, g, sub, ec);
+  const bool active = SEG     ? element_of_seg<DIM>(a, g, ec, sx, s_act)
+                      : STORE ? element_linear<DIM>(a, g, ec)
+                              : element_of<DIM>(a, g, sub, ec);
   const long e = ec[0] + (long)a.m.nel[0] * (ec[1] + (long)a.m.nel[1] * ec[2]);
   // first-touch flags per axis: is this element (segment, along x in segment
   // scheduling) the first scheduled one among the (at most two) sharing its
@@ -498,7 +501,24 @@ __global__ __launch_bounds__(256) void k_thermal(AsmArgs a) {
   }
   __syncthreads();  // all reads of s_u done before it is reused
 
-  if constexpr (SEG) {
+  if constexpr (STORE) {
+    // 4''. element store: lane j writes column j (for a fixed row the lanes
+    // write consecutive values); k_gather_rows sums them into the CRS rows
+    if constexpr (JAC) {
+      if (active && lane < NB && a.jac) {
+        double* E = a.escr + e * (NB * NB) + lane;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) E[i * NB] = R[i];
+      } else if (active && lane == NB && a.res) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) s_u[g][i] = R[i];
+      }
+      __syncthreads();
+      if (active && lane < NB && a.res) a.rscr[e * NB + lane] = s_u[g][lane];
+    } else {
+      if (active && lane < NB) a.rscr[e * NB + lane] = R[0];
+    }
+  } else if constexpr (SEG) {
     // 4'. segment scatter: the segment's element columns are summed into an
     // LDS image of its rows (groups of even, then odd index, so the two
     // elements sharing a vertex plane never write at once), then the

@@ -1,0 +1,67 @@
+"""Assembly through element matrices in scratch memory and a gather per row
+(the default of small general thermal meshes) against element colouring on the
+same problem: meshes of one element and up, odd counts, every order and rule,
+Dirichlet rows on some and all sides, perturbed and box elements, residual
+alone, accumulation, and sizes on both sides of the rule's bound.
+
+Tolerance: the two sum at most 2^dim <= 8 element terms, and their kernels may
+contract differently over NQ <= 64 points: (8 + 64) eps times the largest
+magnitude, rounded up to 4e-14."""
+import numpy as np
+import pytest
+
+from mrhyde_amd import Problem
+
+pytestmark = pytest.mark.gpu
+
+CASES = [(1, 2, (1, 1), 0.0, 15), (1, 0, (5, 3), 0.0, 1), (1, 4, (17, 9), 0.1, 3), (2, 2, (3, 1), 0.0, 2),
+         (2, 4, (9, 14), 0.1, 15), (2, 6, (2, 2), 0.0, 4), (3, 6, (5, 4), 0.1, 8), (4, 8, (3, 2), 0.0, 1),
+         (5, 10, (2, 3), 0.0, 15), (6, 12, (1, 2), 0.0, 3), (1, 0, (3, 2, 1), 0.0, 3), (1, 2, (1, 1, 1), 0.0, 0),
+         (1, 2, (9, 7, 5), 0.1, 63), (1, 4, (4, 3, 2), 0.0, 16), (2, 2, (2, 3, 4), 0.0, 32), (2, 4, (1, 1, 1), 0.1, 3),
+         (2, 4, (5, 4, 3), 0.1, 63), (2, 6, (2, 1, 3), 0.0, 3), (2, 4, (193, 121), 0.0, 3), (2, 4, (25, 24, 24), 0.1, 3)]
+
+
+@pytest.mark.parametrize("order,quad,n,perturb,dbc", CASES,
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_matches_colouring(order, quad, n, perturb, dbc):
+    from mrhyde_amd import Mhx
+
+    print(f"[element store] p{order} q{quad} {n}", flush=True)
+    rng = np.random.default_rng(order + quad + sum(n))
+    ne = int(np.prod(n))
+    p = Problem(dim=len(n), order=order, quadrature=quad, n=n, k0=np.exp(rng.standard_normal(ne)), diff_u2=0.7,
+                src_elem=rng.standard_normal(ne), modes=[(1.3, (2.0, 0.0, 3.0)[:len(n)])], dbc_sides=dbc, dbc_const=0.3,
+                perturb=perturb)
+    g, c = Mhx(p), Mhx(p)
+    c.set_option("assembly.colouring", 0)
+    assert g.get_option("assembly.colouring") == 0
+    u = rng.standard_normal(g.n_dof)
+    rc, jc = c.assembleJacRes(u)
+    tol_r, tol_j = 4e-14 * np.abs(rc).max(), 4e-14 * np.abs(jc).max()
+    r, j = g.assembleJacRes(u)
+    r2, j2 = g.assembleJacRes(u)
+    np.testing.assert_array_equal(j, j2)
+    np.testing.assert_array_equal(r, r2)
+    assert np.abs(r - rc).max() <= tol_r and np.abs(j - jc).max() <= tol_j
+    assert np.abs(g.assembleRes(u) - rc).max() <= tol_r
+    r0, j0 = rng.standard_normal(g.n_dof), rng.standard_normal(g.nnz)
+    ra, ja = g.assemble(u, r0.copy(), j0.copy(), accumulate=True)
+    rb, jb = c.assemble(u, r0.copy(), j0.copy(), accumulate=True)
+    assert np.abs(ra - rb).max() <= tol_r + 4e-14 * np.abs(r0).max()
+    assert np.abs(ja - jb).max() <= tol_j + 4e-14 * np.abs(j0).max()
+    g.close(), c.close()
+
+
+def test_server_budget_without_scratch():
+    """A budget that holds a request only without the scratch memory still
+    admits it, with the same bits."""
+    from mrhyde_amd import Server
+
+    p = Problem(dim=3, order=1, quadrature=2, n=(12, 11, 10), modes=[(1.0, (np.pi, np.pi, np.pi))], diff_u2=0.5)
+    need = Server.footprint(p)[2]
+    xs = []
+    for budget in (need, need - 8 * 64 * p.n_elem):
+        s = Server(max_active=1, max_cached=1, hbm_budget=budget)
+        xs.append(s.poll(s.submit(p))[0])
+        s.close()
+    np.testing.assert_array_equal(xs[0], xs[1])

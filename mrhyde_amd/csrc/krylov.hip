@@ -14,6 +14,7 @@
 // x += ||r|| d and the stopping test are FP64 with the FP64 Jacobian.
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <mutex>
 #include <type_traits>
@@ -498,7 +499,8 @@ static void op_apply(Ctx& c, const T* A, const Prec<T>& P, const T* v, T* w, T* 
 // forms p at the gathered columns (z + beta p_old, both in cache) into the other
 // of two p vectors.  With a launch per step of the recurrence and per reduction
 // (nine) an iteration of the 64^2 Q1 problem took 25-29 us, nearly all latency;
-// now 13 us (a whole Newton solve of it 11.2 -> 5.3 ms).
+// now 13 us (a whole Newton solve of it 11.2 -> 5.3 ms); k_cg_wg below takes the
+// smallest ones in a single workgroup.
 // Larger systems keep the product apart, with the final reductions still folded
 // into their readers (four launches).
 // The CG scalars stay on the device: rho (two slots, alternating by
@@ -676,12 +678,200 @@ __global__ __launch_bounds__(256) void k_cg_update(long n, const double* __restr
   }
 }
 
+// One-workgroup CG for the smallest systems.  What bounds the two-launch form
+// there is the launches (13 us an iteration however small the system); here one
+// workgroup of 16 wavefronts runs the iterations in a loop, with barriers in
+// place of launches.  A thread owns rows t, t + 1024, ...: x, r and D^-1 stay in
+// its registers, p is in LDS together with each entry's 16-bit LDS offset of p
+// (two entries to a word), and only the matrix values are read again, from a
+// copy with the rows' k-th entries side by side (L2, 340 KB at 64^2 Q1), one
+// chunk ahead.  Rows are padded with zeros to a multiple of kCgWgChunk entries.
+// 64^2 Q1: 8 us an iteration, most of it that stream through one CU; a whole
+// Newton solve 5.1 -> 3.3 ms.  With the CRS rows dealt to four lanes each an
+// iteration took 11 us, without the chunk ahead 8.6.
+// The two sums per iteration meet in LDS (four 16-lane rows a wavefront) and are
+// added in the same order by every thread, so all agree on each branch.
+constexpr int kCgWgRows = 5;          // rows a thread can own
+constexpr int kCgWgChunk = 10;        // entries loaded together
+constexpr int kCgWgLds = 150 * 1024;  // p and the offsets
+constexpr int kCgWgIters = 512;       // iterations a launch runs at most
+
+__device__ __forceinline__ double row16_sum(double v) {
+  v += dpp_move<kDppXor1>(v);
+  v += dpp_move<kDppXor2>(v);
+  v += dpp_move<kDppHalfMirror>(v);
+  return v + dpp_move<0x140>(v);  // row mirror
+}
+// sums of a and b over the workgroup, in every thread; sh: 2 x 64 doubles that
+// no thread reads any more
+__device__ __forceinline__ void wg1024_sum2(double& a, double& b, double* sh) {
+  a = row16_sum(a);
+  b = row16_sum(b);
+  const int t = threadIdx.x;
+  if (t % 16 == 0) sh[t / 16] = a, sh[64 + t / 16] = b;
+  __syncthreads();
+  const double* s = sh + 4 * (t % 16);
+  a = row16_sum((s[0] + s[1]) + (s[2] + s[3]));
+  b = row16_sum((s[64] + s[65]) + (s[66] + s[67]));
+}
+
+// entry k of each row to E[k][row], zero past the row's end
+template <class T>
+__global__ void k_cg_ell(int n, int W, const int32_t* __restrict__ rp, const T* __restrict__ A, T* __restrict__ E) {
+  const int row = blockIdx.x * 256 + threadIdx.x;
+  if (row >= n) return;
+  const int b = rp[row], len = rp[row + 1] - b;
+  for (int k = blockIdx.y; k < W; k += gridDim.y) E[k * n + row] = k < len ? A[b + k] : (T)0;
+}
+
+// Up to `iters` iterations; stops at the end of a window of 16 (the host's
+// window in the other forms) in which ||r|| / bn <= tol or is not finite.
+// out: iterations up to and with that one (or all), its ||r||.  p and rho_old
+// (cgs) are kept for the next launch.
+template <class T>
+__global__ __launch_bounds__(1024) void k_cg_wg(int n, int W, const int32_t* __restrict__ rp,
+                                                const int32_t* __restrict__ colidx, const T* __restrict__ E,
+                                                const T* __restrict__ minv, T* __restrict__ x, T* __restrict__ r,
+                                                T* __restrict__ p, double* __restrict__ cgs, int first, int iters,
+                                                double bn, double tol, double* __restrict__ out) {
+  constexpr int R = kCgWgRows, C = kCgWgChunk;
+  __shared__ __align__(16) unsigned char lds[kCgWgLds];
+  __shared__ __align__(16) double s_sum[2][128];
+  uint32_t* s_ci = (uint32_t*)lds;                              // [W / 2][n]
+  unsigned char* s_pb = lds + 4 * (size_t)(W / 2) * n + (W / 2 * n % 2) * 4;  // p, 8-byte aligned
+  T* s_p = (T*)s_pb;
+  const int t = threadIdx.x;
+  for (int row = t; row < n; row += 1024) {
+    const int b = rp[row], e = rp[row + 1];
+    for (int k = 0; k < W; k += 2) {
+      const unsigned c0 = b + k < e ? colidx[b + k] : row, c1 = b + k + 1 < e ? colidx[b + k + 1] : row;
+      s_ci[k / 2 * n + row] = (c0 | c1 << 16) * (unsigned)sizeof(T);
+    }
+  }
+  T xv[R], rv[R], mv[R];
+  double rz = 0.0, rr = 0.0, ro = first ? 0.0 : cgs[kCgRho];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int row = i * 1024 + t;
+    xv[i] = rv[i] = mv[i] = 0;
+    if (row < n) {
+      xv[i] = x[row], rv[i] = r[row];
+      mv[i] = minv ? minv[row] : (T)1;
+      if (!first) s_p[row] = p[row];
+      rz = fma((double)rv[i], (double)(mv[i] * rv[i]), rz);
+    }
+  }
+  // (opaque, so that addresses are not carried through the iterations: registers)
+  auto own_row = [&](int i) __attribute__((always_inline)) {
+    unsigned row = min(i * 1024 + t, n - 1);
+    asm volatile("" : "+v"(row));
+    return row;
+  };
+  T nx[C];
+  auto load = [&](unsigned row, int k) __attribute__((always_inline)) {
+    const T* Ek = E + (long)k * n;
+#pragma unroll
+    for (int j = 0; j < C; ++j) nx[j] = Ek[j * n + row];
+  };
+  load(own_row(0), 0);
+  wg1024_sum2(rz, rr, s_sum[0]);
+  int it = 0, conv = 0;
+  double rc = 0.0, rn = 0.0;
+  for (;;) {
+    // p = z + beta p (first: p = z)
+    const double beta = ro != 0.0 ? rz / ro : 0.0;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int row = i * 1024 + t;
+      if (row < n) {
+        const T z = mv[i] * rv[i];
+        s_p[row] = first ? z : (T)fma(beta, (double)s_p[row], (double)z);
+      }
+    }
+    first = 0;
+    __syncthreads();
+    // q = A p
+    T q[R];
+    double pq = 0.0, zero = 0.0;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      q[i] = 0;
+      if (i * 1024 < n) {
+        const unsigned row = own_row(i);
+        const uint32_t* ck = s_ci + row;
+        for (int k = 0; k < W; k += C, ck += C / 2 * n) {
+          T a[C];
+          uint32_t o[C / 2];
+#pragma unroll
+          for (int j = 0; j < C; ++j) a[j] = nx[j];
+          // the next entries' values, one step ahead (past the end: the first
+          // ones, for the next iteration)
+          const bool same = k + C < W;
+          const int in = same ? i : (i + 1) * 1024 < n ? i + 1 : 0;
+          load(own_row(in), same ? k + C : 0);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < C / 2; ++j) o[j] = ck[j * n];
+#pragma unroll
+          for (int j = 0; j < C / 2; ++j) {
+            q[i] = fma(a[2 * j], *(const T*)(s_pb + (o[j] & 0xffff)), q[i]);
+            q[i] = fma(a[2 * j + 1], *(const T*)(s_pb + (o[j] >> 16)), q[i]);
+          }
+        }
+        if (i * 1024 + t < n) pq = fma((double)s_p[row], (double)q[i], pq);
+      }
+    }
+    wg1024_sum2(pq, zero, s_sum[1]);
+    const T al = (T)(pq != 0.0 ? rz / pq : 0.0);
+    ro = rz;
+    rz = rr = 0.0;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int row = i * 1024 + t;
+      if (row < n) {
+        xv[i] = fma(al, s_p[row], xv[i]);
+        rv[i] = fma(-al, q[i], rv[i]);
+        rr = fma((double)rv[i], (double)rv[i], rr);
+        rz = fma((double)rv[i], (double)(mv[i] * rv[i]), rz);
+      }
+    }
+    wg1024_sum2(rr, rz, s_sum[0]);
+    ++it;
+    rn = sqrt(rr);
+    if (!conv && (!(rn <= DBL_MAX) || rn / bn <= tol)) conv = it, rc = rn;
+    if (it >= iters || (conv && it % 16 == 0)) break;
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int row = i * 1024 + t;
+    if (row < n) x[row] = xv[i], r[row] = rv[i], p[row] = s_p[row];
+  }
+  if (t == 0) {
+    cgs[kCgRho] = ro;
+    out[0] = conv ? conv : it;
+    out[1] = conv ? rc : rn;
+  }
+}
+
+// The one-workgroup form takes the systems whose p and offsets fit its LDS (2-D
+// Q1 to 70^2, 3-D Q1 to 12^3), without a preconditioner or with the diagonal
+// one.  Row length of its copy of the matrix, 0 where it does not apply.
+template <class T>
+static int cg_one_workgroup(const Ctx& c, int precond, long n) {
+  if ((precond != MHX_PREC_NONE && precond != MHX_PREC_JACOBI) || n > 1024 * kCgWgRows) return 0;
+  long W = c.mesh.nf;
+  for (int d = 0; d < c.mesh.dim; ++d) W *= std::min(2 * c.mesh.p, c.mesh.p * c.mesh.nel[d]) + 1;
+  W = (W + kCgWgChunk - 1) / kCgWgChunk * kCgWgChunk;
+  return ((long)sizeof(T) + 2 * W) * n + 8 <= kCgWgLds ? (int)W : 0;
+}
+
 // Device storage of one CG solve: the Krylov vectors (two directions for the
 // small systems' two-launch iteration), kCgParts x kRedBlocks reduction
 // partials, the CG scalars and one reduction slot.
 template <class T>
 struct CgBufs {
   T *r, *z, *p, *p2, *q;
+  T* ell;  // one-workgroup form: its copy of the matrix
   double *part, *cgs, *slot;
 };
 
@@ -752,7 +942,23 @@ static int cg_run(Ctx& c, const T* A, const Prec<T>& P, const T* b, T* x, double
   int it = 0;
   double hist[kMaxW];
   Profiler off;
-  if (!cycle) precondition();
+  if (const int Wr = cg_one_workgroup<T>(c, P.kind, n)) {
+    hipLaunchKernelGGL(k_cg_ell<T>, dim3((unsigned)((n + 255) / 256), kCgWgChunk), dim3(256), 0, c.stream, (int)n, Wr,
+                       c.rowptr.p, A, v.ell);
+    for (int first = 1; it < maxit && rn / bn > tol; first = 0) {
+      ScopedPhase ph(timers ? c.prof : off, "Krylov::cg_window", c.stream);
+      hipLaunchKernelGGL(k_cg_wg<T>, dim3(1), dim3(1024), 0, c.stream, (int)n, Wr, c.rowptr.p, c.colidx.p, v.ell, minv,
+                         x, v.r, v.p, cgs, first, std::min(kCgWgIters, maxit - it), bn, tol, cgs + kCgHist);
+      MHX_HIP(hipGetLastError());
+      MHX_HIP(hipMemcpyAsync(hist, cgs + kCgHist, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+      MHX_HIP(hipStreamSynchronize(c.stream));
+      it += (int)hist[0];
+      rn = hist[1];
+      if (!std::isfinite(rn)) throw Error{MHX_ERR_NONFINITE, "CG: non-finite residual"};
+    }
+  } else if (!cycle) {
+    precondition();
+  }
   while (it < maxit && rn / bn > tol) {
     const int w = std::min(W, maxit - it);
     {
@@ -792,7 +998,8 @@ static int cg_core(Ctx& c, const T* A, const Prec<T>& P, const T* b, T* x, doubl
   if (cg_two_launch(c, n)) v.tmp.alloc(n);
   ensure_red(c, kCgParts);
   if (c.kw.cgs.n < (size_t)(kCgHist + 16)) c.kw.cgs.alloc(kCgHist + 16);
-  const CgBufs<T> bufs{v.r.p, v.z.p, v.p.p, v.tmp.p, v.q.p, c.kw.part.p, c.kw.cgs.p, c.kw.scal.p + kScalN};
+  if (const int W = cg_one_workgroup<T>(c, P.kind, n)) v.ell.alloc((size_t)W * n);
+  const CgBufs<T> bufs{v.r.p, v.z.p, v.p.p, v.tmp.p, v.q.p, v.ell.p, c.kw.part.p, c.kw.cgs.p, c.kw.scal.p + kScalN};
   return cg_run<T>(c, A, P, b, x, tol, maxit, relres, bufs, true);
 }
 
@@ -1193,7 +1400,9 @@ int krylov_solve_noalloc(Ctx& c, const double* A, const double* b, double* x, co
   const long N = MHX_NOALLOC_MAX_DOF;
   // (the second direction vector of small systems: the free half of p's array)
   double* tail = s + 5 * N + kCgParts * kRedBlocks;
-  CgBufs<double> v{s, s + N, s + 2 * N, s + 2 * N + N / 2, s + 3 * N, s + 5 * N, tail, tail + 128};
+  // (z's array, which the one-workgroup form does not use, for its matrix:
+  // at most 77,000 entries)
+  CgBufs<double> v{s, s + N, s + 2 * N, s + 2 * N + N / 2, s + 3 * N, s + N, s + 5 * N, tail, tail + 128};
   MHX_REQUIRE(!cg_two_launch(c, n) || n <= N / 2, MHX_ERR_STATE, "allocation-free solve: no room for the second direction");
   double* minv = s + 4 * N;
   // the array keeps the last call's contents: the CG scalars start cleared

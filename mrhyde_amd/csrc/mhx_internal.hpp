@@ -188,6 +188,7 @@ struct ScopedPhase {
 template <class T>
 struct KrylovVecs {
   DevBuf<T> r, z, p, q, tmp, tmp2, V, prec;  // prec: 1/diag or nodal block inverses
+  DevBuf<T> ell;                              // one-workgroup CG: the matrix by entry index
   DevBuf<T> rhs, sol;                         // inner system of the refinement loop
 };
 struct KrylovWork {

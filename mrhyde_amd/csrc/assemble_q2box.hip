@@ -189,8 +189,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   const double Jy = 0.5 * (vert(0, cey + 1, 0, 1) - vert(0, cey, 0, 1));
   const double Jz = 0.5 * (vert(0, 0, cez + 1, 2) - vert(0, 0, cez, 2));
   const double iJy2 = 1.0 / (Jy * Jy), iJz2 = 1.0 / (Jz * Jz);
-  const double wyz = fabs(Jy * Jz) * sel3(q1, kT.W[0], kT.W[1], kT.W[2]) * sel3(q2, kT.W[0], kT.W[1], kT.W[2]) *
-                     sel3(q3, kT.W[0], kT.W[1], kT.W[2]);
+  const double ajyz = pact ? fabs(Jy * Jz) : 0.0;
+  const double wq = sel3(q1, kT.W[0], kT.W[1], kT.W[2]) * sel3(q2, kT.W[0], kT.W[1], kT.W[2]) *
+                    sel3(q3, kT.W[0], kT.W[1], kT.W[2]);
   double b1[3], d1[3];
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
@@ -361,15 +362,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         for (int m = 0; m < n_modes; ++m) f = fma(s_myz[m][pp], s_mx[m][q1], f);
       }
       // k = k0 (1 + a u^2) and k' (ThermalPhysics in thermal.hpp)
-      const double w = pact ? wyz * fabs(Jx) : 0.0;
-      const double wk0 = w * k0;
+      // (products in the order of k_q2res)
+      const double aj = ajyz * fabs(Jx);
+      const double wk0 = wq * (aj * k0);
       const double kap = wk0 * fma(diff_u2 * U, U, 1.0);
       const double gx = Gx * iJx2, gy = Gy * iJy2, gz = Gz * iJz2;
       double* F = s_fs + tid;
       F[0] = kap * gx;
       F[243] = kap * gy;
       F[2 * 243] = kap * gz;
-      F[3 * 243] = -w * f;
+      F[3 * 243] = -(wq * (aj * f));
       if constexpr (JAC) {
         const double wkp = wk0 * (2.0 * diff_u2 * U);
         F[4 * 243] = kap;
@@ -431,23 +433,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     }
     if (wv == 2 && lane < 54 && ga_res) {
       const double* Flo = s_fs + (zpy + 3 * zzc) * 9 + zq;
-      double v[3] = {0.0, 0.0, 0.0}, m[3] = {0.0, 0.0, 0.0};  // x, y, value rows
+      // (here and below a row sums each element on its own, then the two: the
+      // order of k_q2res, which has one element in a lane)
+      double l[3] = {0.0, 0.0, 0.0}, v[3] = {0.0, 0.0, 0.0}, m[3] = {0.0, 0.0, 0.0};  // x, y, value rows
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         const double* lo = Flo + 81 * q;
         const double* hi = lo + 27;
         const double hx = hi[0], hy = hi[243], hz = hi[2 * 243], hs = hi[3 * 243];
-        v[0] = fma(kT.B[2][q], lo[0], fma(kT.B[0][q], hx, v[0]));
-        v[1] = fma(kT.B[2][q], lo[243], fma(kT.B[0][q], hy, v[1]));
-        v[2] = fma(kT.D[2][q], lo[2 * 243], fma(kT.D[0][q], hz, v[2]));
-        v[2] = fma(kT.B[2][q], lo[3 * 243], fma(kT.B[0][q], hs, v[2]));
+        l[0] = fma(kT.B[2][q], lo[0], l[0]);
+        l[1] = fma(kT.B[2][q], lo[243], l[1]);
+        l[2] = fma(kT.B[2][q], lo[3 * 243], fma(kT.D[2][q], lo[2 * 243], l[2]));
+        v[0] = fma(kT.B[0][q], hx, v[0]);
+        v[1] = fma(kT.B[0][q], hy, v[1]);
+        v[2] = fma(kT.B[0][q], hs, fma(kT.D[0][q], hz, v[2]));
         m[0] = fma(kT.B[1][q], hx, m[0]);
         m[1] = fma(kT.B[1][q], hy, m[1]);
-        m[2] = fma(kT.D[1][q], hz, fma(kT.B[1][q], hs, m[2]));
+        m[2] = fma(kT.B[1][q], hs, fma(kT.D[1][q], hz, m[2]));
       }
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        s_tr[a * 108 + lane] = v[a];
+        s_tr[a * 108 + lane] = l[a] + v[a];
         s_tr[a * 108 + 54 + lane] = m[a];
       }
     }
@@ -494,17 +500,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       const int r = lane - 48;  // q1, z row, yc; zc = wv & 1
       const int a1 = r % 3, zr = (r / 3) % 2, yc = r / 6;
       const double* Tl = s_tr + zr * 54 + ((wv & 1) * 3 + yc) * 9 + a1;  // low element; the high one 9 on
-      double vx = 0.0, v0 = 0.0, mx = 0.0, m0 = 0.0;
+      double lx = 0.0, l0 = 0.0, vx = 0.0, v0 = 0.0, mx = 0.0, m0 = 0.0;
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         const double* lo = Tl + 3 * q;
         const double* hi = lo + 9;
-        vx = fma(kT.B[2][q], lo[0], fma(kT.B[0][q], hi[0], vx));
-        v0 = fma(kT.D[2][q], lo[108], fma(kT.D[0][q], hi[108], v0));
-        v0 = fma(kT.B[2][q], lo[216], fma(kT.B[0][q], hi[216], v0));
+        lx = fma(kT.B[2][q], lo[0], lx);
+        l0 = fma(kT.B[2][q], lo[216], fma(kT.D[2][q], lo[108], l0));
+        vx = fma(kT.B[0][q], hi[0], vx);
+        v0 = fma(kT.B[0][q], hi[216], fma(kT.D[0][q], hi[108], v0));
         mx = fma(kT.B[1][q], hi[0], mx);
-        m0 = fma(kT.D[1][q], hi[108], fma(kT.B[1][q], hi[216], m0));
+        m0 = fma(kT.B[1][q], hi[216], fma(kT.D[1][q], hi[108], m0));
       }
+      vx += lx;
+      v0 += l0;
       double* o = s_sr[e & 1] + ((yc + 2 * (wv & 1)) * 4 + 2 * zr) * 6 + a1 * 2;
       o[0] = vx;
       o[1] = v0;
@@ -524,15 +533,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       if (Y < N1 && Z < N2) {
         const double* cur = s_sr[e & 1] + lane * 6;
         const double* old = s_sr[(e & 1) ^ 1] + lane * 6;
-        double r0 = 0.0, r1 = 0.0, r2 = 0.0;
+        double r0 = 0.0, r1 = 0.0, r2 = 0.0, ro = 0.0;
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
           const double cx = cur[2 * q], c0 = cur[2 * q + 1];
           r0 = fma(kT.D[0][q], cx, fma(kT.B[0][q], c0, r0));
           r1 = fma(kT.D[1][q], cx, fma(kT.B[1][q], c0, r1));
           r2 = fma(kT.D[2][q], cx, fma(kT.B[2][q], c0, r2));
-          if (e > 0) r0 = fma(kT.D[2][q], old[2 * q], fma(kT.B[2][q], old[2 * q + 1], r0));
+          if (e > 0) ro = fma(kT.D[2][q], old[2 * q], fma(kT.B[2][q], old[2 * q + 1], ro));
         }
+        r0 += ro;
         const long row = 2 * (long)e + (long)N0 * (Y + (long)N1 * Z);
         const double rr[3] = {r0, r1, r2};
 #pragma unroll
@@ -686,6 +696,12 @@ int q2box_segment(const Ctx& c, bool jac) {
 }
 
 void launch_q2box(Ctx& c, AsmArgs& a, bool jac) {
+  // the residual alone: k_q2res, without sine modes (their factors at the 27
+  // points do not fit beside an element's registers).  64^3 us: 162 and 64
+  if (!jac && a.coef.n_modes == 0) {
+    launch_q2res(c, a);
+    return;
+  }
   const int L = q2box_segment(c, jac);
   a.gpb = L;
   a.nseg = (c.mesh.nel[0] + L - 1) / L;
@@ -697,8 +713,7 @@ void launch_q2box(Ctx& c, AsmArgs& a, bool jac) {
     if (jac) hipLaunchKernelGGL((k_q2box<true, true>), grid, block, 0, c.stream, a);
     else hipLaunchKernelGGL((k_q2box<false, true>), grid, block, 0, c.stream, a);
   } else {
-    if (jac) hipLaunchKernelGGL((k_q2box<true, false>), grid, block, 0, c.stream, a);
-    else hipLaunchKernelGGL((k_q2box<false, false>), grid, block, 0, c.stream, a);
+    hipLaunchKernelGGL((k_q2box<true, false>), grid, block, 0, c.stream, a);
   }
   MHX_HIP(hipGetLastError());
 }

@@ -265,6 +265,7 @@ void lagrange_equispaced(int p, double xi, double* L, double* dL);
 bool thermal_supported(int dim, int p, int nq1);
 // Q2 hexahedra on box meshes: row-owned pair-factorised assembly (assemble_q2box.hip)
 bool q2box_applicable(const Ctx& c);
+void launch_q2res(Ctx& c, AsmArgs& a);  // residual alone (assemble_q2res.hip)
 void launch_q2box(Ctx& c, AsmArgs& a, bool jac);
 int q2box_segment(const Ctx& c, bool jac);  // elements per x-segment of a launch
 // element store (assemble_elem.hip): doubles of element matrices where the

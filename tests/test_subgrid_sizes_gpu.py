@@ -1,0 +1,73 @@
+"""Batched subgrid solves at every size per axis (each has its own columns per
+thread), both workgroup sizes and precisions, cubes and boxes with sources,
+against the residual of the oracle's system; and the transfer of large results
+through staging buffers against the same instances in small batches.
+
+Tolerance: the solver's own (1e-10), with a factor two for the residual that the
+oracle's matrix gives in another order of sums."""
+import numpy as np
+import pytest
+
+from conftest import spmv_np
+from mrhyde_amd.abi import Problem
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def systems():
+    from oracle import Oracle
+
+    rng = np.random.default_rng(8)
+    out = {}
+    for box in (False, True):
+        n_axis = np.arange(2, 17, dtype=np.int32)
+        k, g, src, ext, orc = [], [], [], [], []
+        for n in n_axis:
+            ne, nn = int(n) ** 3, (int(n) + 1) ** 3
+            k.append(np.exp(0.5 * rng.standard_normal(ne)))
+            g.append(rng.uniform(-1, 1, nn))
+            src.append(rng.standard_normal(ne))
+            ext.append(rng.uniform(0.5, 2.0, 3) if box else np.ones(3))
+            o = Oracle(Problem(dim=3, order=1, quadrature=2, n=(int(n),) * 3, hi=tuple(ext[-1]), k0=k[-1],
+                               src_elem=src[-1] if box else None, dbc_values=g[-1]))
+            u0 = o.setDirichlet(np.zeros(o.n_dof))
+            orc.append((u0, *o.assembleJacRes(u0), *o.crs_pattern()))
+        out[box] = (n_axis, np.concatenate(k), np.concatenate(g), dict(extent=np.array(ext), src=np.concatenate(src))
+                    if box else {}, orc)
+    return out
+
+
+@pytest.mark.parametrize("box", [False, True])
+@pytest.mark.parametrize("wg", [512, 1024])
+@pytest.mark.parametrize("precision", ["fp64", "fp32-refined"])
+def test_every_size(systems, precision, wg, box):
+    from mrhyde_amd import SubgridBatch
+
+    n_axis, k, g, kw, orc = systems[box]
+    b = SubgridBatch(n_axis, k, g, tol=1e-10, precision=precision, wg_size=wg, **kw)
+    b.solve()
+    x, _, rel, _ = b.results()
+    for i, (u0, res, jac, rp, ci) in enumerate(orc):
+        r = res - spmv_np(rp, ci, jac, b.instance(x, i) - u0)
+        assert rel[i] <= 1e-10 and np.linalg.norm(r) <= 2e-10 * np.linalg.norm(res), (int(n_axis[i]), rel[i])
+    b.close()
+
+
+def test_large_results_equal_small_batches():
+    from mrhyde_amd import SubgridBatch
+
+    rng = np.random.default_rng(4)
+    n_axis = np.full(70, 16, dtype=np.int32)  # 2.75 MB of results
+    k = np.exp(0.3 * rng.standard_normal((70, 16 ** 3)))
+    g = rng.uniform(-1, 1, (70, 17 ** 3))
+    big = SubgridBatch(n_axis, k.ravel(), g.ravel())
+    big.solve()
+    x = big.results()[0]
+    np.testing.assert_array_equal(big.results()[0], x)
+    for lo, hi in ((0, 10), (37, 47), (60, 70)):  # below 1 MiB each
+        s = SubgridBatch(n_axis[lo:hi], k[lo:hi].ravel(), g[lo:hi].ravel())
+        s.solve()
+        np.testing.assert_array_equal(s.results()[0], x[lo * 17 ** 3:hi * 17 ** 3])
+        s.close()
+    big.close()

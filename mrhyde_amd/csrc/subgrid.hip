@@ -478,9 +478,9 @@ struct CopyRing {
     buf = nullptr;
   }
   // worker w's chunks w, w + kWorkers, ... of src -> dst
-  hipError_t work(int w, hipStream_t stream, char* dst, const char* src, size_t bytes, size_t chunk) {
+  hipError_t work(int w, hipStream_t stream, char* dst, const char* src, size_t bytes, size_t chunk, bool own_thread) {
     char* mine = buf + (size_t)w * kChunk;
-    hipError_t e = hipSetDevice(dev);
+    hipError_t e = own_thread ? hipSetDevice(dev) : hipSuccess;
     for (size_t at = (size_t)w * chunk; at < bytes && e == hipSuccess; at += kWorkers * chunk) {
       const size_t len = std::min(chunk, bytes - at);
       e = hipMemcpyAsync(mine, src + at, len, hipMemcpyDeviceToHost, stream);
@@ -492,11 +492,9 @@ struct CopyRing {
   }
 };
 
-static std::shared_ptr<CopyRing> copy_ring() {
+static std::shared_ptr<CopyRing> copy_ring(int dev) {
   static std::mutex mu;
   static std::map<int, std::weak_ptr<CopyRing>> rings;
-  int dev = 0;
-  MHX_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lk(mu);
   std::shared_ptr<CopyRing> r = rings[dev].lock();
   if (!r) rings[dev] = r = std::make_shared<CopyRing>(dev);
@@ -504,6 +502,8 @@ static std::shared_ptr<CopyRing> copy_ring() {
 }
 
 struct Batch {
+  int dev = 0;  // the device it was created on
+  std::mutex ring_mu;              // guards ring
   std::shared_ptr<CopyRing> ring;  // for results(), from the first large copy on
   int n_inst = 0;
   long total_nodes = 0, total_elems = 0;
@@ -571,24 +571,38 @@ static void enqueue(Batch& b, int wg) {
 
 // device array -> host array, complete on return
 static void copy_to_host(Batch& b, void* dst, const void* src, size_t bytes) {
-  if (bytes >= CopyRing::kMinBytes) {
-    if (!b.ring) b.ring = copy_ring();
-    std::unique_lock<std::mutex> lk(b.ring->busy, std::try_to_lock);
+  int dev = -1;
+  MHX_HIP(hipGetDevice(&dev));
+  std::shared_ptr<CopyRing> ring;
+  if (bytes >= CopyRing::kMinBytes && dev == b.dev) {
+    std::lock_guard<std::mutex> lk(b.ring_mu);
+    if (!b.ring) {
+      try {
+        b.ring = copy_ring(dev);
+      } catch (...) {  // no pinned memory to be had: the runtime's path
+        (void)hipGetLastError();
+      }
+    }
+    ring = b.ring;
+  }
+  if (ring) {
+    std::unique_lock<std::mutex> lk(ring->busy, std::try_to_lock);
     if (lk.owns_lock()) {
       const size_t chunk = std::min(CopyRing::kChunk, (bytes + CopyRing::kWorkers - 1) / CopyRing::kWorkers);
       hipError_t err[CopyRing::kWorkers] = {};
-      std::vector<std::thread> th;
-      th.reserve(CopyRing::kWorkers);
-      auto run = [&](int w) { err[w] = b.ring->work(w, b.stream, (char*)dst, (const char*)src, bytes, chunk); };
+      std::thread th[CopyRing::kWorkers];
+      auto run = [&](int w, bool own_thread) {
+        err[w] = ring->work(w, b.stream, (char*)dst, (const char*)src, bytes, chunk, own_thread);
+      };
       int started = 1;
       try {
-        for (; started < CopyRing::kWorkers; ++started) th.emplace_back(run, started);
-      } catch (const std::system_error&) {
+        for (; started < CopyRing::kWorkers; ++started) th[started] = std::thread(run, started, true);
+      } catch (const std::exception&) {
         // no thread to be had: the remaining workers' chunks follow here
       }
-      run(0);
-      for (int w = started; w < CopyRing::kWorkers; ++w) run(w);
-      for (auto& t : th) t.join();
+      run(0, false);
+      for (int w = started; w < CopyRing::kWorkers; ++w) run(w, false);
+      for (int w = 1; w < started; ++w) th[w].join();
       for (hipError_t e : err) MHX_HIP(e);
       return;
     }
@@ -665,6 +679,7 @@ int mhx_batch_create(const mhx_batch_desc* d, mhx_batch** out) {
     MHX_REQUIRE(d && out && d->n_inst > 0 && d->n_axis && d->k && d->g, MHX_ERR_ARG, "bad batch description");
     *out = nullptr;
     b = new mhx_batch();
+    MHX_HIP(hipGetDevice(&b->dev));
     b->desc = *d;
     if (b->desc.tol <= 0) b->desc.tol = 1e-10;
     if (b->desc.max_iters <= 0) b->desc.max_iters = 10000;

@@ -33,15 +33,15 @@ LDS_PEAK_TBS = 256 * 128 * 2.4e9 / 1e12  # 256 CUs x 128 B/clk x 2.4 GHz
 
 # HBM traffic per launch of the dominant assembly kernel (96^3 Q2), keyed by
 # (elements per axis, assembly.colouring), from rocprofv3 --pmc FETCH_SIZE /
-# WRITE_SIZE runs of this bench (mean of the 8 colour launches), scaled by the
-# factors that make the same counters read the known size of the plain copy
-# kernel: FETCH x 2048 B, WRITE x 1024 B.  Colouring 0: k_thermal<jacres>
-# (profiles/k_thermal_q2hex_96cubed.md); colouring 3: k_q2box<jacres>, x-segments
-# of 12 elements (profiles/k_q2box_q2hex_96cubed.md).  Only valid for those
-# workloads.
+# WRITE_SIZE runs of the same assembly, scaled by the factors that make the same
+# counters read the known size of the plain copy kernel: FETCH x 2048 B, WRITE x
+# 1024 B.  Colouring 0: k_thermal<jacres>, mean of its 8 colour launches
+# (profiles/k_thermal_q2hex_96cubed.md); colouring 3: k_q2box<jacres>, one
+# launch, x-segments of 24 elements (profiles/k_q2box_q2hex_96cubed.md).  Only
+# valid for those workloads.
 PMC_TRAFFIC = {(96, 0): {"fetch_kib": 529028.5, "write_kib": 1032647.0, "fetch_scale": 2048, "write_scale": 1024},
-               (96, 3): {"fetch_kib": 326291.6, "write_kib": 720445.1, "fetch_scale": 2048, "write_scale": 1024,
-                         "segment": 12}}
+               (96, 3): {"fetch_kib": 170600.0, "write_kib": 3925000.0, "fetch_scale": 2048, "write_scale": 1024,
+                         "segment": 24}}
 
 
 def c2_problem(n: int):

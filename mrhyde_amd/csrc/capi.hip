@@ -371,7 +371,7 @@ int mhx::ctx_create(const mhx_problem_desc* desc, bool element_store, mhx_ctx** 
   build_box(*c);
   upload_functions(*c);
   // the lattice without node perturbation has axis-aligned box elements: Q2
-  // thermal assembly then defaults to the pencil-streamed kernel
+  // thermal assembly then defaults to the row-owned kernel (k_q2box)
   c->box_mesh = desc->perturb == 0.0;
   if (q2box_applicable(*c)) c->scatter_mode = kPencilStream;
   // small general meshes: element matrices to scratch (now, so that no

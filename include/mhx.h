@@ -384,9 +384,9 @@ int  mhx_l2_error(mhx_ctx* ctx, const double* u, int32_t n_modes, const double* 
  *                         mesh only, MHX_ERR_ARG elsewhere).  Default: 3
  *                         where it applies, 2 for Navier-Stokes, else 0;
  *                         while 0 is the default and not set, small
- *                         thermal meshes (element matrices up to 24 MiB,
- *                         3-D 80 MiB, order 1 128 MiB) are assembled in two
- *                         launches: element matrices, then a sum per row.
+ *                         thermal meshes (element matrices up to 384 MiB)
+ *                         are assembled in two launches: element matrices,
+ *                         then a sum per row.
  *   "assembly.segment"    pencil streaming: elements per x-segment, even,
  *                         2 .. 4096 (default: from the mesh, so that the
  *                         workgroups fill the device evenly).

@@ -13,106 +13,135 @@
 // same fixed order of contributions on every run; Dirichlet rows become e_d
 // (scatter.hpp:208,253; constraints.hpp:125-141) in the same pass.
 //
-// The gather is bound by load latency on small meshes and by the traffic of
-// the element matrices on large ones.  Its 2^dim loads per entry are issued
-// together whether or not the entry has that many contributions: 64^2 Q1
-// 10.3 us with a loop over the contributions, 9.8 us so; Q2 hexes 16^3 55.6
-// and 51.7 us.
+// The gather is bound by load latency on small meshes and by its instructions
+// and the traffic of the element matrices on large ones.  A row collects whole
+// rows of its elements' matrices in an LDS image: every value is loaded once,
+// coalesced, with one address per element.  A lane per CRS entry that fetches
+// the entry's at most 2^dim values (mostly repeats, an address each) took 385 us
+// at 40^3 Q2, this 216.
 
 #include "thermal_kernel.hpp"
 
 namespace mhx {
 
-// LANES lanes walk the entries of one row; the last one sums its residual.
-template <int DIM, int P, int LANES>
-__global__ __launch_bounds__(256) void k_gather_rows(AsmArgs a) {
-  constexpr int P1 = P + 1, NB = ipow(P1, DIM);
-  const unsigned row = (blockIdx.x * 256u + threadIdx.x) / LANES;
-  const int l = threadIdx.x % LANES;
-  if (row >= (unsigned)a.m.ndof) return;
-  int c[3];
-  {
-    const unsigned yz = row / (unsigned)a.m.nn[0];
-    c[0] = (int)(row - yz * (unsigned)a.m.nn[0]);
-    c[2] = DIM == 3 ? (int)(yz / (unsigned)a.m.nn[1]) : 0;
-    c[1] = (int)(yz - (unsigned)c[2] * (unsigned)a.m.nn[1]);
-  }
-  // the row's elements per axis (elo .. ehi) and columns (lo, len)
-  int elo[3] = {0, 0, 0}, ehi[3] = {0, 0, 0}, lo[3] = {0, 0, 0}, len[3] = {1, 1, 1};
+namespace {
+
+// LDS traffic between the lanes of one wavefront (its LDS operations complete
+// in order; the fences keep the compiler from reordering)
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// A row (node) of the lattice and the at most 2^DIM elements around it in the
+// order of the element colours: per axis the even one of two first.  Offsets
+// are 32-bit (the rule below bounds the scratch memory).
+template <int DIM, int P>
+struct RowElems {
+  static constexpr int P1 = P + 1;
+  int c[3], lo[3], len[3];
+  int el[3][2], il[3][2], po[3][2];  // per axis and turn: element, local node, first column in the row
+  bool two[3];
+  __device__ __forceinline__ RowElems(const BoxMesh& m, unsigned row) {
+    const unsigned yz = row / (unsigned)m.nn[0];
+    c[0] = (int)(row - yz * (unsigned)m.nn[0]);
+    c[2] = DIM == 3 ? (int)(yz / (unsigned)m.nn[1]) : 0;
+    c[1] = (int)(yz - (unsigned)c[2] * (unsigned)m.nn[1]);
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) {
-    const int e = c[d] / P;
-    elo[d] = c[d] % P == 0 && e > 0 ? e - 1 : e;
-    ehi[d] = min(e, a.m.nel[d] - 1);
-    lo[d] = P * elo[d];
-    len[d] = P * (ehi[d] - elo[d] + 1) + 1;
-  }
-  const bool fixed = a.fixed[row] != 0, add = a.first_touch == 0;
-  if (fixed && add) return;  // the caller's rows; the diagonal is set afterwards
-  if (a.jac) {
-    const int b = a.rowptr[row], n = len[0] * len[1] * len[2];
-    const float iw = 1.0f / (float)len[0], iy = 1.0f / (float)len[1];
-    for (int q = l; q < n; q += LANES) {
-      // (float reciprocals are exact for these extents, see LatRow)
-      const int run = (int)(((float)q + 0.5f) * iw);
-      const int rz = DIM == 3 ? (int)(((float)run + 0.5f) * iy) : 0;
-      const int j[3] = {lo[0] + q - run * len[0], lo[1] + run - rz * len[1], lo[2] + rz};
-      double* o = a.jac + b + q;
-      double v = add ? *o : 0.0;
-      if (fixed) {
-        v = j[0] == c[0] && j[1] == c[1] && (DIM == 2 || j[2] == c[2]) ? 1.0 : 0.0;
-      } else {
-        // per axis the offset of the first element that holds both nodes (the
-        // even one of two) and the step to the second: 0 where there is none.
-        // All 2^dim loads are issued together (those without an element repeat
-        // an address), then summed in the order of the element colours, so the
-        // sums are those of element colouring to the bit.
-        long off[3], step[3];
-#pragma unroll
-        for (int d = 0, es = 1, ns = 1; d < 3; ++d, ns *= P1) {
-          const bool two = elo[d] != ehi[d] && j[d] == c[d];
-          const int hi = two ? elo[d] & 1 : (int)(j[d] > c[d]);  // start at the high element
-          const int f = hi ? ehi[d] : elo[d];
-          off[d] = (long)es * f * (NB * NB) + ns * ((c[d] - P * f) * NB + (j[d] - P * f));
-          step[d] = two ? (long)es * (NB * NB) - ns * (P * NB + P) : 0;
-          if (hi) step[d] = -step[d];
-          if (DIM == 2 && d == 2) off[d] = step[d] = 0;
-          es *= a.m.nel[d];
-        }
-        const double* E = a.escr + (off[0] + off[1] + off[2]);
-        double w[1 << DIM];
-#pragma unroll
-        for (int k = 0; k < 1 << DIM; ++k)
-          w[k] = E[(k & 1 ? step[0] : 0) + (k & 2 ? step[1] : 0) + (k & 4 ? step[2] : 0)];
-#pragma unroll
-        for (int k = 0; k < 1 << DIM; ++k)
-          if (!((k & 1 && !step[0]) || (k & 2 && !step[1]) || (k & 4 && !step[2]))) v += w[k];
+    for (int d = 0; d < 3; ++d) {
+      if (d >= DIM) {
+        el[d][0] = el[d][1] = il[d][0] = il[d][1] = po[d][0] = po[d][1] = lo[d] = 0;
+        len[d] = 1;
+        two[d] = false;
+        continue;
       }
-      *o = v;
+      const int e = c[d] / P;
+      const int elo = c[d] % P == 0 && e > 0 ? e - 1 : e, ehi = min(e, m.nel[d] - 1);
+      two[d] = elo != ehi;
+      lo[d] = P * elo;
+      len[d] = P * (ehi - elo + 1) + 1;
+      el[d][0] = two[d] && (elo & 1) ? ehi : elo;
+      el[d][1] = elo + ehi - el[d][0];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        il[d][t] = c[d] - P * el[d][t];
+        po[d][t] = P * (el[d][t] - elo);
+      }
     }
   }
-  if (a.res && l == LANES - 1) {
-    double v = add ? a.res[row] : 0.0;
-    if (!fixed)
-      for (int k = 0; k < 1 << DIM; ++k) {
-        // colour order: the even element of two first
-        int ee[3];
-        bool in = true;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const int kd = (k >> d) & 1;
-          in = in && !(kd && elo[d] == ehi[d]);
-          ee[d] = kd ^ (elo[d] != ehi[d] ? elo[d] & 1 : 0) ? ehi[d] : elo[d];
-        }
-        if (!in) continue;
-        const int ex = ee[0], ey = ee[1], ez = ee[2];
-        const long e = ex + (long)a.m.nel[0] * (ey + (long)a.m.nel[1] * ez);
-        int il = (c[0] - P * ex) + P1 * (c[1] - P * ey);
-        if constexpr (DIM == 3) il += P1 * P1 * (c[2] - P * ez);
-        v -= a.rscr[e * NB + il];
-      }
-    a.res[row] = v;
+  __device__ __forceinline__ bool has(int k) const {
+    return !((k & 1 && !two[0]) || (k & 2 && !two[1]) || (k & 4 && !two[2]));
   }
+  __device__ __forceinline__ unsigned elem(const BoxMesh& m, int k) const {
+    return (unsigned)(el[0][k & 1] + m.nel[0] * (el[1][k >> 1 & 1] + m.nel[1] * el[2][k >> 2 & 1]));
+  }
+  __device__ __forceinline__ unsigned local(int k) const {
+    return (unsigned)(il[0][k & 1] + P1 * (il[1][k >> 1 & 1] + P1 * il[2][k >> 2 & 1]));
+  }
+};
+
+// the residual of row r from its elements' parts
+template <int DIM, int P>
+__device__ __forceinline__ void gather_residual(const AsmArgs& a, unsigned row, const RowElems<DIM, P>& r, bool fixed) {
+  constexpr int NB = ipow(P + 1, DIM);
+  const bool add = a.first_touch == 0;
+  double w[1 << DIM], v = add ? a.res[row] : 0.0;
+#pragma unroll
+  for (int k = 0; k < 1 << DIM; ++k) w[k] = a.rscr[r.elem(a.m, k) * (unsigned)NB + r.local(k)];
+#pragma unroll
+  for (int k = 0; k < 1 << DIM; ++k) v = r.has(k) ? v - w[k] : v;
+  if (!fixed) a.res[row] = v;
+  else if (!add) a.res[row] = 0.0;
+}
+
+}  // namespace
+
+// L lanes per row: lane l takes column l of each element's row, and the
+// elements are added one after the other into the row's image in LDS, which
+// leaves in CRS order.
+template <int DIM, int P, int L>
+__global__ __launch_bounds__(256) void k_gather_rows(AsmArgs a) {
+  constexpr int P1 = P + 1, NB = ipow(P1, DIM), G = 256 / L, ROW = ipow(2 * P + 1, DIM);
+  static_assert(NB <= L && L <= 64, "one column of an element's row per lane");
+  __shared__ double s_img[G][ROW];
+  const int g = threadIdx.x / L, l = threadIdx.x % L;
+  const unsigned row = blockIdx.x * (unsigned)G + g;
+  if (row >= (unsigned)a.m.ndof) return;
+  const RowElems<DIM, P> r(a.m, row);
+  const bool fixed = a.fixed[row] != 0, add = a.first_touch == 0;
+  const int b = a.rowptr[row], n = r.len[0] * r.len[1] * r.len[2];
+  const unsigned col = min(l, NB - 1);
+  double w[1 << DIM];
+#pragma unroll
+  for (int k = 0; k < 1 << DIM; ++k)
+    if (__any(r.has(k))) w[k] = a.escr[(r.elem(a.m, k) * (unsigned)NB + r.local(k)) * (unsigned)NB + col];
+  double* img = s_img[g];
+  for (int q = l; q < n; q += L) img[q] = add ? a.jac[b + q] : 0.0;
+  const int j0 = l % P1, j1 = (l / P1) % P1, j2 = DIM == 3 ? l / (P1 * P1) : 0;
+#pragma unroll
+  for (int k = 0; k < 1 << DIM; ++k)
+    if (__any(r.has(k))) {
+      wave_lds_sync();
+      if (r.has(k) && l < NB)
+        img[j0 + r.po[0][k & 1] + r.len[0] * (j1 + r.po[1][k >> 1 & 1] + r.len[1] * (j2 + r.po[2][k >> 2 & 1]))] += w[k];
+    }
+  wave_lds_sync();
+  if (!fixed) {
+    for (int q = l; q < n; q += L) a.jac[b + q] = img[q];
+  } else if (!add) {  // (accumulating, the caller sets the diagonal afterwards)
+    const int dg = r.c[0] - r.lo[0] + r.len[0] * (r.c[1] - r.lo[1] + r.len[1] * (r.c[2] - r.lo[2]));
+    for (int q = l; q < n; q += L) a.jac[b + q] = q == dg ? 1.0 : 0.0;
+  }
+  if (a.res && l == 0) gather_residual<DIM, P>(a, row, r, fixed);
+}
+
+// the residual alone: a row per lane
+template <int DIM, int P>
+__global__ __launch_bounds__(256) void k_gather_res(AsmArgs a) {
+  const unsigned row = blockIdx.x * 256u + threadIdx.x;
+  if (row >= (unsigned)a.m.ndof) return;
+  gather_residual<DIM, P>(a, row, RowElems<DIM, P>(a.m, row), a.fixed[row] != 0);
 }
 
 namespace {
@@ -129,10 +158,13 @@ void launch_store(Ctx& c, AsmArgs& a, bool jac) {
     MHX_HIP(hipGetLastError());
   }
   ScopedPhase ph(c.prof, "k_gather_rows", c.stream);
-  // lanes per row: an interior row of the order has 9 (2-D Q1) to 27 or more entries
-  constexpr int L = ipow(P + 1, DIM) <= 9 ? 8 : 32;
-  hipLaunchKernelGGL((k_gather_rows<DIM, P, L>), dim3((unsigned)((c.mesh.ndof * L + 255) / 256)), dim3(256), 0,
-                     c.stream, a);
+  const long nr = c.mesh.ndof;
+  if (!jac) {
+    hipLaunchKernelGGL((k_gather_res<DIM, P>), dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, c.stream, a);
+  } else {
+    constexpr int NB = ipow(P + 1, DIM), L = NB <= 4 ? 4 : NB <= 8 ? 8 : NB <= 16 ? 16 : NB <= 32 ? 32 : 64;
+    hipLaunchKernelGGL((k_gather_rows<DIM, P, L>), dim3((unsigned)((nr * L + 255) / 256)), dim3(256), 0, c.stream, a);
+  }
   MHX_HIP(hipGetLastError());
 }
 
@@ -152,23 +184,23 @@ const Entry kStoreTable[] = {
 
 }  // namespace
 
-// Where the two launches beat the 2^dim launches of element colouring
-// (us, residual + Jacobian, colouring / here):
-//   2-D Q1 64^2 23.6/9.8, 256^2 31/24, 1024^2 (128 MiB) 257/240
-//   3-D Q1 16^3 77/15, 32^3 81/44, 64^3 (128 MiB) 360/213
-//   2-D Q2 64^2 36/14, 192^2 (23 MiB) 54/45, 256^2 (41 MiB) 68/68
-//   2-D Q3 64^2 48/25, 96^2 (18 MiB) 57/46, 128^2 (32 MiB) 60/66
-//   2-D Q4 64^2 (20 MiB) 77/43; Q6 32^2 (19 MiB) 260/71
-//   3-D Q2, three points per axis: 8^3 168/24, 16^3 169/52, 24^3 (77 MiB)
-//     176/121, 32^3 (182 MiB) 244/272, 40^3 (356 MiB) 473/592
-// Past these sizes the round trip of the element matrices costs more than the
-// colours' launches.  The bound also keeps the scratch memory small; it is
-// allocated with the context, so no assembly allocates.
+// The two launches against the 2^dim launches of element colouring (us, residual
+// + Jacobian, colouring / here):
+//   2-D Q1 64^2 23.3/10.5, 256^2 31/26, 1024^2 (128 MiB) 258/208
+//   2-D Q2 64^2 36/11, 192^2 55/42, 256^2 (41 MiB) 68/64, 384^2 141/123
+//   2-D Q3 64^2 47/21, 128^2 60/49; Q4 64^2 77/37, 96^2 88/69; Q6 32^2 261/69
+//   3-D Q1 16^3 77/12, 32^3 81/37, 64^3 (128 MiB) 360/192
+//   3-D Q2, three points per axis: 8^3 168/21, 16^3 169/42, 24^3 (77 MiB)
+//     176/96, 32^3 (182 MiB) 243/213, 40^3 (356 MiB) 473/429
+// The gain shrinks as the round trip of the element matrices leaves the caches;
+// past the largest size measured the scratch memory (1.35 times the Jacobian in
+// 3-D Q2) is not spent.  It is allocated with the context, so no assembly
+// allocates.
 int64_t element_store_doubles(const mhx_problem_desc& d) {
   if (d.physics != MHX_PHYS_THERMAL || d.n_functions > 0) return 0;
   // boxes at three points per axis: the row-owned kernel (assemble_q2box.hip)
   if (d.dim == 3 && d.order == 2 && d.quadrature / 2 + 1 == 3 && d.perturb == 0.0) return 0;
-  const double cap = (d.order == 1 ? 128.0 : d.dim == 3 ? 80.0 : 24.0) * (1 << 20);
+  const double cap = 384.0 * (1 << 20);
   int64_t nb = 1;
   double n = 1.0;
   for (int a = 0; a < d.dim; ++a) {

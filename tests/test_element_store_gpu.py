@@ -2,7 +2,7 @@
 (the default of small general thermal meshes) against element colouring on the
 same problem: meshes of one element and up, odd counts, every order and rule,
 Dirichlet rows on some and all sides, perturbed and box elements, residual
-alone, accumulation, and sizes on both sides of the rule's bound.
+alone and accumulation.
 
 Tolerance: the two sum at most 2^dim <= 8 element terms, and their kernels may
 contract differently over NQ <= 64 points: (8 + 64) eps times the largest

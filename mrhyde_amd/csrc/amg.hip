@@ -522,13 +522,18 @@ __global__ __launch_bounds__(32 * kAcGroups) void k_amg_Ac(Geo G, const int32_t*
       }
 #pragma unroll
       for (int u = 0; u < UX; ++u) {
-        if (at[u] < 0) continue;
+        // (a node whose box starts one aggregate on has its coarse entries in
+        // other lanes than the node before it: 181 -> 185 us at 48^3 Q2 with
+        // the order enforced)
+        wave_lds_sync();
+        if (at[u] >= 0) {
 #pragma unroll
-        for (int g = 0; g < NF; ++g) {
-          double t = acc[at[u] + g];
+          for (int g = 0; g < NF; ++g) {
+            double t = acc[at[u] + g];
 #pragma unroll
-          for (int f = 0; f < NF; ++f) t = fma(rv[u][f], v[u][f][g], t);
-          acc[at[u] + g] = t;
+            for (int f = 0; f < NF; ++f) t = fma(rv[u][f], v[u][f][g], t);
+            acc[at[u] + g] = t;
+          }
         }
       }
     }

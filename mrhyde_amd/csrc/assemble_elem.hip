@@ -26,14 +26,6 @@ namespace mhx {
 
 namespace {
 
-// LDS traffic between the lanes of one wavefront (its LDS operations complete
-// in order; the fences keep the compiler from reordering)
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // A row (node) of the lattice and the at most 2^DIM elements around it in the
 // order of the element colours: per axis the even one of two first.  Offsets
 // are 32-bit (the rule below bounds the scratch memory).

@@ -80,14 +80,6 @@ __device__ __forceinline__ void lds_sync() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
-// LDS traffic between the lanes of one wavefront (LDS operations of a
-// wavefront complete in order; the fences keep the compiler from reordering
-// and wait for outstanding ones)
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 // LDS strides, chosen so that 16 lanes of a read or write meet 16 banks: a pair
 // (Y, Y', Z, Z') sits at z pair * 9 + y pair, a (q1, group) row of pairs has 72

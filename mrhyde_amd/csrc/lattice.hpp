@@ -6,6 +6,15 @@
 
 namespace mhx {
 
+// LDS traffic between the lanes of one wavefront (LDS operations of a
+// wavefront complete in order; the fences keep the compiler from reordering
+// and wait for outstanding ones)
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // lattice helpers ------------------------------------------------------------
 template <int DIM, int P>
 __device__ __forceinline__ long node_of(const BoxMesh& m, const int* ec, int j) {

@@ -322,7 +322,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   if (wv == 3 && lane < 54) plane(lpl, (2 * eb + 1 + lpl) % 3);
   // values of the next layer, one step ahead
   const long ce0 = (long)n0 * (cey + (long)n1 * cez);
-  double k0n = ga_k0 ? ga_k0[ce0 + eb] : 1.0, srn = ga_src ? ga_src[ce0 + eb] : 0.0;
+  // (0 in pencils off the mesh: a weight of 0 does not clear a coefficient that
+  // is not finite)
+  double k0n = !pact ? 0.0 : ga_k0 ? ga_k0[ce0 + eb] : 1.0, srn = pact && ga_src ? ga_src[ce0 + eb] : 0.0;
   double un = 0.0;
   if (eb + 1 < x1 && gin) un = ga_u[gbase + 2 * eb + 3 + gpl];
   lds_sync();
@@ -374,7 +376,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     }
     // the gathered nodes of the next planes; coefficients of the next layer
     if (tid < 98) s_u[gpl][gn] = un;
-    if (e + 1 < x1) {
+    if (pact && e + 1 < x1) {
       if (ga_k0) k0n = ga_k0[ce0 + e + 1];
       if (ga_src) srn = ga_src[ce0 + e + 1];
     }

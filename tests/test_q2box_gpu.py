@@ -135,3 +135,33 @@ def test_q2box_refused_where_it_does_not_apply():
     with pytest.raises(MhxError):
         q1.set_option("assembly.colouring", 3)
     q1.close()
+
+
+@pytest.mark.parametrize("modes", [False, True])
+@pytest.mark.parametrize("what", ["k0", "src_elem"])
+@pytest.mark.parametrize("ec", [(0, 0, 0), (3, 0, 0), (2, 2, 1)])
+def test_nonfinite_coefficient_stays_in_its_element(ec, what, modes):
+    """An infinite coefficient of one element reaches the rows of that
+    element's nodes and no others: the rest keeps its bits."""
+    from mrhyde_amd import Mhx
+    from mrhyde_amd.abi import Problem
+
+    n = (5, 4, 3)
+    coef = {"k0": lognormal(60, 0.5, 1), "src_elem": np.random.default_rng(2).uniform(0, 1, 60)}
+    kw = dict(modes=[(2.0, (PI, PI, PI))]) if modes else {}
+    g = Mhx(Problem(dim=3, order=2, quadrature=4, n=n, diff_u2=1.0, dbc_sides=0, **coef, **kw))
+    coef[what] = coef[what].copy()
+    coef[what][ec[0] + n[0] * (ec[1] + n[1] * ec[2])] = np.inf
+    b = Mhx(Problem(dim=3, order=2, quadrature=4, n=n, diff_u2=1.0, dbc_sides=0, **coef, **kw))
+    u = np.random.default_rng(3).standard_normal(g.n_dof)
+    (r, j), (rb, jb) = g.assembleJacRes(u), b.assembleJacRes(u)
+    node = np.arange(g.n_dof)
+    c = (node % 11, node // 11 % 9, node // 99)
+    inside = np.logical_and.reduce([(c[a] >= 2 * ec[a]) & (c[a] <= 2 * ec[a] + 2) for a in range(3)])
+    rp, _ = g.crs_pattern()
+    rows = np.repeat(node, np.diff(rp))
+    assert not np.isfinite(rb[inside]).all()
+    np.testing.assert_array_equal(rb[~inside], r[~inside])
+    np.testing.assert_array_equal(jb[~inside[rows]], j[~inside[rows]])
+    np.testing.assert_array_equal(b.assembleRes(u)[~inside], r[~inside])
+    g.close(), b.close()

@@ -513,8 +513,13 @@ typedef struct mhx_batch_desc {
 int  mhx_batch_create(const mhx_batch_desc* desc, mhx_batch** out);
 int  mhx_batch_solve(mhx_batch* b, int32_t flags);
 /* Host copies: x (concatenated nodal solutions), iterations, FP64 relative
- * residual and refinement sweeps per instance (any pointer may be NULL). */
+ * residual and refinement sweeps per instance (any pointer may be NULL).
+ * Large x leaves through pinned host buffers of the library, 8 MiB per device
+ * from the first such call on. */
 int  mhx_batch_results(mhx_batch* b, double* x, int32_t* iters, double* relres, int32_t* refinements);
+/* Gives those buffers back (a copy that is using them finishes first; the next
+ * large one allocates them anew).  Returns the bytes released. */
+int64_t mhx_release_host_buffers(void);
 int  mhx_batch_info(const mhx_batch* b, int64_t* total_nodes, int32_t* wg_size, double* last_ms);
 int  mhx_batch_set_wg(mhx_batch* b, int32_t wg_size);
 void mhx_batch_destroy(mhx_batch* b);

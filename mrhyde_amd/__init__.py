@@ -6,7 +6,8 @@ without the GPU library.  Everything else lives in libmhx.so; accessing
 """
 from .abi import Problem, rng_fill  # noqa: F401
 
-_LAZY = {"Mhx", "MhxError", "krylov_opts", "rng", "SubgridBatch", "Server", "function_eval"}
+_LAZY = {"Mhx", "MhxError", "krylov_opts", "rng", "SubgridBatch", "Server", "function_eval",
+         "release_host_buffers"}
 
 
 def __getattr__(name):

@@ -48,6 +48,7 @@ def _load() -> C.CDLL:
         "mhx_batch_info": (C.c_int, [vp, C.POINTER(i64), C.POINTER(i32), C.POINTER(C.c_double)]),
         "mhx_batch_set_wg": (C.c_int, [vp, i32]),
         "mhx_batch_destroy": (None, [vp]),
+        "mhx_release_host_buffers": (i64, []),
         "mhx_set_option": (C.c_int, [vp, C.c_char_p, i64]),
         "mhx_get_option": (C.c_int, [vp, C.c_char_p, C.POINTER(i64)]),
         "mhx_state_ptr": (C.c_int, [vp, i32, C.POINTER(C.c_void_p), C.POINTER(i64)]),
@@ -89,7 +90,8 @@ EXPORTED = [
     "mhx_dirichlet_mask", "mhx_set_dirichlet", "mhx_dof_coords", "mhx_assemble", "mhx_spmv", "mhx_linear_solve",
     "mhx_nonlinear_solve", "mhx_l2_error", "mhx_profile_enable", "mhx_profile_read", "mhx_profile_reset",
     "mhx_synchronize", "mhx_set_stream", "mhx_set_option", "mhx_get_option", "mhx_copy_probe", "mhx_mfma_probe", "mhx_batch_create", "mhx_batch_solve",
-    "mhx_batch_results", "mhx_batch_info", "mhx_batch_set_wg", "mhx_batch_destroy","mhx_state_ptr", "mhx_state_upload", "mhx_state_download", "mhx_rng_fill", "mhx_version",
+    "mhx_batch_results", "mhx_batch_info", "mhx_batch_set_wg", "mhx_batch_destroy", "mhx_release_host_buffers",
+    "mhx_state_ptr", "mhx_state_upload", "mhx_state_download", "mhx_rng_fill", "mhx_version",
     "mhx_footprint", "mhx_ctx_update", "mhx_server_create", "mhx_server_submit", "mhx_server_poll",
     "mhx_server_info", "mhx_server_last_error", "mhx_server_destroy", "mhx_amg_setup", "mhx_amg_level",
     "mhx_set_time_state", "mhx_write_matrix_market", "mhx_write_vector_market", "mhx_read_matrix_market",

@@ -540,6 +540,12 @@ class SubgridBatch:
         return x[self.offsets[i]:self.offsets[i + 1]]
 
 
+def release_host_buffers() -> int:
+    """Give back the pinned host memory that large SubgridBatch.results() copies
+    hold between calls (8 MiB per device); returns the bytes released."""
+    return lib.mhx_release_host_buffers()
+
+
 class Server:
     """Request loop over mhx_server_*: independent steady solves of mixed mesh
     size, admitted by device-memory footprint, run concurrently (one stream

@@ -54,6 +54,28 @@ def test_every_size(systems, precision, wg, box):
     b.close()
 
 
+def test_result_buffers_outlive_batches_and_are_given_back():
+    from mrhyde_amd import SubgridBatch, release_host_buffers
+
+    rng = np.random.default_rng(5)
+    n_axis = np.full(300, 16, dtype=np.int32)  # 11.8 MB of results
+    args = n_axis, np.exp(0.3 * rng.standard_normal(300 * 16 ** 3)), rng.uniform(-1, 1, 300 * 17 ** 3)
+    release_host_buffers()
+    xs = []
+    for keep in (True, True, False):
+        b = SubgridBatch(*args, wg_size=512)
+        b.solve()
+        xs.append(b.results()[0])
+        if not keep:  # given back in the batch's life: the next copy allocates anew
+            assert release_host_buffers() == 8 << 20
+            xs.append(b.results()[0])
+        b.close()
+    for x in xs[1:]:
+        np.testing.assert_array_equal(x, xs[0])
+    assert release_host_buffers() == 8 << 20
+    assert release_host_buffers() == 0
+
+
 def test_large_results_equal_small_batches():
     from mrhyde_amd import SubgridBatch
 

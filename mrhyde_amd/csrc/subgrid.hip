@@ -578,12 +578,24 @@ static void enqueue(Batch& b, int wg) {
   MHX_HIP(hipGetLastError());
 }
 
+// Ordinary host memory, which the runtime would copy through a staging buffer:
+// pinned and managed memory takes a transfer straight from the device (14.4 MB
+// into pinned memory 0.26 ms, through the ring 0.48).
+static bool ordinary_memory(const void* p) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();  // memory that the runtime does not know
+    return true;
+  }
+  return at.type == hipMemoryTypeUnregistered;
+}
+
 // device array -> host array, complete on return
 static void copy_to_host(Batch& b, void* dst, const void* src, size_t bytes) {
   int dev = -1;
   MHX_HIP(hipGetDevice(&dev));
   std::shared_ptr<CopyRing> ring;
-  if (bytes >= CopyRing::kMinBytes && dev == b.dev) {
+  if (bytes >= CopyRing::kMinBytes && dev == b.dev && ordinary_memory(dst)) {
     try {
       ring = copy_ring(dev);
     } catch (...) {  // no pinned memory to be had: the runtime's path

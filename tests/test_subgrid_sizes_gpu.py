@@ -76,6 +76,24 @@ def test_result_buffers_outlive_batches_and_are_given_back():
     assert release_host_buffers() == 0
 
 
+def test_pinned_destination_needs_no_buffers():
+    import torch
+
+    from mrhyde_amd import SubgridBatch, capi, release_host_buffers
+
+    rng = np.random.default_rng(6)
+    n_axis = np.full(300, 16, dtype=np.int32)
+    b = SubgridBatch(n_axis, np.exp(0.3 * rng.standard_normal(300 * 16 ** 3)), rng.uniform(-1, 1, 300 * 17 ** 3),
+                     wg_size=512)
+    b.solve()
+    out = torch.zeros(b.total_nodes, dtype=torch.float64, pin_memory=True)
+    release_host_buffers()
+    assert capi.lib.mhx_batch_results(b._h, out.data_ptr(), None, None, None) == 0
+    assert release_host_buffers() == 0
+    np.testing.assert_array_equal(out.numpy(), b.results()[0])
+    b.close()
+
+
 def test_large_results_equal_small_batches():
     from mrhyde_amd import SubgridBatch
 

@@ -76,6 +76,26 @@ def test_result_buffers_outlive_batches_and_are_given_back():
     assert release_host_buffers() == 0
 
 
+def test_results_in_chunks_equal_small_batches():
+    """10.4 MB through the buffers (chunks that do not divide it), and sizes on
+    both sides of the line, below which no buffers are taken."""
+    from mrhyde_amd import SubgridBatch, release_host_buffers
+
+    rng = np.random.default_rng(7)
+    n_axis = np.full(265, 16, dtype=np.int32)
+    k, g = np.exp(0.3 * rng.standard_normal((265, 16 ** 3))), rng.uniform(-1, 1, (265, 17 ** 3))
+    release_host_buffers()
+    out = {}
+    for m, held in ((60, 0), (93, 0), (94, 8 << 20), (265, 8 << 20)):  # 2.25, 3.49, 3.52 and 9.93 MiB
+        b = SubgridBatch(n_axis[:m], k[:m].ravel(), g[:m].ravel(), wg_size=512)
+        b.solve()
+        out[m] = b.results()[0]
+        b.close()
+        assert release_host_buffers() == held
+    for m in (60, 93, 94):
+        np.testing.assert_array_equal(out[m], out[265][:m * 17 ** 3])
+
+
 def test_pinned_destination_needs_no_buffers():
     import torch
 

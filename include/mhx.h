@@ -382,11 +382,12 @@ int  mhx_l2_error(mhx_ctx* ctx, const double* u, int32_t n_modes, const double* 
  *                         x-segment and writes each row once; 3-D Q2
  *                         thermal with 3x3x3 Gauss on an unperturbed box
  *                         mesh only, MHX_ERR_ARG elsewhere).  Default: 3
- *                         where it applies, 2 for Navier-Stokes, else 0;
- *                         while 0 is the default and not set, small
- *                         thermal meshes (element matrices up to 384 MiB)
- *                         are assembled in two launches: element matrices,
- *                         then a sum per row.
+ *                         where it applies, 2 for Navier-Stokes, else 0.
+ *   "assembly.element_store"  1 (default): where assembly.colouring is 0,
+ *                         steady thermal assembly of small meshes (element
+ *                         matrices up to 384 MiB) runs in two launches:
+ *                         element matrices, then a sum per row (same sums
+ *                         in the same order); 0: element colouring.
  *   "assembly.segment"    pencil streaming: elements per x-segment, even,
  *                         2 .. 4096 (default: from the mesh, so that the
  *                         workgroups fill the device evenly).

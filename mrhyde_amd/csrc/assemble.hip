@@ -194,7 +194,8 @@ void assemble_thermal(Ctx& c, const double* u, double* res, double* jac, bool wa
     ScopedPhase ph(c.prof, want_jac ? "AssemblyManager::assembleJacRes" : "AssemblyManager::assembleRes", c.stream);
     if (a.xp.active) launch_thermal_expr(c, a, want_jac);
     else if (c.scatter_mode == kPencilStream && !a.hist && q2box_applicable(c)) launch_q2box(c, a, want_jac);
-    else if (c.scatter_auto && !a.hist && c.escr.p) launch_element_store(c, a, want_jac);
+    else if (c.scatter_mode == kElementColouring && c.store_on && !a.hist && c.escr.p)
+      launch_element_store(c, a, want_jac);
     else f(c, a, want_jac);
     // boundary groups, after the volume groups
     if (want_res) neumann_residual(c, res);

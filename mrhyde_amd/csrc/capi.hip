@@ -993,7 +993,14 @@ int mhx_set_option(mhx_ctx* ctx, const char* name, int64_t value) {
       return MHX_ERR_ARG;
     }
     ctx->scatter_mode = (int)value;
-    ctx->scatter_auto = false;
+    return MHX_OK;
+  }
+  if (k == "assembly.element_store") {
+    if (value != 0 && value != 1) {
+      ctx->err = "assembly.element_store must be 0 or 1";
+      return MHX_ERR_ARG;
+    }
+    ctx->store_on = value != 0;
     return MHX_OK;
   }
   if (k == "assembly.segment") {
@@ -1065,6 +1072,10 @@ int mhx_get_option(const mhx_ctx* ctx, const char* name, int64_t* value) {
   }
   if (k == "assembly.colouring") {
     *value = ctx->scatter_mode;
+    return MHX_OK;
+  }
+  if (k == "assembly.element_store") {
+    *value = ctx->store_on ? 1 : 0;
     return MHX_OK;
   }
   if (k == "krylov.spmv_lanes") {

@@ -238,7 +238,7 @@ struct Ctx {
   int amg_omega_pct = 40;  // block-Jacobi smoother: damping in percent
   int nfield = 1;  // unknowns per node (consecutive DOFs): block size of block Jacobi
   int scatter_mode = kElementColouring;
-  bool scatter_auto = true;   // assembly.colouring not set by the caller
+  bool store_on = true;       // assembly.element_store
   DevBuf<double> escr, rscr;  // element matrices and residuals (allocated where the element store applies)
   bool box_mesh = false;  // every element an axis-aligned box (structured box, no node perturbation)
   int q2_segment = 0;     // pencil streaming: elements per x-segment (even; 0: chosen per launch)

@@ -33,7 +33,7 @@ def test_matches_colouring(order, quad, n, perturb, dbc):
                 src_elem=rng.standard_normal(ne), modes=[(1.3, (2.0, 0.0, 3.0)[:len(n)])], dbc_sides=dbc, dbc_const=0.3,
                 perturb=perturb)
     g, c = Mhx(p), Mhx(p)
-    c.set_option("assembly.colouring", 0)
+    c.set_option("assembly.element_store", 0)
     assert g.get_option("assembly.colouring") == 0
     u = rng.standard_normal(g.n_dof)
     rc, jc = c.assembleJacRes(u)
@@ -50,6 +50,43 @@ def test_matches_colouring(order, quad, n, perturb, dbc):
     assert np.abs(ra - rb).max() <= tol_r + 4e-14 * np.abs(r0).max()
     assert np.abs(ja - jb).max() <= tol_j + 4e-14 * np.abs(j0).max()
     g.close(), c.close()
+
+
+def _routes(g, u):
+    """Names of the kernels that one assembly of residual and Jacobian runs."""
+    g.profile_reset()
+    g.profile(True)
+    g.assembleJacRes(u)
+    g.profile(False)
+    return {k for k, v in g.profile_read().items() if k.startswith("k_") and v[1]}
+
+
+PROBLEMS = {"general": dict(dim=2, order=1, quadrature=2, n=(9, 8)), "box": dict(dim=3, order=2, quadrature=4, n=(3, 2, 2)),
+            "navier-stokes": dict(dim=2, order=1, quadrature=2, n=(6, 5), physics=2, mu=0.1, supg=True, pspg=True)}
+
+
+@pytest.mark.parametrize("kind", list(PROBLEMS))
+def test_assembly_options_survive_a_round_trip(kind):
+    """Reading the assembly options and setting them to what was read, before
+    and after other values, leaves the route of the default."""
+    from mrhyde_amd import Mhx
+
+    g = Mhx(Problem(**PROBLEMS[kind]))
+    u = np.random.default_rng(1).standard_normal(g.n_dof)
+    first = _routes(g, u)
+    assert ("k_gather_rows" in first) == (kind == "general"), first
+    names = ("assembly.colouring", "assembly.element_store")
+    saved = {k: g.get_option(k) for k in names}
+    for k in names:
+        g.set_option(k, saved[k])
+    assert _routes(g, u) == first
+    g.set_option("assembly.colouring", 1)
+    g.set_option("assembly.element_store", 0)
+    assert "k_gather_rows" not in _routes(g, u)
+    for k in names:
+        g.set_option(k, saved[k])
+    assert _routes(g, u) == first and {k: g.get_option(k) for k in names} == saved
+    g.close()
 
 
 def test_server_budget_without_scratch():

@@ -389,8 +389,10 @@ int  mhx_l2_error(mhx_ctx* ctx, const double* u, int32_t n_modes, const double* 
  *                         element matrices, then a sum per row (same sums
  *                         in the same order); 0: element colouring.
  *   "assembly.segment"    pencil streaming: elements per x-segment, even,
- *                         2 .. 4096 (default: from the mesh, so that the
- *                         workgroups fill the device evenly).
+ *                         2 .. 4096 (default: from the mesh and the kernel,
+ *                         so that the workgroups fill the device evenly;
+ *                         reading it gives the Jacobian's, and setting
+ *                         that value keeps the default).
  *   "krylov.spmv_lanes"   lanes that share one CRS row in the sparse
  *                         matrix-vector product: 4, 8, 16, 32 or 64 (default
  *                         chosen from the mean row length at context build;

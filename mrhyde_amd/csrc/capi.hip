@@ -1008,7 +1008,9 @@ int mhx_set_option(mhx_ctx* ctx, const char* name, int64_t value) {
       ctx->err = "assembly.segment must be an even element count in [2, 4096]";
       return MHX_ERR_ARG;
     }
-    ctx->q2_segment = (int)value;
+    // (the automatic length stays automatic: it follows the kernel that runs)
+    ctx->q2_segment = 0;
+    if (value != q2box_segment(*ctx, true)) ctx->q2_segment = (int)value;
     return MHX_OK;
   }
   if (k == "krylov.spmv_lanes") {

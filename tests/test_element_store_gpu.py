@@ -89,6 +89,27 @@ def test_assembly_options_survive_a_round_trip(kind):
     g.close()
 
 
+def test_segment_survives_a_round_trip():
+    """assembly.segment read and set to what was read stays automatic: it still
+    follows the kernel (sine modes leave room for fewer workgroups)."""
+    from mrhyde_amd import Mhx
+
+    modes = [(1.0, (np.pi, np.pi, np.pi))]
+    kw = dict(dim=3, order=2, quadrature=4, n=(192, 2, 6))
+    ref = {m: Mhx(Problem(**kw, modes=modes if m else [])).get_option("assembly.segment") for m in (False, True)}
+    assert ref[False] != ref[True], ref
+    g = Mhx(Problem(**kw))
+    g.set_option("assembly.segment", g.get_option("assembly.segment"))
+    g.update(Problem(**kw, modes=modes))
+    assert g.get_option("assembly.segment") == ref[True]
+    g.set_option("assembly.segment", 6)
+    assert g.get_option("assembly.segment") == 6
+    g.set_option("assembly.segment", ref[True])
+    g.update(Problem(**kw))
+    assert g.get_option("assembly.segment") == ref[False]
+    g.close()
+
+
 def test_server_budget_without_scratch():
     """A budget that holds a request only without the scratch memory still
     admits it, with the same bits."""

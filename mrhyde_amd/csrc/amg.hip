@@ -1120,6 +1120,7 @@ struct Amg {
   int sweeps = kBjSweeps;   // block-Jacobi sweeps before and after the coarse correction
   double omega = kBjOmega;  // block-Jacobi damping
   int nf = 1;
+  bool built = false;  // a set-up is complete
   int64_t setup_count = 0;
   int64_t reuse_count = 0;  // set-ups answered by refreshing the fine level only
 };
@@ -1234,7 +1235,7 @@ void amg_setup(Ctx& c, const double* A, bool fp32) {
   // set-up and refresh only what the fine-level smoother reads from the new
   // operator (its diagonal, or its nodal block inverses); the fine operator
   // itself is the new one, passed to every V-cycle
-  if (c.amg_reuse && H.setup_count > 0 && H.fp32 == fp32 && H.nf == nf && H.smoother == smoother &&
+  if (c.amg_reuse && H.built && H.fp32 == fp32 && H.nf == nf && H.smoother == smoother &&
       !H.lv.empty() && H.lv[0]->n == c.mesh.ndof) {
     AmgLevel& L0 = *H.lv[0];
     H.A0 = A;
@@ -1272,6 +1273,7 @@ void amg_setup(Ctx& c, const double* A, bool fp32) {
   H.omega = c.amg_omega_pct * 0.01;
   H.nf = nf;
   ++H.setup_count;
+  H.built = false;  // (until the end: a set-up that fails leaves nothing to reuse)
 
   // level 0: the context's lattice and pattern
   int nlev = 0;
@@ -1440,6 +1442,7 @@ void amg_setup(Ctx& c, const double* A, bool fp32) {
     }
   }
   MHX_HIP(hipGetLastError());
+  H.built = true;
 }
 
 // Chebyshev coefficients of one level (Ifpack2's three-term recurrence)

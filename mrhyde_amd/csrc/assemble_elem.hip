@@ -187,7 +187,8 @@ const Entry kStoreTable[] = {
 // The gain shrinks as the round trip of the element matrices leaves the caches;
 // past the largest size measured the scratch memory (1.35 times the Jacobian in
 // 3-D Q2) is not spent.  It is allocated with the context, so no assembly
-// allocates.
+// allocates, given back when an option or a time state takes the assembly
+// elsewhere, and for a solve that would otherwise run out of memory.
 int64_t element_store_doubles(const mhx_problem_desc& d) {
   if (d.physics != MHX_PHYS_THERMAL || d.n_functions > 0) return 0;
   // boxes at three points per axis: the row-owned kernel (assemble_q2box.hip)
@@ -208,7 +209,37 @@ int64_t element_store_bytes(const mhx_problem_desc& d) {
   return 8 * n + 8 * n / (d.dim == 3 ? p1 * p1 * p1 : p1 * p1);
 }
 
+bool element_store_release(Ctx& c) {
+  if (!c.escr.p || c.store_captured) return false;
+  (void)hipStreamSynchronize(c.stream);
+  c.escr.release();
+  c.rscr.release();
+  return true;
+}
+
+void element_store_fit(Ctx& c) {
+  const int64_t n = c.store_on && c.scatter_mode == kElementColouring && c.bdf_order == 0 && !c.xh.active
+                        ? element_store_doubles(c.desc)
+                        : 0;
+  if (!n) {
+    (void)element_store_release(c);
+  } else if (!c.escr.p) {
+    try {
+      c.rscr.alloc((size_t)c.mesh.ne * c.nb);
+      c.escr.alloc((size_t)n);
+    } catch (const Error&) {  // no room: element colouring
+      (void)hipGetLastError();
+      c.rscr.release();
+    }
+  }
+}
+
 void launch_element_store(Ctx& c, AsmArgs& a, bool jac) {
+  if (!c.store_captured) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c.stream, &cap) != hipSuccess) (void)hipGetLastError();
+    c.store_captured = cap != hipStreamCaptureStatusNone;
+  }
   a.escr = c.escr.p;
   a.rscr = c.rscr.p;
   a.blocked = 0;

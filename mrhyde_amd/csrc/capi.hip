@@ -132,7 +132,7 @@ struct VecArg {
     if (device) {
       dev = const_cast<double*>(p);
     } else {
-      stage.alloc(std::max<size_t>(n, 1));
+      or_without_store(c, [&] { stage.alloc(std::max<size_t>(n, 1)); });
       dev = stage.p;
       if (copy_in && p) MHX_HIP(hipMemcpyAsync(dev, p, n * sizeof(double), hipMemcpyHostToDevice, c.stream));
     }
@@ -270,10 +270,12 @@ __global__ __launch_bounds__(256) void k_copy_probe(int64_t n, const double* __r
 // ---- Newton (SolverManager::nonlinearSolver, solverManager_solvers.hpp:290-643) --
 static int newton(Ctx& c, double* u, const mhx_newton_opts& o, mhx_solve_stats* st) {
   const long n = c.mesh.ndof;
-  c.res.alloc(n);
-  c.jac.alloc(c.nnz);
-  c.aux.alloc(n);
-  c.du.alloc(n);
+  or_without_store(c, [&] {
+    c.res.alloc(n);
+    c.jac.alloc(c.nnz);
+    c.aux.alloc(n);
+    c.du.alloc(n);
+  });
   DevBuf<double>& du = c.du;
   MHX_HIP(hipMemsetAsync(du.p, 0, n * sizeof(double), c.stream));
   double first = 0.0, alpha = 1.0;
@@ -374,20 +376,13 @@ int mhx::ctx_create(const mhx_problem_desc* desc, bool element_store, mhx_ctx** 
   // thermal assembly then defaults to the row-owned kernel (k_q2box)
   c->box_mesh = desc->perturb == 0.0;
   if (q2box_applicable(*c)) c->scatter_mode = kPencilStream;
-  // small general meshes: element matrices to scratch (now, so that no
-  // assembly allocates), rows gathered
-  if (const int64_t ed = element_store ? element_store_doubles(*desc) : 0) {
-    try {
-      c->rscr.alloc((size_t)c->mesh.ne * c->nb);
-      c->escr.alloc((size_t)ed);
-    } catch (const Error&) {  // no room: element colouring
-      (void)hipGetLastError();
-      c->rscr.release();
-    }
-  }
   // Navier-Stokes: x-segments merged in LDS (each row's x-runs written once
   // per segment) by default
   if (desc->physics == MHX_PHYS_NAVIER_STOKES) c->scatter_mode = kSegmentMerge;
+  // small general meshes: element matrices to scratch (now, so that no
+  // assembly allocates), rows gathered
+  c->store_on = element_store;
+  element_store_fit(*c);
   c->desc.k0 = nullptr;
   c->desc.src_elem = nullptr;
   c->desc.dbc_values = nullptr;
@@ -524,7 +519,7 @@ int mhx_spmv(mhx_ctx* ctx, const double* jac_vals, const double* x, double* y, i
     if (dev) {
       A = jac_vals;
     } else {
-      jstage.alloc(ctx->nnz);
+      or_without_store(*ctx, [&] { jstage.alloc(ctx->nnz); });
       MHX_HIP(hipMemcpyAsync(jstage.p, jac_vals, ctx->nnz * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
       A = jstage.p;
     }
@@ -553,7 +548,7 @@ int mhx_linear_solve(mhx_ctx* ctx, const double* jac_vals, const double* r, doub
     if (dev) {
       A = jac_vals;
     } else {
-      jstage.alloc(ctx->nnz);
+      or_without_store(*ctx, [&] { jstage.alloc(ctx->nnz); });
       MHX_HIP(hipMemcpyAsync(jstage.p, jac_vals, ctx->nnz * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
       A = jstage.p;
     }
@@ -625,6 +620,7 @@ static void set_stage_state(Ctx& c, double dt, int32_t bdf_order, const double* 
     c.alpha_t = 0.0;
     c.alpha_u = 1.0;
     c.hist_u.release();
+    element_store_fit(c);
     return;
   }
   MHX_REQUIRE(c.desc.physics == MHX_PHYS_THERMAL, MHX_ERR_UNSUPPORTED, "time integration is built for the thermal module");
@@ -645,6 +641,7 @@ static void set_stage_state(Ctx& c, double dt, int32_t bdf_order, const double* 
       {25.0 / 12.0, -4.0, 3.0, -4.0 / 3.0, 1.0 / 4.0},
       {137.0 / 60.0, -5.0, 5.0, -10.0 / 3.0, 75.0 / 60.0, -1.0 / 5.0},
       {147.0 / 60.0, -6.0, 15.0 / 2.0, -20.0 / 3.0, 225.0 / 60.0, -72.0 / 60.0, 1.0 / 6.0}};
+  (void)element_store_release(c);  // (the transient kernel runs element colouring)
   const long n = c.mesh.ndof;
   const bool dev = (flags & MHX_DEVICE_PTRS) != 0;
   const double* prev = u_prev;
@@ -746,7 +743,7 @@ int mhx_amg_setup(mhx_ctx* ctx, const double* jac_vals, int32_t flags) {
     if (flags & MHX_DEVICE_PTRS) {
       A = jac_vals;
     } else {
-      jstage.alloc(ctx->nnz);
+      or_without_store(*ctx, [&] { jstage.alloc(ctx->nnz); });
       MHX_HIP(hipMemcpyAsync(jstage.p, jac_vals, ctx->nnz * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
       A = jstage.p;
     }
@@ -754,7 +751,7 @@ int mhx_amg_setup(mhx_ctx* ctx, const double* jac_vals, int32_t flags) {
     MHX_REQUIRE(ctx->jac_valid && ctx->jac.p, MHX_ERR_STATE, "no Jacobian held by the context");
     A = ctx->jac.p;
   }
-  amg_setup(*ctx, A, false);
+  or_without_store(*ctx, [&] { amg_setup(*ctx, A, false); });
   MHX_HIP(hipStreamSynchronize(ctx->stream));
   return amg_levels(*ctx);
   MHX_GUARD_END(ctx)
@@ -993,6 +990,7 @@ int mhx_set_option(mhx_ctx* ctx, const char* name, int64_t value) {
       return MHX_ERR_ARG;
     }
     ctx->scatter_mode = (int)value;
+    element_store_fit(*ctx);
     return MHX_OK;
   }
   if (k == "assembly.element_store") {
@@ -1001,6 +999,7 @@ int mhx_set_option(mhx_ctx* ctx, const char* name, int64_t value) {
       return MHX_ERR_ARG;
     }
     ctx->store_on = value != 0;
+    element_store_fit(*ctx);
     return MHX_OK;
   }
   if (k == "assembly.segment") {
@@ -1124,7 +1123,7 @@ int mhx_state_ptr(mhx_ctx* ctx, int32_t which, double** dev_ptr, int64_t* count)
   size_t n = 0;
   DevBuf<double>& b = state_buf(ctx, which, n);
   if (b.n != n) {
-    b.alloc(n);
+    or_without_store(*ctx, [&] { b.alloc(n); });
     MHX_HIP(hipMemsetAsync(b.p, 0, n * sizeof(double), ctx->stream));
     MHX_HIP(hipStreamSynchronize(ctx->stream));
   }
@@ -1140,7 +1139,7 @@ int mhx_state_upload(mhx_ctx* ctx, int32_t which, const double* host, int64_t co
   size_t n = 0;
   DevBuf<double>& b = state_buf(ctx, which, n);
   MHX_REQUIRE((size_t)count == n, MHX_ERR_ARG, "count does not match the buffer size");
-  if (b.n != n) b.alloc(n);
+  if (b.n != n) or_without_store(*ctx, [&] { b.alloc(n); });
   MHX_HIP(hipMemcpyAsync(b.p, host, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
   MHX_HIP(hipStreamSynchronize(ctx->stream));
   return MHX_OK;

@@ -1438,13 +1438,17 @@ int krylov_solve(Ctx& c, const double* A, const double* b, double* x, const mhx_
   int it, refs = 0;
   const int maxit = o.max_iters > 0 ? o.max_iters : 100;
   const double tol = o.tol > 0 ? o.tol : 1e-7;
-  if (o.precond & MHX_PREC_FP32) {
-    it = mixed_solve(c, A, b, x, o, maxit, tol, &rel, &refs);
-  } else {
-    const Prec<double> P = build_prec<double>(c, A, pk, c.kw.d);
-    if (o.solver == MHX_KRYLOV_CG) it = cg_core<double>(c, A, P, b, x, tol, maxit, &rel);
-    else it = gmres_core<double>(c, A, P, b, x, o.restart > 0 ? o.restart : 50, tol, maxit, &rel);
-  }
+  // (every allocation comes before the first change of x)
+  or_without_store(c, [&] {
+    refs = 0;
+    if (o.precond & MHX_PREC_FP32) {
+      it = mixed_solve(c, A, b, x, o, maxit, tol, &rel, &refs);
+    } else {
+      const Prec<double> P = build_prec<double>(c, A, pk, c.kw.d);
+      if (o.solver == MHX_KRYLOV_CG) it = cg_core<double>(c, A, P, b, x, tol, maxit, &rel);
+      else it = gmres_core<double>(c, A, P, b, x, o.restart > 0 ? o.restart : 50, tol, maxit, &rel);
+    }
+  });
   if (st) {
     st->iters += it;
     st->rel_res = rel;

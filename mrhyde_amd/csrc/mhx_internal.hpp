@@ -239,6 +239,7 @@ struct Ctx {
   int nfield = 1;  // unknowns per node (consecutive DOFs): block size of block Jacobi
   int scatter_mode = kElementColouring;
   bool store_on = true;       // assembly.element_store
+  bool store_captured = false;  // a captured graph holds escr's and rscr's addresses
   DevBuf<double> escr, rscr;  // element matrices and residuals (allocated where the element store applies)
   bool box_mesh = false;  // every element an axis-aligned box (structured box, no node perturbation)
   int q2_segment = 0;     // pencil streaming: elements per x-segment (even; 0: chosen per launch)
@@ -273,6 +274,24 @@ int q2box_segment(const Ctx& c, bool jac);  // elements per x-segment of a launc
 // residuals; and its launches
 int64_t element_store_doubles(const mhx_problem_desc& d);
 int64_t element_store_bytes(const mhx_problem_desc& d);
+// The scratch memory is held while the context's steady assembly uses it: take
+// it if it does (without, where there is no room) and give it back if not;
+// give it back in any case, true if there was any (both: not while a captured
+// graph holds its address)
+void element_store_fit(Ctx& c);
+bool element_store_release(Ctx& c);
+// f(c) with the scratch memory given back and f run again where memory runs
+// out; f must not have changed its results before it allocates
+template <class F>
+auto or_without_store(Ctx& c, F&& f) -> decltype(f()) {
+  try {
+    return f();
+  } catch (const Error& e) {
+    if (e.code != MHX_ERR_NOMEM || !element_store_release(c)) throw;
+    (void)hipGetLastError();
+  }
+  return f();
+}
 // mhx_ctx_create; element_store = false leaves its scratch memory out
 int ctx_create(const mhx_problem_desc* desc, bool element_store, mhx_ctx** out);
 void launch_element_store(Ctx& c, AsmArgs& a, bool jac);

@@ -99,3 +99,54 @@ def test_batch_rejects_bad_boxes():
         SubgridBatch(np.array([2], dtype=np.int32), k, g, extent=[[1.0, 0.0, 1.0]])
     with pytest.raises(ValueError):
         SubgridBatch(np.array([2], dtype=np.int32), k, g, src=np.ones(7))
+
+
+RECLAIM = r"""
+#include <cstdio>
+#include "mhx_internal.hpp"
+using namespace mhx;
+static int calls;
+static int once() {
+  if (++calls == 1) throw Error{MHX_ERR_NOMEM, "first"};
+  return calls;
+}
+static int code_of(Ctx& c, int (*f)()) {
+  try {
+    or_without_store(c, f);
+  } catch (const Error& e) {
+    return e.code;
+  }
+  return 0;
+}
+int main() {
+  Ctx c;
+  auto hold = [&] { c.escr.p = c.rscr.p = (double*)4096, calls = 0; };
+  hold();  // memory runs out: the scratch goes, the call runs again
+  if (or_without_store(c, once) != 2 || c.escr.p || c.rscr.p) return 1;
+  calls = 0;  // nothing to give back
+  if (code_of(c, once) != MHX_ERR_NOMEM || calls != 1) return 2;
+  hold();  // a captured graph holds the address
+  c.store_captured = true;
+  if (code_of(c, once) != MHX_ERR_NOMEM || calls != 1 || !c.escr.p) return 3;
+  c.store_captured = false;  // another error
+  if (code_of(c, [] { return throw Error{MHX_ERR_ARG, ""}, 0; }) != MHX_ERR_ARG || !c.escr.p) return 4;
+  c.escr.p = c.rscr.p = nullptr;
+  return 0;
+}
+"""
+
+
+def test_scratch_is_given_back_where_memory_runs_out():
+    """The optional scratch memory of the two-launch assembly goes, and the call
+    runs again, before an allocation that a solve needs is reported as failed
+    (host code against the library; the addresses are not device memory)."""
+    from mrhyde_amd import build
+
+    with tempfile.TemporaryDirectory() as d:
+        src, exe = os.path.join(d, "r.cpp"), os.path.join(d, "r")
+        open(src, "w").write(RECLAIM)
+        rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+        subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include", f"-I{build.ROOT}/include",
+                        f"-I{build.CSRC}", src, "-o", exe, str(build.OUT), f"-L{rocm}/lib", "-lamdhip64",
+                        f"-Wl,-rpath,{build.PKG}:{rocm}/lib"], check=True)
+        assert subprocess.run([exe]).returncode == 0

@@ -89,6 +89,82 @@ def test_assembly_options_survive_a_round_trip(kind):
     g.close()
 
 
+def _free():
+    import torch
+
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+def test_scratch_is_held_only_while_the_assembly_uses_it():
+    """512^2 Q1: 40 MiB.  Another route or a time state gives them back, the way
+    back to the steady default takes them again, with the same sums throughout."""
+    from mrhyde_amd import Mhx
+
+    g = Mhx(Problem(dim=2, order=1, quadrature=2, n=(512, 512), k0=np.linspace(1, 2, 512 * 512)))
+    u = np.random.default_rng(1).standard_normal(g.n_dof)
+    r, j = g.assembleJacRes(u)
+    g.set_time_state(0.1, 1, [u])  # (the time state's own buffers, which it keeps)
+    g.set_time_state(0.1, 0)
+    size, held = 512 * 512 * (16 + 4) * 8, _free()
+    steps = [(("assembly.colouring", 1), ("assembly.colouring", 0)),
+             (("assembly.element_store", 0), ("assembly.element_store", 1))]
+    for off, on in steps:
+        g.set_option(*off)
+        assert _free() >= held + size
+        ro, jo = g.assembleJacRes(u)
+        assert np.abs(ro - r).max() <= 4e-14 * np.abs(r).max() and np.abs(jo - j).max() <= 4e-14 * np.abs(j).max()
+        g.set_option(*on)
+        assert _free() < held + size
+        rn, jn = g.assembleJacRes(u)
+        np.testing.assert_array_equal(rn, r), np.testing.assert_array_equal(jn, j)
+    g.set_time_state(0.1, 1, [u])
+    assert _free() >= held + size
+    g.assembleJacRes(u)
+    g.set_time_state(0.1, 0)
+    assert _free() < held + size
+    np.testing.assert_array_equal(g.assembleJacRes(u)[1], j)
+    g.close()
+
+
+def test_captured_assembly_keeps_its_scratch():
+    """A captured graph holds the scratch memory's address: the memory stays
+    while options and the time state change, and replays keep their results."""
+    import torch
+
+    from mrhyde_amd import Mhx
+
+    g = Mhx(Problem(dim=2, order=2, quadrature=4, n=(24, 17), perturb=0.1, perturb_seed=2, diff_u2=0.5))
+    rng = np.random.default_rng(2)
+    u = torch.from_numpy(rng.standard_normal(g.n_dof)).cuda()
+    res, jac = torch.zeros(g.n_dof, dtype=torch.float64).cuda(), torch.zeros(g.nnz, dtype=torch.float64).cuda()
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        g.assemble(u, res, jac)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        g.assemble(u, res, jac)
+    for change in (None, ("assembly.colouring", 1), ("assembly.element_store", 0), "time"):
+        if change == "time":
+            g.set_time_state(0.1, 1, [u.cpu().numpy()])
+        elif change:
+            g.set_option(*change)
+        u.copy_(torch.from_numpy(rng.standard_normal(g.n_dof)))
+        filler = [torch.full((1 << 20,), float("nan"), dtype=torch.float64, device="cuda") for _ in range(4)]
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        f = Mhx(Problem(dim=2, order=2, quadrature=4, n=(24, 17), perturb=0.1, perturb_seed=2, diff_u2=0.5))
+        r, j = f.assembleJacRes(u.cpu().numpy())
+        f.close()
+        np.testing.assert_array_equal(res.cpu().numpy(), r)
+        np.testing.assert_array_equal(jac.cpu().numpy(), j)
+        del filler
+    g.close()
+
+
 def test_segment_survives_a_round_trip():
     """assembly.segment read and set to what was read stays automatic: it still
     follows the kernel (sine modes leave room for fewer workgroups)."""

@@ -64,7 +64,8 @@ struct Request {
   std::vector<const char*> fn_name_p, fn_expr_p;
   Key key;
   int64_t n_dof = 0, bytes = 0;
-  bool element_store = true;  // the context gets the scratch memory of the two-launch assembly
+  int64_t store_bytes = 0;    // of these, the optional scratch memory of the two-launch assembly
+  bool element_store = true;  // the context gets it
   clk::time_point t_submit, t_start, t_end;
   bool done = false;
   int status = MHX_OK;
@@ -109,16 +110,24 @@ struct mhx_server {
           ++n_reused;
           return r;
         }
+      // a request does without its scratch memory (same results) before
+      // another context is evicted, or it or a queued one that a worker is
+      // free for has to wait
+      const int64_t need = r->bytes - r->store_bytes;
       int64_t freeable = 0;
       for (const Slot& s : idle) freeable += s.bytes;
-      if (used + r->bytes <= d.hbm_budget || used - freeable + r->bytes <= d.hbm_budget) {
-        while (used + r->bytes > d.hbm_budget && !idle.empty()) {
+      if (used - freeable + need <= d.hbm_budget) {
+        while (used + need > d.hbm_budget && !idle.empty()) {
           used -= idle.front().bytes;
           drop.push_back(idle.front().ctx);
           idle.pop_front();
         }
-        slot = Slot{r->key, nullptr, r->bytes, clk::now()};
-        used += r->bytes;
+        int64_t next = 0, free_workers = d.max_active - n_active - 1;
+        for (const Request* q : queue)
+          if (q != r && free_workers-- > 0) next += q->bytes - q->store_bytes;
+        r->element_store = used + r->bytes + next <= d.hbm_budget;
+        slot = Slot{r->key, nullptr, r->element_store ? r->bytes : need, clk::now()};
+        used += slot.bytes;
         queue.erase(it);
         return r;
       }
@@ -231,11 +240,8 @@ int mhx_server_submit(mhx_server* s, const mhx_problem_desc* desc, int64_t* tick
   int64_t nnz = 0;
   int rc = mhx_footprint(desc, &s->d.newton.linear, &r->n_dof, &nnz, &r->bytes);
   if (rc != MHX_OK) return rc;
-  if (r->bytes > s->d.hbm_budget) {  // do without the optional scratch memory (same results)
-    r->element_store = false;
-    r->bytes -= element_store_bytes(*desc);
-  }
-  if (r->bytes > s->d.hbm_budget) return MHX_ERR_NOMEM;  // could never be admitted
+  r->store_bytes = element_store_bytes(*desc);
+  if (r->bytes - r->store_bytes > s->d.hbm_budget) return MHX_ERR_NOMEM;  // could never be admitted
   r->desc = *desc;
   long ne = (long)desc->nx * desc->ny * (desc->dim == 3 ? desc->nz : 1);
   if (desc->k0) {

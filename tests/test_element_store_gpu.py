@@ -199,3 +199,23 @@ def test_server_budget_without_scratch():
         xs.append(s.poll(s.submit(p))[0])
         s.close()
     np.testing.assert_array_equal(xs[0], xs[1])
+
+
+def test_server_evicts_nothing_for_scratch():
+    """A budget that holds two contexts only if one does without its scratch
+    memory keeps both: the third request finds the first one's context."""
+    from mrhyde_amd import Server
+
+    a = Problem(dim=3, order=1, quadrature=2, n=(12, 11, 10), modes=[(1.0, (np.pi, np.pi, np.pi))])
+    b = Problem(dim=3, order=1, quadrature=2, n=(11, 11, 10), modes=[(1.0, (np.pi, np.pi, np.pi))])
+    s = Server(max_active=1, max_cached=4)
+    alone = s.poll(s.submit(b))[0]
+    s.close()
+    s = Server(max_active=1, max_cached=4, hbm_budget=Server.footprint(a)[2] + Server.footprint(b)[2] - 8)
+    s.poll(s.submit(a))
+    x = s.poll(s.submit(b))[0]
+    s.poll(s.submit(a))
+    info = s.info()
+    assert info["created"] == 2 and info["reused"] == 1 and info["bytes_held"] <= info["budget"], info
+    np.testing.assert_array_equal(x, alone)
+    s.close()

@@ -79,7 +79,7 @@ struct StoreRow {
   T* __restrict__ y;
   struct Pre {};
   __device__ __forceinline__ Pre load(long) const { return {}; }
-  __device__ __forceinline__ void operator()(long row, T v, Pre) const { y[row] = v; }
+  __device__ __forceinline__ void operator()(long row, double v, Pre) const { y[row] = (T)v; }
 };
 
 template <class T>
@@ -100,8 +100,10 @@ static void spmv_t(Ctx& c, const TA* A, const TX* s, const TX* x, TX* y) {
       return;
     }
   }
+  // (sums in FP64, also of FP32 products: a lane's chain here is longer than in
+  // k_spmv, 25 terms against 16; same time, 64^3 Q2 372 us an iteration)
   if (!s && q2_product_applies(c)) {
-    q2_product<TX>(c, A, x, StoreRow<TX>{y});
+    q2_product<double>(c, A, x, StoreRow<TX>{y});
     return;
   }
   long n = c.mesh.ndof;
@@ -688,7 +690,9 @@ __global__ __launch_bounds__(256) void k_cg_update(long n, const double* __restr
 // chunk ahead.  Rows are padded with zeros to a multiple of kCgWgChunk entries.
 // 64^2 Q1: 8 us an iteration, most of it that stream through one CU; a whole
 // Newton solve 5.1 -> 3.3 ms.  With the CRS rows dealt to four lanes each an
-// iteration took 11 us, without the chunk ahead 8.6.
+// iteration took 11 us, without the chunk ahead 8.6.  FP32 entries (the inner
+// solves of refinement) are summed in FP64, since a row is one chain here:
+// 6.0 us an iteration, in FP32 5.2 at up to 1.5 times the error of four lanes.
 // The two sums per iteration meet in LDS (four 16-lane rows a wavefront) and are
 // added in the same order by every thread, so all agree on each branch.
 constexpr int kCgWgRows = 5;          // rows a thread can own
@@ -797,6 +801,7 @@ __global__ __launch_bounds__(1024) void k_cg_wg(int n, int W, const int32_t* __r
     for (int i = 0; i < R; ++i) {
       q[i] = 0;
       if (i * 1024 < n) {
+        double sum = 0.0;  // (the whole row in one chain: FP64 also for FP32 entries)
         const unsigned row = own_row(i);
         const uint32_t* ck = s_ci + row;
         for (int k = 0; k < W; k += C, ck += C / 2 * n) {
@@ -814,10 +819,11 @@ __global__ __launch_bounds__(1024) void k_cg_wg(int n, int W, const int32_t* __r
           for (int j = 0; j < C / 2; ++j) o[j] = ck[j * n];
 #pragma unroll
           for (int j = 0; j < C / 2; ++j) {
-            q[i] = fma(a[2 * j], *(const T*)(s_pb + (o[j] & 0xffff)), q[i]);
-            q[i] = fma(a[2 * j + 1], *(const T*)(s_pb + (o[j] >> 16)), q[i]);
+            sum = fma((double)a[2 * j], (double)*(const T*)(s_pb + (o[j] & 0xffff)), sum);
+            sum = fma((double)a[2 * j + 1], (double)*(const T*)(s_pb + (o[j] >> 16)), sum);
           }
         }
+        q[i] = (T)sum;
         if (i * 1024 + t < n) pq = fma((double)s_p[row], (double)q[i], pq);
       }
     }

@@ -698,6 +698,7 @@ __global__ __launch_bounds__(256) void k_cg_update(long n, const double* __restr
 constexpr int kCgWgRows = 5;          // rows a thread can own
 constexpr int kCgWgChunk = 10;        // entries loaded together
 constexpr int kCgWgLds = 150 * 1024;  // p and the offsets
+constexpr int kCgWgRowBytes = 130 * 8;  // values of a padded row (see the rule)
 constexpr int kCgWgIters = 512;       // iterations a launch runs at most
 
 __device__ __forceinline__ double row16_sum(double v) {
@@ -860,14 +861,21 @@ __global__ __launch_bounds__(1024) void k_cg_wg(int n, int W, const int32_t* __r
 }
 
 // The one-workgroup form takes the systems whose p and offsets fit its LDS (2-D
-// Q1 to 70^2, 3-D Q1 to 12^3), without a preconditioner or with the diagonal
-// one.  Row length of its copy of the matrix, 0 where it does not apply.
+// Q1 to 70^2, 3-D Q1 to 12^3, 2-D Q2 to 23^2), without a preconditioner or with
+// the diagonal one, and whose rows are short enough: its time grows with the
+// row, which one thread walks, that of the two launches hardly.  FP64 us an
+// iteration, one workgroup / two launches: Q1 16^2 3.5/12.0, 70^2 8.4/13.0, 12^3
+// 12.8/14.1; 2-D Q2 23^2 12.4/13.5; Q3 12^2 13.4/14.0; Q4 (rows padded to 90) 6^2
+// 12.2/15.4; Q5 (130) 4^2 16.5/16.3, 3-D Q2 (130) 3^3 17.3/17.4, 4x4x3 17.1/18.2;
+// Q6 (170) 3^2 20.8/14.8; FP32 wins at every length (Q6 13.1/15.1).  Row length
+// of its copy of the matrix, 0 where it does not apply.
 template <class T>
 static int cg_one_workgroup(const Ctx& c, int precond, long n) {
   if ((precond != MHX_PREC_NONE && precond != MHX_PREC_JACOBI) || n > 1024 * kCgWgRows) return 0;
   long W = c.mesh.nf;
   for (int d = 0; d < c.mesh.dim; ++d) W *= std::min(2 * c.mesh.p, c.mesh.p * c.mesh.nel[d]) + 1;
   W = (W + kCgWgChunk - 1) / kCgWgChunk * kCgWgChunk;
+  if ((long)sizeof(T) * W > kCgWgRowBytes) return 0;
   return ((long)sizeof(T) + 2 * W) * n + 8 <= kCgWgLds ? (int)W : 0;
 }
 

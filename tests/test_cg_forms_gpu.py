@@ -62,3 +62,27 @@ def test_matches_numpy(order, n, precond):
         assert abs(st["iters"] - it) <= 2 + it // 50
         assert np.linalg.norm(b - A @ x) <= 1.01e-9 * np.linalg.norm(b)
     g.close()
+
+
+@pytest.mark.parametrize("order,n", [(4, (6, 6)), (5, (4, 4)), (6, (3, 3)), (6, (2, 3))],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else f"p{v}")
+def test_long_rows_match_numpy(order, n):
+    """Rows of 81 to 169 entries, on both sides of the longest that one
+    workgroup takes: the iterate after 7 iterations, and the solution."""
+    from mrhyde_amd import Mhx
+
+    print(f"[cg] p{order} {n} jacobi", flush=True)
+    rng = np.random.default_rng(order + sum(n))
+    g = Mhx(Problem(dim=2, order=order, quadrature=2 * order, n=n, k0=np.exp(0.3 * rng.standard_normal(np.prod(n))),
+                    dbc_sides=1))
+    _, j = g.assembleJacRes(np.zeros(g.n_dof))
+    rp, ci = g.crs_pattern()
+    A = sp.csr_matrix((j, ci, rp), shape=(g.n_dof, g.n_dof))
+    b = rng.standard_normal(g.n_dof)
+    b[np.asarray(g.dirichlet_mask(), bool)] = 0.0
+    ref, it = pcg(A, b, A.diagonal(), 1e-14, 7)
+    x, st = g.linearSolver(j, b, solver="cg", precond="jacobi", tol=1e-14, max_iters=it)
+    assert np.abs(x - ref).max() <= 1e-10 * np.abs(ref).max()
+    x, st = g.linearSolver(j, b, solver="cg", precond="jacobi", tol=1e-9, max_iters=3000)
+    assert np.linalg.norm(b - A @ x) <= 1.01e-9 * np.linalg.norm(b)
+    g.close()

@@ -1,9 +1,10 @@
-"""CPU replay of the assembly kernels' scatter schedules (k_thermal, k_ns).
+"""CPU replay of the assembly kernels' scatter schedules (k_thermal, k_ns) and
+of the kernels that own their rows (k_q2box, k_q2res, k_gather_rows: at the end).
 
-The three schedules of `assembly.colouring` are restated here from the kernel's
-index arithmetic (lattice.hpp `element_of`, `element_of_seg`, `axis_key`;
-assemble.hip `launch_colors`, the first-touch flags and the x-segment LDS image)
-and replayed on small lattices:
+The three scattering schedules of `assembly.colouring` are restated here from
+the kernel's index arithmetic (lattice.hpp `element_of`, `element_of_seg`,
+`axis_key`; assemble.hip `launch_colors`, the first-touch flags and the x-segment
+LDS image) and replayed on small lattices:
 
 * every element is assembled exactly once;
 * race freedom: two work units that may run at the same time never write the
@@ -408,185 +409,212 @@ def test_segment_loops_visit_every_slot_once(dim, p, block):
 
 
 # ---------------------------------------------------------------------------
-# pencil streaming (assemble_q2box.hip, assembly.colouring = 3, Q2 hexahedra):
-# a 64-lane wavefront walks an x-segment of one element pencil two elements
-# per step.  Restated from the kernel's round / lane arithmetic: every write
-# is (entry, contributing elements, first-touch flag); the replay checks that
-# each CRS entry receives the contribution of every element holding both of
-# its nodes exactly once, has exactly one first writer that runs before all
-# other writers, and that no two writers of an entry can run at once.
+# row-owned kernels (one writer per row, one launch): assemble_q2box.hip
+# (assembly.colouring = 3, Q2 hexahedra on boxes), assemble_q2res.hip (its
+# residual alone) and the row gather of assemble_elem.hip.  Restated from the
+# kernels' lane arithmetic: every write is (CRS position or row, contributing
+# elements in the order of the sums).  The replay checks that every entry of the
+# CRS pattern is written once, at its position, with the contribution of every
+# element that holds both of its nodes exactly once.
 # ---------------------------------------------------------------------------
-def pencil_units(nel, seg):
-    nseg = (nel[0] + seg - 1) // seg
-    for col in range(8):
-        cx, cy, cz = col & 1, (col >> 1) & 1, (col >> 2) & 1
-        cn = [(nseg - cx + 1) // 2, (nel[1] - cy + 1) // 2, (nel[2] - cz + 1) // 2]
-        for t in range(cn[0] * cn[1] * cn[2]):
-            tt = t
-            sx = 2 * (tt % cn[0]) + cx
-            tt //= cn[0]
-            ey = 2 * (tt % cn[1]) + cy
-            tt //= cn[1]
-            ez = 2 * tt + cz
-            yield col, t, sx, ey, ez, nseg
+def node_elems(node, nel, p=2):
+    """Elements holding a lattice node."""
+    rng = []
+    for c, n in zip(node, nel):
+        cand = [c // p - 1, c // p] if c % p == 0 else [c // p]
+        rng.append([e for e in cand if 0 <= e < n])
+    return sorted(itertools.product(*rng))
 
 
-def pencil_writes(nel, seg):
-    """[(launch, wg, entry, contributors, first)] for the Jacobian and
-    [(launch, wg, row, contributors, first)] for the residual."""
-    nn = [2 * n + 1 for n in nel]
+def axis_row(c, n, p=2):
+    """First column and number of columns of lattice coordinate c."""
+    if c % p:
+        return c - c % p, p + 1
+    lo, hi = max(c - p, 0), min(c + p, p * n)
+    return lo, hi - lo + 1
+
+
+def crs(nel, p=2):
+    """Positions of all entries: {(row node, column node): position}, x fastest."""
+    nn = [p * n + 1 for n in nel]
+    pos, k = {}, 0
+    for Z, Y, X in itertools.product(*(range(m) for m in reversed(nn))):
+        box = [range(lo, lo + ln) for lo, ln in (axis_row(c, n, p) for c, n in zip((X, Y, Z), nel))]
+        for z, y, x in itertools.product(*reversed(box)):
+            pos[((X, Y, Z), (x, y, z))] = k
+            k += 1
+    return pos
+
+
+def q2_prefix(X):
+    e = X >> 1
+    return (3 if e == 0 else 8 * e + 3) if X & 1 else (0 if e == 0 else 8 * e - 2)
+
+
+def q2box_writes(nel, seg):
+    """Writes of k_q2box: [(CRS position, contributing elements)], [(row node, contributing elements)]."""
+    n0, n1, n2 = nel
+    N1, N2 = 2 * n1 + 1, 2 * n2 + 1
+    T0, T1 = 8 * n0 + 1, 8 * n1 + 1
+    nseg, cn1, cn2 = -(-n0 // seg), (n1 + 2) // 2, (n2 + 2) // 2
     jw, rw = [], []
-    for col, wg, sx, ey, ez, nseg in pencil_units(nel, seg):
-        x0 = sx * seg
-        x1 = min(x0 + seg, nel[0])
-        flx, fhx = sx == 0 or sx % 2 == 0, sx == nseg - 1 or sx % 2 == 0
-        fly, fhy = ey == 0 or ey % 2 == 0, ey == nel[1] - 1 or ey % 2 == 0
-        flz, fhz = ez == 0 or ez % 2 == 0, ez == nel[2] - 1 or ez % 2 == 0
-        Y0, Z0 = 2 * ey, 2 * ez
-        carry = {}   # (r, l) -> contributions of B's last-plane run, by column
-        rcarry = {}  # l -> residual contributions
-        for xa in range(x0, x1, 2):
-            hasB = xa + 1 < x1
-            first_step, last_step = xa == x0, xa + 2 >= x1
-            el = {0: (xa, ey, ez), 1: (xa + 1, ey, ez)}
-            # residual (lane l < 27 of half h: test function i = l)
-            R = {}
-            for h in (0, 1):
-                if h == 1 and not hasB:
-                    continue
-                for l in range(27):
-                    R[(h, l)] = [el[h]]
-            newr = {}
-            for h in (0, 1):
-                if h == 1 and not hasB:
-                    continue
-                ex = xa + h
-                for l in range(27):
-                    i1, i2, i3 = l % 3, (l // 3) % 3, l // 9
-                    X = 2 * ex + i1
-                    contrib = list(R[(h, l)])
-                    write, xsh, xfirst = True, False, True
-                    if h == 0 and i1 == 2:
-                        if hasB:
-                            contrib = contrib + R[(1, l - 2)]
-                        elif x1 < nel[0]:
-                            xsh, xfirst = True, fhx
-                    elif h == 0 and i1 == 0:
-                        if not first_step:
-                            contrib = rcarry[l + 2] + contrib
-                        elif x0 > 0:
-                            xsh, xfirst = True, flx
-                    elif h == 1 and i1 == 0:
-                        write = False
-                    elif h == 1 and i1 == 2:
-                        newr[l] = contrib
-                        write = last_step
-                        if last_step and x1 < nel[0]:
-                            xsh, xfirst = True, fhx
-                    if write:
-                        ysh, zsh = i2 != 1, i3 != 1
-                        first = (not xsh or xfirst) and (not ysh or (fly if i2 == 0 else fhy)) and \
-                                (not zsh or (flz if i3 == 0 else fhz))
-                        rw.append((col, wg, (X, Y0 + i2, Z0 + i3), tuple(contrib), first))
-            rcarry.update(newr)
-            # Jacobian rounds
-            for r in range(9):
-                m = r // 3
-                for h in (0, 1):
-                    if h == 1 and not hasB:
+    # elements of an axis that an assembled pair 0..7 of block e sums: vertex row
+    # 2e against columns 2e-2 .. 2e+2, interior row 2e+1 against 2e .. 2e+2
+    pair_elems = lambda e, q, n: [v for v in ((e - 1,), (e - 1,), (e - 1, e), (e,), (e,), (e,), (e,), (e,))[q]  # noqa: E731
+                                  if 0 <= v < n]
+    for block in range(nseg * cn1 * cn2):
+        bq = block // nseg
+        x0 = (block - bq * nseg) * seg
+        x1 = min(x0 + seg, n0)
+        ey0, ez0 = 2 * (bq % cn1), 2 * (bq // cn1)
+        for wv in range(4):
+            ey, ez = ey0 + (wv & 1), ez0 + (wv >> 1)
+            if ey > n1 or ez > n2:
+                continue
+            EYv, EYm = (5 if 0 < ey < n1 else 3), (3 if ey < n1 else 0)
+            EZv, EZm = (5 if 0 < ez < n2 else 3), (3 if ez < n2 else 0)
+            nr = [EYv * EZv, EYm * EZv, EYv * EZm, EYm * EZm]
+            lb = [sum(nr[:j]) for j in range(5)]
+            assert lb[4] <= 64
+            zs, ys = [q2_prefix(2 * ez + k) * T1 * T0 for k in (0, 1)], [q2_prefix(2 * ey + k) * T0 for k in (0, 1)]
+            line = [zs[j >> 1] + (EZm if j >> 1 else EZv) * ys[j & 1] for j in range(4)]
+            carry = [None] * 64
+            for e in range(max(x0 - 1, 0), x1):
+                staged = {}  # LDS slot -> elements of the sum
+                width = 8 if e > 0 else 6
+                last = {}
+                for lane in range(lb[4]):
+                    j = sum(lane >= lb[k] for k in (1, 2, 3))
+                    pt = lane - lb[j]
+                    EY = 3 if j & 1 else EYv
+                    iy, iz = pt % EY, pt // EY
+                    yp = 5 + iy if j & 1 else (2 + iy if ey == 0 else iy)
+                    zp = 5 + iz if j >> 1 else (2 + iz if ez == 0 else iz)
+                    yz = list(itertools.product(pair_elems(ey, yp, n1), pair_elems(ez, zp, n2)))
+                    own = [(e, y, z) for y, z in yz]
+                    if e > 0:
+                        c = carry[lane] or []
+                        for k in range(5):
+                            staged[8 * lb[j] + 5 * pt + k] = (c if k < 2 else c + own if k == 2 else own)
+                        for k in range(3):
+                            staged[8 * lb[j] + 5 * nr[j] + 3 * pt + k] = own
+                    else:
+                        for k in range(3):
+                            staged[6 * lb[j] + 3 * pt + k] = own
+                            staged[6 * lb[j] + 3 * nr[j] + 3 * pt + k] = own
+                    for k in range(3):
+                        last[3 * lane + k] = own
+                    carry[lane] = own
+                if e >= x0:
+                    assert sorted(staged) == list(range(width * lb[4]))
+                    for idx, els in staged.items():
+                        j = sum(idx >= width * lb[k] for k in (1, 2, 3))
+                        at = idx - width * lb[j]
+                        jw.append((line[j] + at + (8 * nr[j] * e - 2 * nr[j] if e > 0 else 0), els))
+                    if e + 1 == n0:
+                        for idx, els in last.items():
+                            j = sum(idx >= 3 * lb[k] for k in (1, 2, 3))
+                            jw.append((line[j] + nr[j] * (8 * n0 - 2) + idx - 3 * lb[j], els))
+            # residual rows of the block (16 lanes of the workgroup, four a block)
+            for e in range(x0, x1):
+                for j in range(4):
+                    Y, Z = 2 * ey + (j & 1), 2 * ez + (j >> 1)
+                    if Y >= N1 or Z >= N2:
                         continue
-                    ex = xa + h
-                    for l in range(32):
-                        pp = l + 32 * (r % 3)
-                        if pp >= 81:
-                            continue
-                        i1 = m if h else 2 - m
-                        j2, j3, i2, i3 = pp % 3, (pp // 3) % 3, (pp // 9) % 3, pp // 27
-                        X = 2 * ex + i1
-                        # this lane's run: columns 2 ex + j1, j1 = 0..2, element ex
-                        own = {2 * ex + j1: [el[h]] for j1 in range(3)}
-                        cols = {}
-                        xsh_first, xsh_last = False, False
-                        if m == 1:
-                            cols = own
-                        elif m == 0:
-                            if h == 0:
-                                cols = dict(own)
-                                if hasB:
-                                    cols[2 * ex + 2] = own[2 * ex + 2] + [el[1]]
-                                else:
-                                    xsh_last = x1 < nel[0]
-                            else:
-                                cols = {2 * ex + 1: own[2 * ex + 1], 2 * ex + 2: own[2 * ex + 2]}
-                        elif h == 0:
-                            if not first_step:
-                                c = carry[(r, l)]
-                                cols = {2 * ex - 2: c[2 * ex - 2], 2 * ex - 1: c[2 * ex - 1],
-                                        2 * ex: c[2 * ex] + own[2 * ex], 2 * ex + 1: own[2 * ex + 1],
-                                        2 * ex + 2: own[2 * ex + 2]}
-                            else:
-                                cols = own
-                                xsh_first = x0 > 0
-                        else:
-                            carry[(r, l)] = own
-                            if last_step:
-                                cols = own
-                                xsh_last = x1 < nel[0]
-                        if not cols:
-                            continue
-                        ysh = i2 == j2 and i2 != 1
-                        zsh = i3 == j3 and i3 != 1
-                        yz = (not ysh or (fly if i2 == 0 else fhy)) and (not zsh or (flz if i3 == 0 else fhz))
-                        ks = sorted(cols)
-                        for k, cxv in enumerate(ks):
-                            first = yz
-                            if xsh_first and k == 0:
-                                first = first and flx
-                            if xsh_last and k == len(ks) - 1:
-                                first = first and fhx
-                            ent = ((X, Y0 + i2, Z0 + i3), (cxv, Y0 + j2, Z0 + j3))
-                            jw.append((col, wg, ent, tuple(cols[cxv]), first))
+                    es = [(ey,) if j & 1 else (ey - 1, ey), (ez,) if j >> 1 else (ez - 1, ez)]
+                    yz = [(y, z) for y, z in itertools.product(*es) if 0 <= y < n1 and 0 <= z < n2]
+                    for k in range(3 if e + 1 == n0 else 2):
+                        xs = ([e - 1] if e > 0 else []) + [e] if k == 0 else [e]
+                        rw.append(((2 * e + k, Y, Z), [(x, y, z) for x in xs for y, z in yz]))
     return jw, rw
 
 
-def q2_node_elems(node, nel):
-    """Elements holding a Q2 lattice node."""
-    out = []
-    rng = []
-    for d in range(3):
-        c = node[d]
-        cand = [c // 2 - 1, c // 2] if c % 2 == 0 else [c // 2]
-        rng.append([e for e in cand if 0 <= e < nel[d]])
-    for e in itertools.product(*rng):
-        out.append(e)
-    return out
-
-
-@pytest.mark.parametrize("seg", [2, 4, 6, 12])
+@pytest.mark.parametrize("seg", [2, 4, 12])
 @pytest.mark.parametrize("nel", [(5, 4, 3), (7, 3, 2), (8, 1, 1), (1, 1, 1), (2, 5, 7), (13, 2, 3)])
-def test_pencil_schedule(nel, seg):
-    jw, rw = pencil_writes(nel, seg)
-    for writes, is_res in ((jw, False), (rw, True)):
-        by = {}
-        for col, wg, ent, contrib, first in writes:
-            by.setdefault(ent, []).append((col, wg, contrib, first))
-        if is_res:
-            expect = {tuple(n) for n in itertools.product(*(range(2 * n + 1) for n in nel))}
-        else:
-            expect = pattern_entries(3, 2, nel)
-        assert set(by) == expect, "writes do not cover the pattern exactly"
-        for ent, ws in by.items():
-            # each element holding both nodes contributes exactly once
-            if is_res:
-                want = sorted(q2_node_elems(ent, nel))
-            else:
-                er, ec_ = set(q2_node_elems(ent[0], nel)), set(q2_node_elems(ent[1], nel))
-                want = sorted(er & ec_)
-            got = sorted(e for w in ws for e in w[2])
-            assert got == want, f"{ent}: contributions {got} != {want}"
-            # concurrency: one writer per entry per launch (across and within workgroups)
-            launches = [w[0] for w in ws]
-            assert len(launches) == len(set(launches)), f"{ent}: two writers in one launch {ws}"
-            firsts = [w for w in ws if w[3]]
-            assert len(firsts) == 1, f"{ent}: {len(firsts)} first writers {ws}"
-            assert all(w[0] > firsts[0][0] for w in ws if not w[3]), f"{ent}: a later touch precedes the first"
+def test_row_owned_schedule(nel, seg):
+    jw, rw = q2box_writes(nel, seg)
+    pos = crs(nel)
+    assert {k for k, _ in pos.items()} == pattern_entries(3, 2, nel)
+    at = {p: ent for ent, p in pos.items()}
+    assert sorted(p for p, _ in jw) == list(range(len(pos))), "entries not written exactly once"
+    for p, els in jw:
+        r, c = at[p]
+        assert sorted(els) == sorted(set(node_elems(r, nel)) & set(node_elems(c, nel))), (r, c, els)
+    assert len(rw) == len({r for r, _ in rw}) == (2 * nel[0] + 1) * (2 * nel[1] + 1) * (2 * nel[2] + 1)
+    for r, els in rw:
+        assert sorted(els) == node_elems(r, nel), (r, els)
+
+
+@pytest.mark.parametrize("walk", [1, 2, 5, 48])
+@pytest.mark.parametrize("nel", [(1, 1, 1), (6, 7, 1), (7, 6, 2), (8, 8, 3), (14, 13, 9), (15, 1, 4)])
+def test_residual_tiles_own_every_row_once(nel, walk):
+    """k_q2res: 8 x 8 lanes of elements, 7 x 7 of them own the rows 2e and 2e + 1
+    of block e per axis and take the lower neighbour's share from the lane (x,
+    y) or the layer (z) before."""
+    n0, n1, n2 = nel
+    tx, ty, nb = (n0 + 7) // 7, (n1 + 7) // 7, n2 + 1
+    rows = {}
+    for bx, by, bz in itertools.product(range(tx), range(ty), range(-(-nb // walk))):
+        z0, z1 = bz * walk, min((bz + 1) * walk, nb)
+        layers = list(range(max(z0 - 1, 0), z1))
+        for lx, ly in itertools.product(range(8), range(8)):
+            ex, ey = 7 * bx + lx - 1, 7 * by + ly - 1
+            if not (lx > 0 and ly > 0 and ex <= n0 and ey <= n1):
+                continue
+            for z in range(z0, z1):
+                for i, j, k in itertools.product(range(2), range(2), range(2)):
+                    r = (2 * ex + i, 2 * ey + j, 2 * z + k)
+                    if any(c > 2 * n for c, n in zip(r, nel)):
+                        continue
+                    assert z == 0 or k or z - 1 in layers
+                    els = itertools.product((ex - 1, ex) if i == 0 else (ex,), (ey - 1, ey) if j == 0 else (ey,),
+                                            (z - 1, z) if k == 0 else (z,))
+                    els = sorted(e for e in els if all(0 <= c < n for c, n in zip(e, nel)))
+                    assert r not in rows, f"row {r} owned twice"
+                    rows[r] = els
+    assert set(rows) == set(itertools.product(*(range(2 * n + 1) for n in nel)))
+    for r, els in rows.items():
+        assert els == node_elems(r, nel), (r, els)
+
+
+@pytest.mark.parametrize("dim,p,nel", [(2, 1, (5, 3)), (2, 2, (3, 4)), (2, 3, (2, 3)), (2, 6, (1, 2)), (3, 1, (3, 2, 4)),
+                                       (3, 2, (2, 3, 1))])
+def test_row_gather(dim, p, nel):
+    """k_gather_rows: each element around a row adds its row of element matrix
+    into the row's image at the columns' places, in the order of the element
+    colours (the even one of two along an axis first)."""
+    nel3 = list(nel) + [1] * (3 - dim)
+    p1, nn = p + 1, [p * n + 1 if d < dim else 1 for d, n in enumerate(nel3)]
+    for X, Y, Z in itertools.product(*(range(m) for m in nn)):
+        row = (X, Y, Z)
+        lo, ln, el, il, po, two = ([0] * 3, [1] * 3, [[0, 0] for _ in range(3)], [[0, 0] for _ in range(3)],
+                                   [[0, 0] for _ in range(3)], [False] * 3)
+        for d in range(dim):
+            e = row[d] // p
+            elo, ehi = (e - 1 if row[d] % p == 0 and e > 0 else e), min(e, nel3[d] - 1)
+            two[d], lo[d], ln[d] = elo != ehi, p * elo, p * (ehi - elo + 1) + 1
+            el[d][0] = ehi if two[d] and elo & 1 else elo
+            el[d][1] = elo + ehi - el[d][0]
+            for t in range(2):
+                il[d][t], po[d][t] = row[d] - p * el[d][t], p * (el[d][t] - elo)
+            assert (lo[d], ln[d]) == axis_row(row[d], nel3[d], p)
+        image = {}
+        for k in range(1 << dim):
+            bit = [k >> d & 1 for d in range(3)]
+            if any(bit[d] and not two[d] for d in range(3)):
+                continue
+            ec = tuple(el[d][bit[d]] for d in range(3))
+            assert all(0 <= il[d][bit[d]] <= p for d in range(dim))
+            for jl in itertools.product(range(p1), range(p1), range(p1 if dim == 3 else 1)):
+                slot = sum((jl[d] + po[d][bit[d]]) * m for d, m in enumerate((1, ln[0], ln[0] * ln[1])))
+                col = tuple(p * ec[d] + jl[d] if d < dim else 0 for d in range(3))
+                want = sum((col[d] - lo[d]) * m for d, m in enumerate((1, ln[0], ln[0] * ln[1])))
+                assert slot == want
+                image.setdefault(col, []).append(ec)
+        colour = lambda e: (e[0] & 1) + 2 * (e[1] & 1) + 4 * (e[2] & 1)  # noqa: E731
+        assert len(image) == ln[0] * ln[1] * ln[2]
+        for col, els in image.items():
+            near = [set(node_elems(c, nel3, p)) if dim == 3 else {e + (0,) for e in node_elems(c[:2], nel, p)}
+                    for c in (row, col)]
+            assert sorted(els) == sorted(near[0] & near[1]), (row, col)
+            assert els == sorted(els, key=colour), (row, col, els)

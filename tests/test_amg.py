@@ -358,6 +358,50 @@ def test_device_block_smoother_vcycle_parity(name, sm):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("sweeps", [1, 2, 3, 4])
+@pytest.mark.parametrize("n", [(8, 7, 6), (12, 12, 11)], ids=lambda n: "x".join(map(str, n)))
+def test_block_jacobi_sweeps_parity(n, sweeps, monkeypatch):
+    """Four unknowns per node: the fused sweeps go from one vector into the other
+    and start where their number says (an odd or even count of them), on the
+    fine level with the columns in closed form and from the index stream, and
+    on a coarse level (three levels at 12 x 12 x 11)."""
+    from mrhyde_amd import Mhx, krylov_opts
+    from oracle import amg as oa
+
+    p = Problem(dim=3, order=1, quadrature=2, n=n, physics=MHX_PHYS_NAVIER_STOKES, mu=0.01, supg=True, pspg=True,
+                dbc_sides=1 | 2 | 4 | 16 | 32, lid_sides=8, lid_u=(1.0, 0.0, 0.0), pin_pressure=True)
+    g = Mhx(p)
+    g.set_option("amg.smoother", 1)
+    g.set_option("amg.sweeps", sweeps)
+    u = g.setDirichlet(1e-3 * np.random.default_rng(3).standard_normal(g.n_dof))
+    _, j = g.assembleJacRes(u)
+    rp, ci = g.crs_pattern()
+    A = sp.csr_matrix((j, ci, rp), shape=(g.n_dof, g.n_dof))
+    r = np.random.default_rng(9).standard_normal(g.n_dof)
+    # the oracle's cycle on the operators of the device's hierarchy
+    nl = g.buildAMGPreconditioner(j)
+    levels = [dict(A=A if l == 0 else g.amg_level(l, "A")[0], dinv=None) for l in range(nl)]
+    for l in range(nl - 1):
+        levels[l].update(P=g.amg_level(l, "P")[0], R=g.amg_level(l, "R")[0])
+    levels[-1]["Cinv"] = g.amg_level(nl - 1, "Cinv")[0]
+    assert nl == (2 if n == (8, 7, 6) else 3)
+    monkeypatch.setattr(oa, "BJ_SWEEPS", sweeps)
+    z = oa.vcycle(levels, r, "block_jacobi", 4)
+    w = A @ z
+    ref = (w @ r) / (w @ w) * z
+    print(f"[amg-sweeps] {n} {sweeps} levels={nl}", flush=True)
+    xs = []
+    for lat in (1, 0):
+        g.set_option("krylov.lattice_columns", lat)
+        x, st = g.linearSolver(j, r, opts=krylov_opts(solver="gmres", tol=1e-30, max_iters=1, precond="amg"))
+        assert st["iters"] == 1
+        np.testing.assert_allclose(x, ref, rtol=0, atol=1e-10 * np.abs(ref).max())
+        xs.append(x)
+    np.testing.assert_array_equal(xs[0], xs[1])
+    g.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("sm", list(SMOOTHERS))
 @pytest.mark.parametrize("name,solver", [("3d_q2_linear", "cg"), ("2d_ns_cavity", "gmres"),
                                          ("3d_q1_nonlinear", "gmres"), ("3d_ns_cavity", "gmres")])

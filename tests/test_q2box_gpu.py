@@ -1,10 +1,10 @@
-"""The pencil-streamed Q2 box assembly (assembly.colouring = 3) against the
-oracle: every Jacobian entry and residual within 1e-12, for x-segments of
-several lengths (segment ends inside the mesh, odd tails with one element
-in the last step), accumulate mode, a sine-mode source, Dirichlet rows on
+"""The row-owned Q2 box assembly (assembly.colouring = 3) against the oracle:
+every Jacobian entry and residual within 1e-12, for x-segments of several
+lengths (segment ends inside the mesh, where the layer before is evaluated
+again for its share), accumulate mode, a sine-mode source, Dirichlet rows on
 every side, and the same bits on a second assembly and against the
 residual-only pass.  Meshes with ragged extents (1, 2, 3, 5, 7 elements per
-axis) cover the pencil and segment boundaries on all three axes."""
+axis) cover the ends of the 2 x 2 pencil blocks and of the segments."""
 import numpy as np
 import pytest
 
@@ -118,8 +118,8 @@ def test_q2box_matches_element_colouring(pairs):
     r0, j0 = g.assembleJacRes(u)
     g.set_option("assembly.colouring", 3)
     r3, j3 = g.assembleJacRes(u)
-    assert_entries_close(j3, j0, rp, what="pencil vs element colouring Jacobian")
-    assert_entries_close(r3, r0, None, what="pencil vs element colouring residual")
+    assert_entries_close(j3, j0, rp, what="row-owned vs element colouring Jacobian")
+    assert_entries_close(r3, r0, None, what="row-owned vs element colouring residual")
 
 
 def test_q2box_refused_where_it_does_not_apply():

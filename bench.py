@@ -4,12 +4,13 @@
 Workload (one GPU): [0,1]^3, 96^3 Q2 hexahedra (193^3 = 7,189,057 DOFs,
 454,756,609 CRS nonzeros), 3x3x3 Gauss points, k(T,x) = k0_e (1 + T^2) with
 k0_e = exp(0.5 z_e) (z_e ~ N(0,1), seed 2024), source f_e ~ U[0,1] (seed 2025),
-T = 0 on x = 0 and x = 1.  A step is one full J+R assembly (eight colour
-launches of the fused kernel; the first element to touch an entry stores it,
-Dirichlet rows included) with u, res and J resident in HBM.
+T = 0 on x = 0 and x = 1.  A step is one full J+R assembly (one launch of the
+row-owned kernel, which writes every CRS entry once, Dirichlet rows included)
+with u, res and J resident in HBM.
 
 Prints one JSON line: assembly MDOF/s plus the roofline of the dominant kernel
-(algorithmic bytes B_asm per launch / its mean HIP-event duration) and a CPU
+(its measured HBM traffic per launch, or B_min where that is not on record, /
+its mean HIP-event duration) and a CPU
 baseline (the oracle on the full problem, OpenMP on the host's threads, with
 one GMRES iteration); beside them the GMRES iteration rate on the assembled
 Jacobian and the batched-subgrid solve rate.
@@ -52,7 +53,8 @@ def c2_problem(n: int):
 
 def b_asm(ne: int, n_e: int, n_c: int, n_vert: int, dim: int) -> float:
     """Algorithmic bytes of one coloured J+R assembly (element-matrix read+write,
-    u gather, residual read+write, coefficients, vertex coordinates)."""
+    u gather, residual read+write, coefficients, vertex coordinates): a count of
+    the method, which no kernel that owns its rows moves."""
     return ne * (16 * n_e * n_e + 24 * n_e + 8 * n_c) + 8 * dim * n_vert
 
 
@@ -423,27 +425,29 @@ def subgrid_bench(steps: int, per_call_sample: int = 16):
     out = {"workload": "4096 unit-cube Q1 thermal subproblems, n^3 elements, n in {4,6,8,12,16}, "
                        "lognormal k (sigma 1), random Dirichlet data, Jacobi-PCG to 1e-10",
            "n_instances": int(len(n_axis)), "total_nodes": int(((n_axis.astype(np.int64) + 1) ** 3).sum())}
-    nodes = (n_axis.astype(np.int64) + 1) ** 3
+    inner = (n_axis.astype(np.int64) - 1) ** 3
     for prec in ("fp64", "fp32-refined"):
         b = SubgridBatch(n_axis, k, g, tol=1e-10, precision=prec, use_graph=True)
         b.solve()
         ms = [b.solve() for _ in range(steps)]
         _, it, rel, refs = b.results()
         t = float(np.mean(ms))
-        # per node and PCG iteration: 27 p + 8 k LDS reads, 8x(8+1) FMAs in the
-        # stencil, ~10 flop of vector updates
-        node_its = float((nodes * it).sum())
+        # per interior node and PCG iteration, planes at the ends of a thread's
+        # run left out: the sweep reads 9 p and 4 k from LDS and takes 42 flop,
+        # the vector updates two reads and a write of p and 14 flop
+        node_its = float((inner * it).sum())
         out[prec] = {"ms_per_batch": round(t, 3), "solves_per_s": round(len(n_axis) / (t * 1e-3), 1),
                      "max_relres": float(rel.max()), "mean_iters": float(it.mean()), "wg_size": b.wg_size,
                      "mean_refinements": float(refs.mean()),
                      "node_iterations_per_s": round(node_its / (t * 1e-3), 1),
-                     "est_tflops": round(154.0 * node_its / (t * 1e-3) / 1e12, 2),
-                     "est_lds_TBps": round((35.0 * (8 if prec == "fp64" else 4)) * node_its / (t * 1e-3) / 1e12, 2)}
-        # the two ceilings of the on-chip solve: vector FP64 (FP32 inner:
-        # the FP32 vector rate) and LDS bandwidth (128 B per clock per CU,
-        # 256 CUs at 2.4 GHz = 78.6 TB/s)
+                     "est_tflops": round(56.0 * node_its / (t * 1e-3) / 1e12, 2),
+                     "est_lds_TBps": round((16.0 * (8 if prec == "fp64" else 4)) * node_its / (t * 1e-3) / 1e12, 2)}
+        # the two ceilings of the on-chip solve, neither of which it is near
+        # (an instance per CU and its dependent iterations): vector FP64 (FP32
+        # inner: the FP32 vector rate) and LDS bandwidth (128 B per clock per
+        # CU, 256 CUs at 2.4 GHz = 78.6 TB/s)
         flop_peak = 78.6 if prec == "fp64" else 157.3
-        out[prec]["roofline"] = {"bound": "lds", "achieved": out[prec]["est_lds_TBps"], "peak": LDS_PEAK_TBS,
+        out[prec]["roofline"] = {"bound": "latency", "achieved": out[prec]["est_lds_TBps"], "peak": LDS_PEAK_TBS,
                                  "unit": "TB/s", "frac": round(out[prec]["est_lds_TBps"] / LDS_PEAK_TBS, 4),
                                  "flop_frac": round(out[prec]["est_tflops"] / flop_peak, 4),
                                  "flop_peak_TFLOPs": flop_peak}
@@ -546,13 +550,13 @@ def main():
     mean_launch_ms = k_ms / max(k_cnt, 1)
     n_vert = (n + 1) ** 3
     B = b_asm(g.n_elem, 27, 2, n_vert, 3)
-    B_launch = B / launches_per_step
-    achieved = B_launch / (mean_launch_ms * 1e-3) / 1e9
     B_min = 8 * g.nnz + 16 * g.n_dof + 8 * 2 * g.n_elem + 8 * 3 * n_vert
     pmc = PMC_TRAFFIC.get((n, colouring))
     if pmc and pmc.get("segment", segment) != segment:
         pmc = None  # measured at another segment length
     traffic = (pmc["fetch_kib"] * pmc["fetch_scale"] + pmc["write_kib"] * pmc["write_scale"]) if pmc else None
+    B_launch = traffic if pmc else B_min / launches_per_step
+    achieved = B_launch / (mean_launch_ms * 1e-3) / 1e9
 
     # achievable-bandwidth reference: plain device copy of known size
     import ctypes as C
@@ -613,14 +617,18 @@ def main():
         "data": "synthetic (seeded lognormal k0, uniform source, random u)",
         "config": {"workload": f"nonlinear thermal J+R assembly, {n}^3 Q2 hex, 3x3x3 Gauss, k=k0(1+T^2)",
                    "n_dof": g.n_dof, "nnz": g.nnz, "n_elem": g.n_elem, "parallelism": "single GPU"},
-        "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
+        "roofline": {"bound": "issue" if colouring == 3 else "hbm", "achieved": round(achieved, 1),
+                     "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": round(achieved / HBM_PEAK_GBS, 4),
+                     "bytes": "measured traffic" if pmc else "B_min", "traffic": traffic,
                      "traffic_source": "rocprofv3 --pmc FETCH_SIZE/WRITE_SIZE, copy-kernel calibrated" if pmc else None,
                      "traffic_per": "launch",
                      "kernel": kname, "launches_per_step": launches_per_step,
                      "mean_launch_ms": round(mean_launch_ms, 5), "bytes_per_launch": B_launch,
-                     "B_asm": B, "B_min": B_min, "copy_probe_GBps": probe,
-                     "colouring": {0: "element", 1: "block", 2: "x-segments", 3: "pencil streaming"}[colouring],
+                     "B_min": B_min, "B_min_frac": round(B_min / launches_per_step / (mean_launch_ms * 1e-3) / 1e9
+                                                         / HBM_PEAK_GBS, 4),
+                     "B_asm_count": B, "copy_probe_GBps": probe,
+                     "colouring": {0: "element", 1: "block", 2: "x-segments", 3: "row-owned"}[colouring],
                      "segment": segment if colouring == 3 else None},
         "cpu_baseline": cpu,
         "mfma_contraction_probe": mfma,

@@ -184,8 +184,9 @@ const Entry kStoreTable[] = {
 //   3-D Q1 16^3 77/12, 32^3 81/37, 64^3 (128 MiB) 360/192
 //   3-D Q2, three points per axis: 8^3 168/21, 16^3 169/42, 24^3 (77 MiB)
 //     176/96, 32^3 (182 MiB) 243/213, 40^3 (356 MiB) 473/429
-// The gain shrinks as the round trip of the element matrices leaves the caches;
-// past the largest size measured the scratch memory (1.35 times the Jacobian in
+// The gain shrinks as the round trip of the element matrices leaves the caches.
+// No size measured was slower here: the line bounds the memory.  Past the
+// largest size measured the scratch memory (1.35 times the Jacobian in
 // 3-D Q2) is not spent.  It is allocated with the context, so no assembly
 // allocates, given back when an option or a time state takes the assembly
 // elsewhere, and for a solve that would otherwise run out of memory.

@@ -667,8 +667,8 @@ bool q2box_applicable(const Ctx& c) {
 // Elements per x-segment.  A workgroup repeats the layer before its segment
 // and fills its pipeline (about two layers), and the device runs `slots`
 // workgroups at a time: the fewest layers in sequence win.  96^3, us by
-// segment: 8 1,953, 12 1,924, 16 1,865, 24 1,877, 48 1,896, 96 2,014; 16^3: 2
-// 26.4, 4 31.2, 8 38.9, 16 64.4.
+// segment: 8 1,814, 12 1,730, 16 1,689, 24 1,676 (taken), 32 1,670, 48 1,691, 96
+// 1,807; 16^3: 2 24.8 (taken), 4 27.9, 8 34.7, 16 58.0.
 static int q2_auto_segment(const Ctx& c, int slots) {
   const int n0 = c.mesh.nel[0];
   const long nyz = (long)((c.mesh.nel[1] + 2) / 2) * ((c.mesh.nel[2] + 2) / 2);

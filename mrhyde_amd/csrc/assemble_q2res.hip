@@ -5,9 +5,12 @@
 // want the residual alone (line searches and convergence checks of Newton's
 // method), with an element source but no sine modes.
 //
-// What bounds it: FP64 issue (about 1,400 operations an element), so there are
-// no barriers and a lane evaluates one element in registers by sum
-// factorisation; a wavefront covers 8 x 8 elements in x and y and walks z.  Node
+// What bounds it: latency.  About 1,400 operations an element (1.6 times that
+// with the elements evaluated twice) take 20 of the 64 us of a 64^3 mesh; two
+// thirds of the wavefronts' cycles wait, at two wavefronts per SIMD, for loads
+// and for the 50 registers that spill.  So there are no barriers and a lane
+// evaluates one element in registers by sum factorisation; a wavefront covers
+// 8 x 8 elements in x and y and walks z.  Node
 // rows 2e and 2e + 1 of block e sum the elements e - 1 and e: the z neighbour's
 // share comes from the layer before (through LDS, 27 doubles a lane, to keep
 // the registers at two wavefronts per SIMD), the y neighbour's by a lane

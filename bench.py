@@ -492,9 +492,9 @@ def main():
     ap.add_argument("--n", type=int, default=96, help="elements per axis")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--colouring", type=int, default=-1,
-                    help="assembly schedule: -1 the context's default (3, pencil streaming, on this box mesh), "
+                    help="assembly schedule: -1 the context's default (3, rows owned, on this box mesh), "
                          "0 element colouring, 1 block colouring, 2 x-segments")
-    ap.add_argument("--segment", type=int, default=0, help="pencil streaming: elements per x-segment (0 = default)")
+    ap.add_argument("--segment", type=int, default=0, help="rows owned: elements per x-segment (0 = default)")
     ap.add_argument("--probe-gib", type=float, default=1.0, help="size of the plain-copy bandwidth probe")
     ap.add_argument("--skip-subgrid", action="store_true", help="skip the batched-subgrid measurement")
     ap.add_argument("--krylov-iters", type=int, default=100, help="GMRES iterations timed (0 = skip)")

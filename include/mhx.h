@@ -377,7 +377,7 @@ int  mhx_l2_error(mhx_ctx* ctx, const double* u, int32_t n_modes, const double* 
  *                         row's share as contiguous runs; Navier-Stokes:
  *                         segments of 8 (3-D) / 16 (2-D) elements; block
  *                         colouring runs element colouring there),
- *                         3 = pencil streaming (one launch: a workgroup
+ *                         3 = rows owned (one launch: a workgroup
  *                         owns the rows of 2 x 2 element pencils, walks an
  *                         x-segment and writes each row once; 3-D Q2
  *                         thermal with 3x3x3 Gauss on an unperturbed box
@@ -388,7 +388,7 @@ int  mhx_l2_error(mhx_ctx* ctx, const double* u, int32_t n_modes, const double* 
  *                         matrices up to 384 MiB) runs in two launches:
  *                         element matrices, then a sum per row (same sums
  *                         in the same order); 0: element colouring.
- *   "assembly.segment"    pencil streaming: elements per x-segment, even,
+ *   "assembly.segment"    rows owned: elements per x-segment, even,
  *                         2 .. 4096 (default: from the mesh and the kernel,
  *                         so that the workgroups fill the device evenly;
  *                         reading it gives the Jacobian's, and setting

@@ -76,7 +76,7 @@ static void launch_colors(Ctx& c, AsmArgs& a, bool jac) {
   using C = Cfg<DIM, P, NQ1>;
   const int ncol = 1 << DIM;
   // the transient variant is built for element colouring only, and so is
-  // every order when pencil streaming is selected but does not apply
+  // every order when the row-owned kernel is selected but does not apply
   const int mode = (a.hist || c.scatter_mode == kPencilStream) ? (int)kElementColouring : c.scatter_mode;
   // the segment schedule needs two elements per workgroup (even and odd
   // phases); every built order has at least four

@@ -242,7 +242,7 @@ struct Ctx {
   bool store_captured = false;  // a captured graph holds escr's and rscr's addresses
   DevBuf<double> escr, rscr;  // element matrices and residuals (allocated where the element store applies)
   bool box_mesh = false;  // every element an axis-aligned box (structured box, no node perturbation)
-  int q2_segment = 0;     // pencil streaming: elements per x-segment (even; 0: chosen per launch)
+  int q2_segment = 0;     // row-owned kernel: elements per x-segment (even; 0: chosen per launch)
   std::shared_ptr<Amg> amg;  // built by a solve with the AMG preconditioner, kept for reuse of its buffers
   // time-integration state (mhx_set_time_state); bdf_order 0 = steady
   int bdf_order = 0;

@@ -274,10 +274,10 @@ int q2box_segment(const Ctx& c, bool jac);  // elements per x-segment of a launc
 // residuals; and its launches
 int64_t element_store_doubles(const mhx_problem_desc& d);
 int64_t element_store_bytes(const mhx_problem_desc& d);
-// The scratch memory is held while the context's steady assembly uses it: take
-// it if it does (without, where there is no room) and give it back if not;
-// give it back in any case, true if there was any (both: not while a captured
-// graph holds its address)
+// Take the scratch memory if the context's options and time state use it
+// (without, where there is no room) and give it back if not; give it back in any
+// case, true if there was any (both: not while a captured graph holds its
+// address)
 void element_store_fit(Ctx& c);
 bool element_store_release(Ctx& c);
 // f(c) with the scratch memory given back and f run again where memory runs

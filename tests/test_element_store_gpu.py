@@ -88,8 +88,11 @@ def test_assembly_options_survive_a_round_trip(kind):
 
 
 def _free():
+    import gc
+
     import torch
 
+    gc.collect()  # (contexts that earlier tests left)
     torch.cuda.synchronize()
     return torch.cuda.mem_get_info()[0]
 
